@@ -85,6 +85,28 @@ int wsl_decode_attention_step_fwd(const void* qkv, int64_t ldqkv, int64_t batch,
 int wsl_swiglu_fwd(const void* gate_up, int64_t ld, int64_t rows, int64_t ffn, void* out, int64_t ldo,
                    void* stream);
 
+/* ---- The same work for a whole prompt (positions 0..seq-1 of every sequence) ----
+ * Token t = b * seq + p of k, v, q and out is row t; it takes row p of `rope` (cos | sin,
+ * [>= seq, 2 * head_dim] fp32). head_dim 64 or 128; 16-byte aligned rows.
+ *
+ * k [batch * seq, n_kv_heads * head_dim] RMS-normed over head_dim and rotated, and v, written
+ * to the caches at positions 0..seq-1 (seq <= cache_len). Replaces k_norm, apply_rotary_emb
+ * and the cache copies (qwen3/model/model.py:73-90,195-206). */
+int wsl_kv_norm_rope_fwd(const void* k, int64_t ldk, const void* v, int64_t ldv, int64_t batch, int64_t seq,
+                         int64_t n_kv_heads, int64_t head_dim, const void* k_norm_w, float eps, const float* rope,
+                         void* k_cache, void* v_cache, int64_t cache_len, void* stream);
+/* out [batch * seq, n_heads * head_dim] = causal softmax(rope(rmsnorm(q)) . K^T * scale) . V
+ * per head over the caches' positions 0..seq-1, query head i on kv head i / (n_heads /
+ * n_kv_heads). Replaces q_norm, apply_rotary_emb, repeat_kv and the attention
+ * (qwen3/model/model.py:73-102,195-218). scale > 0. */
+int wsl_prefill_attention_fwd(const void* q, int64_t ldq, int64_t batch, int64_t seq, int64_t n_heads,
+                              int64_t n_kv_heads, int64_t head_dim, const void* q_norm_w, float eps,
+                              const float* rope, const void* k_cache, const void* v_cache, int64_t cache_len,
+                              float scale, void* out, int64_t ldo, void* stream);
+/* wsl_swiglu_fwd on two projections' own outputs: out = silu(gate) * up [rows, ffn]. */
+int wsl_swiglu_pair_fwd(const void* gate, int64_t ldg, const void* up, int64_t ldu, int64_t rows, int64_t ffn,
+                        void* out, int64_t ldo, void* stream);
+
 /* out[row] = index of the largest x[row, 0..n) (bf16): the greedy token of a row of logits
  * (scripts/generate/_generation.py:26-29 with top_k = 1 keeps only the argmax). Ties give
  * the first index and NaN counts as largest, as torch.argmax. Rows that are 16-byte aligned

@@ -63,6 +63,9 @@ EXPORTED = (
     "wsl_decode_attention_step_workspace_bytes",
     "wsl_decode_attention_step_fwd",
     "wsl_swiglu_fwd",
+    "wsl_kv_norm_rope_fwd",
+    "wsl_prefill_attention_fwd",
+    "wsl_swiglu_pair_fwd",
     "wsl_argmax_rows_fwd",
     "wsl_argmax_rows_workspace_bytes",
     "wsl_lora_linear_fused_supported",
@@ -261,6 +264,17 @@ def _declare(lib: ctypes.CDLL) -> None:
         _c_vp, ctypes.c_size_t, _c_vp]                       # workspace, bytes, stream
     lib.wsl_swiglu_fwd.restype = ctypes.c_int
     lib.wsl_swiglu_fwd.argtypes = [_c_vp, _c_i64, _c_i64, _c_i64, _c_vp, _c_i64, _c_vp]
+    lib.wsl_kv_norm_rope_fwd.restype = ctypes.c_int
+    lib.wsl_kv_norm_rope_fwd.argtypes = [
+        _c_vp, _c_i64, _c_vp, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64,  # k, ldk, v, ldv, batch, seq, n_kv, head_dim
+        _c_vp, ctypes.c_float, _c_vp, _c_vp, _c_vp, _c_i64, _c_vp]     # k_norm_w, eps, rope, k_cache, v_cache, cache_len, stream
+    lib.wsl_prefill_attention_fwd.restype = ctypes.c_int
+    lib.wsl_prefill_attention_fwd.argtypes = [
+        _c_vp, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64,  # q, ldq, batch, seq, n_heads, n_kv, head_dim
+        _c_vp, ctypes.c_float, _c_vp, _c_vp, _c_vp, _c_i64,     # q_norm_w, eps, rope, k_cache, v_cache, cache_len
+        ctypes.c_float, _c_vp, _c_i64, _c_vp]                   # scale, out, ldo, stream
+    lib.wsl_swiglu_pair_fwd.restype = ctypes.c_int
+    lib.wsl_swiglu_pair_fwd.argtypes = [_c_vp, _c_i64, _c_vp, _c_i64, _c_i64, _c_i64, _c_vp, _c_i64, _c_vp]
     lib.wsl_lora_linear_fused_supported.restype = ctypes.c_int
     lib.wsl_lora_linear_fused_supported.argtypes = [_c_i64, _c_i64, _c_i64, _c_i64, ctypes.c_int32]
     lib.wsl_lora_linear_fused_fwd.restype = ctypes.c_int

@@ -750,6 +750,10 @@ int dfail(int code, const char* msg) {
 }
 }  // namespace
 
+namespace wsl {
+int decode_fail(int code, const char* msg) { return dfail(code, msg); }
+}  // namespace wsl
+
 extern "C" {
 
 const char* wsl_decode_last_error(void) { return g_derr; }

@@ -953,6 +953,97 @@ def _swiglu_fake(gate_up):
     return gate_up.new_empty((*gate_up.shape[:-1], gate_up.shape[-1] // 2), dtype=torch.bfloat16)
 
 
+# ------------------------------------------------------------------------------------------
+# The same work for a whole prompt, positions 0..seq-1 (include/wsl_decode.h). Inference only.
+# ------------------------------------------------------------------------------------------
+def _check_prompt(rows: int, k_cache: torch.Tensor, v_cache: torch.Tensor, rope: torch.Tensor) -> int:
+    """seq of a prompt of `rows` tokens over the caches' batch, after the checks that the
+    prompt ops share."""
+    b, _, L, hd = k_cache.shape
+    if k_cache.shape != v_cache.shape or not (k_cache.is_contiguous() and v_cache.is_contiguous()):
+        raise ValueError("k_cache and v_cache must be contiguous [b, n_kv_heads, L, head_dim]")
+    if k_cache.dtype != torch.bfloat16 or v_cache.dtype != torch.bfloat16:
+        raise TypeError("k_cache and v_cache must be bfloat16")
+    if b == 0 or rows % b != 0:
+        raise ValueError(f"{rows} tokens do not divide over {b} sequences")
+    seq = rows // b
+    if rope.dtype != torch.float32 or not rope.is_contiguous() or rope.dim() != 2 or rope.shape[1] != 2 * hd \
+            or rope.shape[0] < seq:
+        raise ValueError(f"rope must be contiguous fp32 [>= {seq}, {2 * hd}] (cos | sin); got {tuple(rope.shape)}")
+    return seq
+
+
+@torch.library.custom_op("wsl::kv_norm_rope", mutates_args=("k_cache", "v_cache"), device_types="cuda")
+def kv_norm_rope_op(k: torch.Tensor, v: torch.Tensor, k_norm_w: torch.Tensor, eps: float, rope: torch.Tensor,
+                    k_cache: torch.Tensor, v_cache: torch.Tensor) -> None:
+    """k [b * seq, n_kv_heads * hd] (normed, rotated) and v into the caches [b, n_kv_heads, L, hd]
+    at positions 0..seq-1."""
+    dev = _check_device(k, v, k_norm_w, rope, k_cache, v_cache)
+    b, nkv, L, hd = k_cache.shape
+    k2, v2 = _bf16_2d(k, "k"), _bf16_2d(v, "v")
+    seq = _check_prompt(k2.shape[0], k_cache, v_cache, rope)
+    if k2.shape != v2.shape or k2.shape[1] != nkv * hd or k_norm_w.shape != (hd,):
+        raise ValueError(f"k {tuple(k2.shape)}, v {tuple(v2.shape)} and k_norm_w {tuple(k_norm_w.shape)} do not match "
+                         f"{nkv} heads of {hd}")
+    kw = k_norm_w.to(torch.bfloat16).contiguous()
+    with torch.cuda.device(dev):
+        rc = _native.lib().wsl_kv_norm_rope_fwd(
+            k2.data_ptr(), k2.stride(0), v2.data_ptr(), v2.stride(0), b, seq, nkv, hd, kw.data_ptr(), float(eps),
+            rope.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), L, _stream(dev))
+    _native.check(rc, "wsl_kv_norm_rope_fwd", decode=True)
+
+
+@kv_norm_rope_op.register_fake
+def _kv_norm_rope_fake(k, v, k_norm_w, eps, rope, k_cache, v_cache):
+    return None
+
+
+@torch.library.custom_op("wsl::prefill_attention", mutates_args=(), device_types="cuda")
+def prefill_attention_op(q: torch.Tensor, q_norm_w: torch.Tensor, eps: float, rope: torch.Tensor,
+                         k_cache: torch.Tensor, v_cache: torch.Tensor, n_heads: int, scale: float) -> torch.Tensor:
+    """Causal attention of a prompt: q [b * seq, n_heads * hd] normed and rotated, against positions
+    0..seq-1 of the caches [b, n_kv_heads, L, hd] (see kv_norm_rope) -> [b * seq, n_heads * hd]."""
+    dev = _check_device(q, q_norm_w, rope, k_cache, v_cache)
+    b, nkv, L, hd = k_cache.shape
+    q2 = _bf16_2d(q, "q")
+    seq = _check_prompt(q2.shape[0], k_cache, v_cache, rope)
+    if q2.shape[1] != n_heads * hd or q_norm_w.shape != (hd,):
+        raise ValueError(f"q {tuple(q2.shape)} and q_norm_w {tuple(q_norm_w.shape)} do not match {n_heads} heads of {hd}")
+    qw = q_norm_w.to(torch.bfloat16).contiguous()
+    out = torch.empty((q2.shape[0], n_heads * hd), dtype=torch.bfloat16, device=dev)
+    with torch.cuda.device(dev):
+        rc = _native.lib().wsl_prefill_attention_fwd(
+            q2.data_ptr(), q2.stride(0), b, seq, n_heads, nkv, hd, qw.data_ptr(), float(eps), rope.data_ptr(),
+            k_cache.data_ptr(), v_cache.data_ptr(), L, float(scale), out.data_ptr(), out.stride(0), _stream(dev))
+    _native.check(rc, "wsl_prefill_attention_fwd", decode=True)
+    return out
+
+
+@prefill_attention_op.register_fake
+def _prefill_attention_fake(q, q_norm_w, eps, rope, k_cache, v_cache, n_heads, scale):
+    return q.new_empty((q.numel() // q.shape[-1], n_heads * k_cache.shape[3]), dtype=torch.bfloat16)
+
+
+@torch.library.custom_op("wsl::swiglu_pair", mutates_args=(), device_types="cuda")
+def swiglu_pair_op(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
+    """silu(gate) * up for two tensors of one shape."""
+    dev = _check_device(gate, up)
+    if gate.shape != up.shape:
+        raise ValueError(f"gate {tuple(gate.shape)} and up {tuple(up.shape)} differ")
+    g2, u2 = _bf16_2d(gate, "gate"), _bf16_2d(up, "up")
+    out = torch.empty(g2.shape, dtype=torch.bfloat16, device=dev)
+    with torch.cuda.device(dev):
+        rc = _native.lib().wsl_swiglu_pair_fwd(g2.data_ptr(), g2.stride(0), u2.data_ptr(), u2.stride(0), g2.shape[0],
+                                               g2.shape[1], out.data_ptr(), out.stride(0), _stream(dev))
+    _native.check(rc, "wsl_swiglu_pair_fwd", decode=True)
+    return out.view(gate.shape)
+
+
+@swiglu_pair_op.register_fake
+def _swiglu_pair_fake(gate, up):
+    return gate.new_empty(gate.shape, dtype=torch.bfloat16)
+
+
 @torch.library.custom_op("wsl::argmax_rows", mutates_args=(), device_types="cuda")
 def argmax_rows_op(x: torch.Tensor) -> torch.Tensor:
     """int64 index of the largest element of each row (first on ties, NaN largest)."""

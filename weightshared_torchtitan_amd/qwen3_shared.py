@@ -249,6 +249,8 @@ class SharedQwen3(nn.Module):
         if s > a.max_seq_len:
             raise IndexError(f"sequence of {s} tokens exceeds max_seq_len {a.max_seq_len} (the RoPE table)")
         pk = self._decode_pack() if (self.prefill_grouped and not torch.is_grad_enabled()) else None
+        if self._prefill_fused_ok(tokens, cache):
+            return self._forward_fused(tokens, cache, pk)
         h = self.tok_embeddings(tokens)
         rc = self.rope[:s].view(1, s, 1, 2 * a.head_dim)
         rep = a.n_heads // a.n_kv_heads
@@ -276,6 +278,65 @@ class SharedQwen3(nn.Module):
             h = self._ffn(l, h, pk)
         h = self.norm(h)
         return self.tok_embeddings.tied_logits(h)
+
+    # Inference forwards take the library's own kernels between the projections (q/k norm, RoPE,
+    # cache write, attention, residual add + RMSNorm, SwiGLU) where they cover the model; off, and
+    # wherever gradients are recorded, those are torch ops.
+    prefill_fusion = True
+
+    def _prefill_fused_ok(self, tokens: torch.Tensor, cache: Optional[KVCache]) -> bool:
+        """Whether this forward may take the fused prompt kernels: inference in bf16 on the GPU
+        outside autocast, head sizes the attention kernel has, a contiguous cache that holds the
+        prompt, and no hook on the norm modules (the fused kernels do not call them)."""
+        a = self.args
+        if not self.prefill_fusion or torch.is_grad_enabled() or tokens.device.type != "cuda" \
+                or torch.is_autocast_enabled("cuda") or tokens.numel() == 0:
+            return False
+        if a.head_dim not in (64, 128) or a.n_heads % a.n_kv_heads != 0 or a.dim % 8 != 0 or a.dim > 8192 \
+                or a.hidden_dim % 8 != 0:
+            return False
+        if cache is not None:
+            b, s = tokens.shape
+            shape = (a.n_layers, b, a.n_kv_heads, cache.max_len, a.head_dim)
+            if any(t.dtype != torch.bfloat16 or t.device != tokens.device or t.shape != shape or not t.is_contiguous()
+                   for t in (cache.k, cache.v)) or s > cache.max_len:
+                return False
+        for m in self.modules():
+            if isinstance(m, RMSNorm) and (m._forward_hooks or m._forward_pre_hooks):
+                return False
+        return all(p.dtype == torch.bfloat16 and p.device == tokens.device for p in self.parameters())
+
+    def _forward_fused(self, tokens: torch.Tensor, cache: Optional[KVCache], pk: Optional[dict]) -> torch.Tensor:
+        """``forward`` with the prompt kernels of include/wsl_decode.h between the projections."""
+        a = self.args
+        b, s = tokens.shape
+        rope = self.rope.float().contiguous()
+        h = self.tok_embeddings(tokens).view(b * s, a.dim)
+        if cache is None:  # one layer's keys and values
+            k_new = h.new_empty(b, a.n_kv_heads, s, a.head_dim)
+            v_new = torch.empty_like(k_new)
+        y = None
+        for l in range(a.n_layers):
+            blk = self.base_blocks[a.block_of(l)]
+            at = blk.attention
+            if y is None:
+                x = ops.rmsnorm_op(h, blk.attention_norm.weight, blk.attention_norm.eps)
+            else:
+                x, h = ops.add_rmsnorm_op(y, h, blk.attention_norm.weight, blk.attention_norm.eps)
+            qkv = self._grouped(l, "qkv", x, pk)
+            if qkv is None:
+                qkv = [self._proj(l, n, x) for n in ("wq", "wk", "wv")]
+            kc, vc = (cache.k[l], cache.v[l]) if cache is not None else (k_new, v_new)
+            ops.kv_norm_rope_op(qkv[1], qkv[2], at.k_norm.weight, at.k_norm.eps, rope, kc, vc)
+            o = ops.prefill_attention_op(qkv[0], at.q_norm.weight, at.q_norm.eps, rope, kc, vc, a.n_heads,
+                                         a.head_dim ** -0.5)
+            x, h = ops.add_rmsnorm_op(self._proj(l, "wo", o), h, blk.ffn_norm.weight, blk.ffn_norm.eps)
+            gu = self._grouped(l, "gu", x, pk)
+            if gu is None:
+                gu = [self._proj(l, "w1", x), self._proj(l, "w3", x)]
+            y = self._proj(l, "w2", ops.swiglu_pair_op(gu[0], gu[1]))
+        x, _ = ops.add_rmsnorm_op(y, h, self.norm.weight, self.norm.eps)
+        return self.tok_embeddings.tied_logits(x.view(b, s, a.dim))
 
     # ------------------------------------------------------------------ decode
     def _decode_pack(self) -> dict:
