@@ -244,8 +244,8 @@ int wsl_lora_linear_bwd_weights(const void* x, int64_t ldx, const void* gy, int6
  * wsl_lora_linear_bwd_input_supported returns 1 for the layouts taken: N a multiple of 64,
  * K and r multiples of 8 (K of 16 for fp8), r <= WSL_MAX_RANK, gy, W, A, B and dx 16-byte
  * aligned with leading dimensions multiples of 8 (fp8 ldw of 16; dx: 8-byte aligned, ldd a
- * multiple of 4); the rest return WSL_E_SHAPE (or WSL_E_ALIGN), and a caller multiplies by
- * a transposed copy of W instead.
+ * multiple of 4); the rest return WSL_E_SHAPE (or WSL_E_ALIGN): wsl_lora_linear_bwd_input_any
+ * takes a bf16 W in any layout.
  * Workspace (256-byte aligned) from wsl_lora_linear_bwd_input_workspace_bytes: the forward's
  * prefill scratch for [M, K] outputs plus the transposed A and B. fp32 accumulation, T =
  * bf16(scale * gy . B) rounded once, as the forward.
@@ -259,6 +259,26 @@ int wsl_lora_linear_bwd_input(const void* gy, int64_t ldg, const void* w, int64_
                               float scale, void* dx, int64_t lddx,
                               int64_t M, int64_t N, int64_t K, int64_t r,
                               void* workspace, size_t workspace_bytes, void* stream);
+
+/*
+ * wsl_lora_linear_bwd_input for a bf16 W in any layout (any N, K, r up to WSL_MAX_RANK, any
+ * leading dimensions, element-aligned pointers), on bounds-checked matrix-core tiles that read W
+ * and A where they lie. Workspace (256-byte aligned): bf16(scale * gy . B) [M, r].
+ */
+int wsl_lora_linear_bwd_input_any_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t r, size_t* bytes);
+int wsl_lora_linear_bwd_input_any(const void* gy, int64_t ldg, const void* w, int64_t ldw, const void* a, int64_t lda,
+                                  const void* b, int64_t ldb, float scale, void* dx, int64_t lddx, int64_t M,
+                                  int64_t N, int64_t K, int64_t r, void* workspace, size_t workspace_bytes,
+                                  void* stream);
+
+/*
+ * LoRA factors of a rank that the tiled kernels do not take (off 8), padded with zeros: a
+ * [n_groups * r, K] -> a_out [n_groups * r_padded, K] (each group's rows followed by zero rows),
+ * b [N, r] -> b_out [N, r_padded], both outputs dense. A LoRA linear with the padded factors is
+ * that with the original ones.
+ */
+int wsl_lora_pad_rank(const void* a, int64_t lda, const void* b, int64_t ldb, int32_t n_groups, int64_t r,
+                      int64_t r_padded, int64_t K, int64_t N, void* a_out, void* b_out, void* stream);
 
 /*
  * Factorized embedding:  out[t, :] = E[ids[t], :] . P^T      (k -> hidden)

@@ -1,0 +1,133 @@
+"""The products for layouts off the tiled kernels (csrc/lora_generic.hip) at the edges of their
+tiles (64 x 64 over k steps of 128; 128 x 128 over 64 where those fill the chip), with odd
+strides and unaligned pointers, forward and every gradient against plain torch in float64; and
+ranks off 8 on grid shapes, which the ops pad with zeros onto the tiled kernels."""
+import sys
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+TOL = 1e-2  # one rounding of T or U and one of the result to bf16, of the largest value
+
+
+def _say(msg):
+    print(msg, flush=True)
+    sys.stdout.flush()
+
+
+def rel(x, ref):
+    return ((x.double() - ref).abs().max() / ref.abs().max().clamp_min(1e-30)).item()
+
+
+def view(t, odd):
+    """t as it is, or a view of odd stride and odd element offset into a wider buffer of NaN."""
+    if not odd:
+        return t
+    big = torch.full((t.shape[0], t.shape[1] + 5), float("nan"), dtype=t.dtype, device=t.device)
+    v = big[:, 1:1 + t.shape[1]]
+    v.copy_(t)
+    return v
+
+
+def inputs(gpu, M, N, K, r, seed, odd=False):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    mk = lambda *s, std=1.0: view((torch.randn(*s, device=gpu, generator=g) * std).bfloat16(), odd)  # noqa: E731
+    return mk(M, K), mk(N, K, std=0.05), mk(r, K, std=0.05), mk(N, r, std=0.05), mk(M, N)
+
+
+def check_all(gpu, M, N, K, r, odd=False, seed=0, s=2.0):
+    from weightshared_torchtitan_amd import ops
+    x, w, a, b, gy = inputs(gpu, M, N, K, r, seed + M + 3 * N + 7 * K, odd)
+    X, W, A, B, G = (t.double() for t in (x, w, a, b, gy))
+    y = ops.lora_linear_op(x, w, None, a, b, s)
+    assert rel(y, X @ W.t() + s * (X @ A.t()) @ B.t()) <= TOL
+    assert rel(ops.lora_linear_op(x, None, None, a, b, s), s * (X @ A.t()) @ B.t()) <= TOL
+    assert rel(ops.lora_linear_op(x, w, None, None, None, s), X @ W.t()) <= TOL
+    assert rel(ops.lora_linear_bwd_input_op(gy, w, None, a, b, s), G @ W + s * (G @ B) @ A) <= TOL
+    assert rel(ops.lora_linear_bwd_input_op(gy, w, None, None, None, s), G @ W) <= TOL
+    for need_w in (False, True):
+        got = ops.lora_linear_weight_grads_op(x, gy, a, b, s, need_w, True, True)
+        again = ops.lora_linear_weight_grads_op(x, gy, a, b, s, need_w, True, True)
+        assert all(torch.equal(p, q) for p, q in zip(got, again))
+        assert rel(got[1], s * (G @ B).t() @ X) <= TOL and rel(got[2], s * G.t() @ (X @ A.t())) <= TOL
+        if need_w:
+            assert rel(got[0], G.t() @ X) <= TOL
+
+
+CASES = [
+    # M, N, K, r, odd strides and offsets
+    (1, 1, 1, 1, False),
+    (1, 100, 72, 3, True),
+    (5, 63, 127, 7, False),
+    (64, 64, 129, 9, False),       # one k past a step
+    (65, 65, 128, 8, True),        # one row and column past a tile, rows unaligned
+    (127, 129, 256, 16, True),     # grid sizes on unaligned rows
+    (200, 333, 77, 31, False),
+    (777, 150, 1000, 12, False),
+    (130, 260, 136, 256, False),   # the largest rank
+    (2100, 2090, 100, 5, False),   # 128-wide tiles
+    (2049, 2177, 65, 33, True),
+]
+
+
+@pytest.mark.parametrize("M,N,K,r,odd", CASES)
+def test_generic_layouts(gpu, M, N, K, r, odd):
+    _say(f"[generic products] M={M} N={N} K={K} r={r} odd={odd}")
+    check_all(gpu, M, N, K, r, odd)
+
+
+@pytest.mark.parametrize("M,N,K,r", [(1, 512, 1024, 4), (64, 256, 512, 1), (200, 384, 256, 12), (300, 520, 192, 20),
+                                     (130, 128, 64, 63), (600, 1024, 1024, 4), (100, 192, 256, 250)])
+def test_ranks_off_8_on_grid_shapes(gpu, M, N, K, r):
+    """Decode, prefill, split-K and rank pre-pass forms on padded factors."""
+    _say(f"[rank off 8] M={M} N={N} K={K} r={r}")
+    check_all(gpu, M, N, K, r)
+
+
+@pytest.mark.parametrize("M,K,r,gn", [(8, 1024, 4, (256, 128)), (200, 256, 12, (256, 256, 128)), (96, 200, 12, (60, 33))])
+def test_grouped_and_shared_base_ranks_off_8(gpu, M, K, r, gn):
+    from weightshared_torchtitan_amd import ops
+    _say(f"[grouped, rank off 8] M={M} K={K} r={r} groups={gn}")
+    G = len(gn)
+    x, w, _, b, _ = inputs(gpu, M, sum(gn), K, r, 5)
+    a = inputs(gpu, M, 8, K, G * r, 6)[2]
+    y = ops.lora_linear_grouped_op(x, w, None, a, b, 2.0, list(gn)).double()
+    n0 = 0
+    for j, n in enumerate(gn):
+        ref = x.double() @ w[n0:n0 + n].double().t() + 2.0 * (x.double() @ a[j * r:(j + 1) * r].double().t()) @ b[n0:n0 + n].double().t()
+        assert rel(y[:, n0:n0 + n], ref) <= TOL
+        n0 += n
+    n = gn[0]
+    bs = torch.cat([inputs(gpu, 1, n, K, r, 9 + j)[3] for j in range(G)])
+    y = ops.lora_linear_bcast_op(x, w[:n // 2], None, a, bs, 2.0, 1, G).double()
+    rows = torch.arange(n, device=gpu) % (n // 2)
+    for j in range(G):
+        ref = x.double() @ w[rows].double().t() + 2.0 * (x.double() @ a[j * r:(j + 1) * r].double().t()) @ bs[j * n:(j + 1) * n].double().t()
+        assert rel(y[:, j * n:(j + 1) * n], ref) <= TOL
+
+
+@pytest.mark.parametrize("M,N,K,r", [(3, 50, 100, 5), (130, 200, 129, 8)])
+def test_generic_fp8_base(gpu, M, N, K, r):
+    from weightshared_torchtitan_amd import ops, quantize_fp8_per_channel
+    _say(f"[generic fp8] M={M} N={N} K={K} r={r}")
+    x, w, a, b, _ = inputs(gpu, M, N, K, r, 3)
+    q, sc = quantize_fp8_per_channel(w)
+    y = ops.lora_linear_op(x, q, sc, a, b, 1.0)
+    ref = x.double() @ (q.double() * sc.double()[:, None]).t() + (x.double() @ a.double().t()) @ b.double().t()
+    assert rel(y, ref) <= TOL
+
+
+def test_nan_stays_in_its_rows_and_columns(gpu):
+    """A NaN or infinity of one row meets only that row's outputs, in products whose tiles are padded."""
+    from weightshared_torchtitan_amd import ops
+    x, w, a, b, gy = inputs(gpu, 70, 100, 100, 5, 4)
+    x[3, 99] = float("nan")
+    w[7, 2] = float("inf")
+    y = ops.lora_linear_op(x, w, None, a, b, 2.0)
+    bad = ~y.isfinite()
+    assert bool(bad[3].all()) and bool(bad[:, 7].all())
+    bad[3] = False
+    bad[:, 7] = False
+    assert not bad.any()

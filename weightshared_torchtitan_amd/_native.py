@@ -50,6 +50,9 @@ EXPORTED = (
     "wsl_lora_linear_bwd_input_supported",
     "wsl_lora_linear_bwd_input_workspace_bytes",
     "wsl_lora_linear_bwd_input",
+    "wsl_lora_linear_bwd_input_any_workspace_bytes",
+    "wsl_lora_linear_bwd_input_any",
+    "wsl_lora_pad_rank",
     "wsl_factorized_embedding_fwd",
     "wsl_last_error",
     "wsl_version",
@@ -237,6 +240,24 @@ def _declare(lib: ctypes.CDLL) -> None:
         _c_vp, ctypes.c_size_t,          # workspace, bytes
         _c_vp,                           # stream
     ]
+    lib.wsl_lora_linear_bwd_input_any_workspace_bytes.restype = ctypes.c_int
+    lib.wsl_lora_linear_bwd_input_any_workspace_bytes.argtypes = [_c_i64, _c_i64, _c_i64, _c_i64,
+                                                                  ctypes.POINTER(ctypes.c_size_t)]
+    lib.wsl_lora_linear_bwd_input_any.restype = ctypes.c_int
+    lib.wsl_lora_linear_bwd_input_any.argtypes = [
+        _c_vp, _c_i64, _c_vp, _c_i64,    # gy, ldg, w, ldw
+        _c_vp, _c_i64, _c_vp, _c_i64,    # a, lda, b, ldb
+        ctypes.c_float,                  # scale
+        _c_vp, _c_i64,                   # dx, lddx
+        _c_i64, _c_i64, _c_i64, _c_i64,  # M, N, K, r
+        _c_vp, ctypes.c_size_t,          # workspace, bytes
+        _c_vp,                           # stream
+    ]
+    lib.wsl_lora_pad_rank.restype = ctypes.c_int
+    lib.wsl_lora_pad_rank.argtypes = [
+        _c_vp, _c_i64, _c_vp, _c_i64,                  # a, lda, b, ldb
+        ctypes.c_int32, _c_i64, _c_i64, _c_i64, _c_i64,  # n_groups, r, r_padded, K, N
+        _c_vp, _c_vp, _c_vp]                           # a_out, b_out, stream
     lib.wsl_decode_last_error.restype = ctypes.c_char_p
     lib.wsl_decode_last_error.argtypes = []
     lib.wsl_rmsnorm_fwd.restype = ctypes.c_int
@@ -388,6 +409,13 @@ def bwd_input_workspace_bytes(M: int, N: int, K: int, r: int) -> int:
     out = ctypes.c_size_t(0)
     check(lib().wsl_lora_linear_bwd_input_workspace_bytes(M, N, K, r, ctypes.byref(out)),
           "wsl_lora_linear_bwd_input_workspace_bytes")
+    return int(out.value)
+
+
+def bwd_input_any_workspace_bytes(M: int, N: int, K: int, r: int) -> int:
+    out = ctypes.c_size_t(0)
+    check(lib().wsl_lora_linear_bwd_input_any_workspace_bytes(M, N, K, r, ctypes.byref(out)),
+          "wsl_lora_linear_bwd_input_any_workspace_bytes")
     return int(out.value)
 
 

@@ -697,6 +697,64 @@ int wsl_lora_linear_bwd_input(const void* gy, int64_t ldg, const void* w, int64_
   return WSL_OK;
 }
 
+int wsl_lora_linear_bwd_input_any_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t r, size_t* bytes) {
+  clear_err();
+  if (bytes == nullptr) return fail(WSL_E_INVALID_ARG, "bytes must not be NULL");
+  const int rc = validate_sizes(M, N, K, r, WSL_DTYPE_BF16);
+  if (rc != WSL_OK) return rc;
+  *bytes = layout_bytes(generic_data(M, r));
+  return WSL_OK;
+}
+
+int wsl_lora_linear_bwd_input_any(const void* gy, int64_t ldg, const void* w, int64_t ldw, const void* a, int64_t lda,
+                                  const void* b, int64_t ldb, float scale, void* dx, int64_t lddx, int64_t M,
+                                  int64_t N, int64_t K, int64_t r, void* workspace, size_t workspace_bytes,
+                                  void* stream) {
+  clear_err();
+  int rc = validate_sizes(M, N, K, r, WSL_DTYPE_BF16);
+  if (rc != WSL_OK) return rc;
+  if (M == 0) return WSL_OK;
+  if (gy == nullptr || w == nullptr || dx == nullptr) return fail(WSL_E_INVALID_ARG, "gy, w and dx must not be NULL");
+  if (r > 0 && (a == nullptr || b == nullptr)) return fail(WSL_E_INVALID_ARG, "r > 0 needs a and b");
+  if (ldg < N || ldw < K || lddx < K || (r > 0 && (lda < K || ldb < r)))
+    return fail(WSL_E_SHAPE, "a leading dimension is below its row length");
+  if (((uintptr_t)gy & 1) || ((uintptr_t)w & 1) || ((uintptr_t)dx & 1) || ((uintptr_t)a & 1) || ((uintptr_t)b & 1))
+    return fail(WSL_E_ALIGN, "pointers must be aligned to their element size");
+  const size_t need = generic_data(M, r);
+  if (workspace == nullptr || workspace_bytes < layout_bytes(need))
+    return fail(WSL_E_WORKSPACE, "workspace of %zu bytes required (got %zu)", layout_bytes(need), workspace_bytes);
+  if ((uintptr_t)workspace & 255) return fail(WSL_E_ALIGN, "workspace must be 256-byte aligned");
+  rc = check_device();
+  if (rc != WSL_OK) return rc;
+  const wsl::LoraArgs p =
+      bwd_input_args(gy, ldg, w, ldw, WSL_DTYPE_BF16, nullptr, a, lda, b, ldb, scale, dx, lddx, M, N, K, r, stream);
+  const hipError_t e = wsl::launch_bwd_input_generic(
+      p, reinterpret_cast<uint16_t*>(reinterpret_cast<char*>(workspace) + wsl::kCounterBytes + half_of(workspace_bytes)));
+  if (e != hipSuccess) return fail(WSL_E_LAUNCH, "kernel launch failed: %s", hipGetErrorString(e));
+  return WSL_OK;
+}
+
+int wsl_lora_pad_rank(const void* a, int64_t lda, const void* b, int64_t ldb, int32_t n_groups, int64_t r,
+                      int64_t r_padded, int64_t K, int64_t N, void* a_out, void* b_out, void* stream) {
+  clear_err();
+  if (n_groups < 1 || n_groups > WSL_MAX_GROUPS)
+    return fail(WSL_E_SHAPE, "n_groups must be in [1, %d] (got %d)", WSL_MAX_GROUPS, (int)n_groups);
+  const int rc = validate_sizes(0, N, K, r_padded, WSL_DTYPE_BF16);
+  if (rc != WSL_OK) return rc;
+  if (r < 1 || r > r_padded || lda < K || ldb < r)
+    return fail(WSL_E_SHAPE, "need 1 <= r <= r_padded, lda >= K and ldb >= r");
+  if (a == nullptr || b == nullptr || a_out == nullptr || b_out == nullptr)
+    return fail(WSL_E_INVALID_ARG, "pointers must not be NULL");
+  if (((uintptr_t)a & 1) || ((uintptr_t)b & 1) || ((uintptr_t)a_out & 1) || ((uintptr_t)b_out & 1))
+    return fail(WSL_E_ALIGN, "pointers must be aligned to their element size");
+  const int dc = check_device();
+  if (dc != WSL_OK) return dc;
+  const hipError_t e = wsl::launch_pad_rank(a, lda, b, ldb, n_groups, r, r_padded, K, N, a_out, b_out,
+                                            reinterpret_cast<hipStream_t>(stream));
+  if (e != hipSuccess) return fail(WSL_E_LAUNCH, "kernel launch failed: %s", hipGetErrorString(e));
+  return WSL_OK;
+}
+
 int wsl_lora_linear_fused_supported(int64_t M, int64_t N, int64_t K, int64_t r, int32_t fuse) {
   const bool sizes_ok = validate_sizes(M, N, K, r, WSL_DTYPE_BF16) == WSL_OK && M >= 1;
   clear_err();  // a query leaves no error behind

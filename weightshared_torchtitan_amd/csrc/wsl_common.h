@@ -239,7 +239,17 @@ bool decode_argmax_supported(const LoraArgs& p);
 size_t decode_argmax_keys_bytes(int64_t M);
 hipError_t launch_decode_argmax(const LoraArgs& p, void* keys, int64_t* out);
 
+// The same contracts on any layout (csrc/lora_generic.hip): the forward, the weight gradients by
+// the token route (t, u: [M, r] bf16 scratch) and the input gradient (bf16 W; u as before).
 hipError_t launch_generic(const LoraArgs& p);
+hipError_t launch_weight_grads_generic(const LoraArgs& p, const void* gy, int64_t ldg, void* dw, int64_t lddw,
+                                       void* da, int64_t ldda, void* db, int64_t lddb, int64_t r, uint16_t* t,
+                                       uint16_t* u);
+hipError_t launch_bwd_input_generic(const LoraArgs& p, uint16_t* u);
+// a [groups * r, K] and b [N, r] with each group's rows of a and the columns of b padded with
+// zeros to rank rp: a_out [groups * rp, K], b_out [N, rp].
+hipError_t launch_pad_rank(const void* a, int64_t lda, const void* b, int64_t ldb, int groups, int64_t r, int64_t rp,
+                           int64_t K, int64_t N, void* a_out, void* b_out, hipStream_t st);
 
 hipError_t launch_factorized_embedding(const int64_t* ids, int64_t n_ids, const void* emb,
                                        int64_t lde, int64_t vocab, int64_t k, const void* proj,

@@ -130,6 +130,33 @@ def workspace(dev: torch.device, stream: int, nbytes: int, kind: str = "lora") -
     return buf
 
 
+def _rows16(t: torch.Tensor) -> bool:
+    """Whether every row of a 2-D bf16 tensor starts on 16 bytes."""
+    return t.data_ptr() % 16 == 0 and t.stride(0) % 8 == 0
+
+
+def _pads_rank(r: int, x: torch.Tensor, K: int) -> bool:
+    """Whether LoRA factors of rank r on x [M, K] go padded to a multiple of 8: where the tiled
+    kernels then take the call (its reduction on their grid, its rows aligned), and below 8, where
+    the generic products would load the factors' short rows one element at a time."""
+    return r % 8 != 0 and (r < 8 or (K % 64 == 0 and _rows16(x)))
+
+
+def _pad_rank(a: torch.Tensor, b: torch.Tensor, groups: int) -> tuple[torch.Tensor, torch.Tensor, int]:
+    """a [groups * r, K] and b [N, r] with zeros up to the next rank in multiples of 8, and that
+    rank (one launch): the same LoRA term, on factors whose rows the tiled kernels take."""
+    N, r = b.shape
+    K, rp = a.shape[1], (r + 7) // 8 * 8
+    both = torch.empty(groups * rp * K + N * rp, dtype=torch.bfloat16, device=b.device)
+    ap, bp = both[:groups * rp * K].view(groups * rp, K), both[groups * rp * K:].view(N, rp)
+    with torch.cuda.device(b.device):
+        rc = _native.lib().wsl_lora_pad_rank(a.data_ptr(), a.stride(0), b.data_ptr(), b.stride(0), groups, r, rp, K, N,
+                                             ap.data_ptr(), bp.data_ptr(),
+                                             torch.cuda.current_stream(b.device).cuda_stream)
+    _native.check(rc, "wsl_lora_pad_rank")
+    return ap, bp, rp
+
+
 def _out_features(w: Optional[torch.Tensor], b: Optional[torch.Tensor]) -> int:
     if w is not None:
         return w.shape[0]
@@ -180,6 +207,8 @@ def lora_linear_op(x: torch.Tensor, w: Optional[torch.Tensor], w_scale: Optional
             raise TypeError("a and b must be bfloat16")
     y = torch.empty((M, N), dtype=torch.bfloat16, device=dev)
     if M > 0:
+        if _pads_rank(r, x2, K):
+            a, b, r = _pad_rank(a, b, 1)
         ws_bytes = _native.workspace_bytes(M, N, K, r, w_dtype)
         stream = torch.cuda.current_stream(dev).cuda_stream
         ws = workspace(dev, stream, ws_bytes)
@@ -212,8 +241,9 @@ def lora_linear_bwd_input_op(gy: torch.Tensor, w: torch.Tensor, w_scale: Optiona
     float8_e4m3fn with w_scale [N] fp32: W = bf16(w * w_scale[:, None]) row by row),
     a [r, K] and b [N, r] as the forward takes them (a and b None: r = 0):
     wsl_lora_linear_bwd_input, the fused kernel reading w where it lies as the reduction rows
-    of its tiles. Layouts that entry point does not take (N off the 64 grid, K or r off 8,
-    unaligned rows) run the forward op on a transposed copy of W."""
+    of its tiles. Ranks off 8 are padded with zeros. Layouts that entry point does not take (N off
+    the 64 grid, K off 8, unaligned rows) run on wsl_lora_linear_bwd_input_any, or, where the
+    forward's tiled kernels take the transposed problem, the forward op on a copy of W^T."""
     dev = _check_device(gy, w, w_scale, a, b)
     gy2 = _row_major(gy.reshape(-1, gy.shape[-1]), "grad_y")
     w = _row_major(w, "w")
@@ -243,9 +273,21 @@ def lora_linear_bwd_input_op(gy: torch.Tensor, w: torch.Tensor, w_scale: Optiona
     L = _native.lib()
     wdt = _native.WSL_DTYPE_FP8_E4M3 if fp8 else _native.WSL_DTYPE_BF16
     ws_ptr = w_scale.data_ptr() if fp8 else None
+    if _pads_rank(r, gy2, N):
+        a, b, r = _pad_rank(a, b, 1)
     if not L.wsl_lora_linear_bwd_input_supported(gy2.data_ptr(), gy2.stride(0), w.data_ptr(), w.stride(0), wdt,
                                                  ws_ptr, _dev_ptr(a), a.stride(0) if r else 0, _dev_ptr(b),
                                                  b.stride(0) if r else 0, dx.data_ptr(), K, M, N, K, r):
+        if not fp8 and not (N % 64 == 0 and K % 4 == 0 and _rows16(gy2)):
+            stream = torch.cuda.current_stream(dev).cuda_stream
+            ws = workspace(dev, stream, _native.bwd_input_any_workspace_bytes(M, N, K, r))
+            with torch.cuda.device(dev):
+                rc = L.wsl_lora_linear_bwd_input_any(
+                    gy2.data_ptr(), gy2.stride(0), w.data_ptr(), w.stride(0), _dev_ptr(a), a.stride(0) if r else 0,
+                    _dev_ptr(b), b.stride(0) if r else 0, float(scale), dx.data_ptr(), K, M, N, K, r, ws.data_ptr(),
+                    ws.numel(), stream)
+            _native.check(rc, "wsl_lora_linear_bwd_input_any")
+            return dx
         wt = ((w.float() * w_scale[:, None]).to(torch.bfloat16) if fp8 else w).t().contiguous()
         return lora_linear_op(gy2, wt, None, b.t().contiguous() if r else None, a.t().contiguous() if r else None,
                               float(scale))
@@ -278,8 +320,8 @@ def lora_linear_weight_grads_op(x: torch.Tensor, gy: torch.Tensor, a: Optional[t
     """dw = gy^T . x [N, K], da = scale (gy . b)^T . x [r, K], db = scale gy^T . (x . a^T)
     [N, r], each only when asked for (else an empty tensor), bf16 from bf16 x [M, K],
     gy [M, N], a [r, K], b [N, r] (wsl_lora_linear_bwd_weights: dW over the tokens on the
-    fused kernel's tile loop, reading x and gy as they lie, da and db from dW; layouts off
-    the tile grid on the library's scalar kernels)."""
+    fused kernel's tile loop, reading x and gy as they lie, da and db from dW; ranks off 8 padded
+    with zeros, layouts off the tile grid on the library's generic products)."""
     dev = _check_device(x, gy, a, b)
     x2 = _row_major(x.reshape(-1, x.shape[-1]), "x")
     gy2 = _row_major(gy.reshape(-1, gy.shape[-1]), "grad_y")
@@ -305,6 +347,9 @@ def lora_linear_weight_grads_op(x: torch.Tensor, gy: torch.Tensor, a: Optional[t
         return (x2.new_zeros(N, K) if need_w else empty(), x2.new_zeros(r, K) if need_a else empty(),
                 x2.new_zeros(N, r) if need_b else empty())
     L = _native.lib()
+    r0 = r
+    if _pads_rank(r, x2, K) and (r < 8 or (N % 64 == 0 and _rows16(gy2))):
+        a, b, r = _pad_rank(a, b, 1)
     dw = torch.empty((N, K), dtype=torch.bfloat16, device=dev) if need_w else None
     da = torch.empty((r, K), dtype=torch.bfloat16, device=dev) if need_a else None
     db = torch.empty((N, r), dtype=torch.bfloat16, device=dev) if need_b else None
@@ -318,6 +363,8 @@ def lora_linear_weight_grads_op(x: torch.Tensor, gy: torch.Tensor, a: Optional[t
             _dev_ptr(dw), K, _dev_ptr(da), K, _dev_ptr(db), r,
             ws.data_ptr(), ws.numel(), stream)
     _native.check(rc, "wsl_lora_linear_bwd_weights")
+    if r != r0:  # the padding's rows and columns of the gradients are zeros
+        da, db = da[:r0] if need_a else None, db[:, :r0].contiguous() if need_b else None
     return dw if need_w else empty(), da if need_a else empty(), db if need_b else empty()
 
 
@@ -434,6 +481,8 @@ def lora_linear_grouped_op(x: torch.Tensor, w: torch.Tensor, w_scale: Optional[t
             raise TypeError("a and b must be bfloat16")
     y = torch.empty((M, N), dtype=torch.bfloat16, device=dev)
     if M > 0:
+        if _pads_rank(r, x2, K):
+            a, b, r = _pad_rank(a, b, G)
         gn = _native.group_array(group_n)
         ws_bytes = _native.grouped_workspace_bytes(M, K, r, group_n, w_dtype)
         stream = torch.cuda.current_stream(dev).cuda_stream
@@ -508,6 +557,8 @@ def lora_linear_bcast_op(x: torch.Tensor, w: torch.Tensor, w_scale: Optional[tor
         raise ValueError(f"broadcast needs N % base_n == 0 and base_n % g == 0 (N {N}, base_n {base_n}, g {g})")
     y = torch.empty((M, G * N), dtype=torch.bfloat16, device=dev)
     if M > 0:
+        if _pads_rank(r, x2, K):
+            a, b, r = _pad_rank(a, b, G)
         stream = torch.cuda.current_stream(dev).cuda_stream
         ws = workspace(dev, stream, _native.bcast_workspace_bytes(M, N, K, r, G, w_dtype))
         with torch.cuda.device(dev):
