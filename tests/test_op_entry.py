@@ -1,0 +1,132 @@
+"""Calls of the ops go straight to their implementation only where nothing but the kernel has a
+part in them (ops._Op): every torch mechanism that must see a dispatched op still does, recorded
+calls have the gradients of the dispatched op, and mutated operands' versions count up."""
+import pytest
+import torch
+from torch._subclasses.fake_tensor import FakeTensorMode
+from torch.utils._python_dispatch import TorchDispatchMode
+
+from weightshared_torchtitan_amd import ops
+
+
+class Seen(TorchDispatchMode):
+    def __init__(self):
+        super().__init__()
+        self.names = []
+
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        self.names.append(str(func))
+        return func(*args, **(kwargs or {}))
+
+
+def test_mechanisms_that_need_the_dispatcher_are_seen():
+    assert not ops._dispatcher_only()
+    with Seen():
+        assert ops._dispatcher_only()
+    with FakeTensorMode():
+        assert ops._dispatcher_only()
+    with torch.device("meta"):
+        assert ops._dispatcher_only()
+    with torch.autocast("cpu", dtype=torch.bfloat16):
+        assert ops._dispatcher_only()
+    with torch.autograd.forward_ad.dual_level():
+        assert ops._dispatcher_only()
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]):
+        assert ops._dispatcher_only()
+    seen = []
+    torch.func.vmap(lambda t: (seen.append(ops._dispatcher_only()), t)[1])(torch.zeros(2))
+    torch.func.grad(lambda t: (seen.append(ops._dispatcher_only()), t.sum())[1])(torch.zeros(2))
+    torch.jit.trace(lambda t: (seen.append(ops._dispatcher_only()), t + 1)[1], torch.zeros(2), check_trace=False)
+    assert seen == [True] * 3
+    assert not ops._dispatcher_only()
+
+
+def test_tensors_off_the_gpu_and_subclasses_go_to_the_dispatcher(monkeypatch):
+    monkeypatch.setattr(ops.swiglu_op, "_fn", lambda *a: pytest.fail("called directly"))
+    with pytest.raises((RuntimeError, NotImplementedError)):
+        ops.swiglu_op(torch.zeros(2, 16, dtype=torch.bfloat16))
+    assert ops.swiglu_op(torch.zeros(2, 16, dtype=torch.bfloat16, device="meta")).shape == (2, 8)
+    assert ops.swiglu_op(gate_up=torch.zeros(2, 16, dtype=torch.bfloat16, device="meta")).shape == (2, 8)
+
+
+def _args(gpu, grad):
+    g = torch.Generator(device="cuda").manual_seed(0)
+    mk = lambda *s: torch.randn(*s, device=gpu, generator=g).bfloat16().requires_grad_(grad)  # noqa: E731
+    return mk(2, 50, 256), mk(384, 256), None, mk(24, 256), mk(384, 8)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,tail", [("lora_linear", (2.0,)), ("lora_linear_grouped", (2.0, [128, 128, 128])),
+                                       ("lora_linear_bcast", (2.0, 1, 1))])
+def test_direct_calls_equal_dispatched_ones(gpu, name, tail):
+    x, w, ws, a, b = _args(gpu, True)
+    if name != "lora_linear_grouped":
+        a = a[:8].detach().requires_grad_()
+    direct, op = getattr(ops, name + "_op"), getattr(torch.ops.wsl, name)
+    gy = torch.randn(2, 50, 384, device=gpu).bfloat16()
+    got = []
+    for f in (direct, op):
+        packed = []
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: (packed.append(t.shape), t)[1], lambda t: t):
+            y = f(x, w, ws, a, b, *tail)
+        assert len(packed) == 4
+        got.append([y, *torch.autograd.grad(y, [x, w, a, b], gy)])
+        with torch.no_grad():
+            got[-1].append(f(x, w, ws, a, b, *tail))
+        assert not got[-1][-1].requires_grad and y.requires_grad
+        for needs in ([x], [b], [a, w]):  # any subset of the inputs
+            ins = [t if any(t is n for n in needs) else t.detach() for t in (x, w, a, b)]
+            y = f(ins[0], ins[1], ws, ins[2], ins[3], *tail)
+            got[-1] += torch.autograd.grad(y, needs, gy)
+    for p, q in zip(*got):
+        assert torch.equal(p, q)
+
+
+@pytest.mark.gpu
+def test_transforms_see_the_op(gpu):
+    x, w, _, a, b = _args(gpu, False)
+    a = a[:8]
+    want = ops.lora_linear_op(x, w, None, a, b, 2.0)
+    with Seen() as s:
+        assert torch.equal(ops.lora_linear_op(x, w, None, a, b, 2.0), want)
+    assert any("wsl.lora_linear" in n for n in s.names)
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        assert torch.equal(ops.lora_linear_op(x.float(), w.float(), None, a, b, 2.0), want)
+    with torch.autograd.forward_ad.dual_level():
+        dual = torch.autograd.forward_ad.make_dual(x, torch.ones_like(x))
+        out = []
+        for f in (ops.lora_linear_op, torch.ops.wsl.lora_linear):  # neither drops the tangent in silence
+            try:
+                out.append(torch.autograd.forward_ad.unpack_dual(f(dual, w, None, a, b, 2.0)).tangent is None)
+            except (RuntimeError, NotImplementedError):
+                out.append("raised")
+        assert out[0] == out[1]
+
+
+@pytest.mark.gpu
+def test_mutated_operands_count_up(gpu):
+    k = torch.randn(8, 128, device=gpu).bfloat16()
+    kc = torch.zeros(2, 2, 4, 64, device=gpu, dtype=torch.bfloat16)
+    vc = kc.clone()
+    rope = torch.zeros(4, 128, device=gpu)
+    kw = torch.ones(64, device=gpu, dtype=torch.bfloat16)
+    for f in (ops.kv_norm_rope_op, torch.ops.wsl.kv_norm_rope):
+        before = kc._version, vc._version, k._version
+        f(k, k, kw, 1e-6, rope, kc, vc)
+        assert kc._version > before[0] and vc._version > before[1] and k._version == before[2]
+    with torch.inference_mode():
+        ops.kv_norm_rope_op(k, k, kw, 1e-6, rope, torch.zeros_like(kc), torch.zeros_like(vc))
+
+
+@pytest.mark.gpu
+def test_calls_follow_the_current_stream(gpu):
+    x, w, _, a, b = _args(gpu, False)
+    a = a[:8]
+    want = ops.lora_linear_op(x, w, None, a, b, 2.0)
+    torch.cuda.synchronize()
+    s = torch.cuda.Stream()
+    with torch.cuda.stream(s):
+        assert ops._stream(x.device) == s.cuda_stream
+        y = ops.lora_linear_op(x, w, None, a, b, 2.0)
+    s.synchronize()
+    assert ops._stream(x.device) == torch.cuda.current_stream().cuda_stream and torch.equal(y, want)

@@ -15,6 +15,8 @@ from typing import Optional
 
 import contextlib
 import ctypes
+import functools
+import inspect
 import os
 
 import torch
@@ -88,6 +90,96 @@ def _check_device(*ts: Optional[torch.Tensor]) -> torch.device:
     return dev
 
 
+# ------------------------------------------------------------------------------------------
+# Op entry. Every op is a torch custom op (traced, transformed, autocast and profiled by torch's
+# dispatcher). Its dispatch through Python costs 7 us a call (and a recorded call about 15 more),
+# as much as a decode launch takes on the GPU, so a call that nothing but the kernel has a part in
+# goes straight to the op's implementation, and one that only autograd has, to the same formulas
+# as a torch.autograd.Function.
+# ------------------------------------------------------------------------------------------
+_PLAIN_TYPES = (torch.Tensor, torch.nn.Parameter)
+
+
+_is_compiling, _grad_on = torch.compiler.is_compiling, torch.is_grad_enabled
+_dispatch_modes, _function_modes = torch._C._len_torch_dispatch_stack, torch._C._len_torch_function_stack
+_transforms, _tracing = torch._C._functorch.peek_interpreter_stack, torch._C._is_tracing
+_autocast, _profiling = torch._C._is_any_autocast_enabled, torch._C._autograd._profiler_enabled
+_forward_ad = torch.autograd.forward_ad
+
+
+def _dispatcher_only() -> bool:
+    """Whether something in force must see calls as dispatched ops: tracing and compilation, torch
+    modes, functorch transforms, autocast, forward-mode AD, a profiler."""
+    return (_is_compiling() or _dispatch_modes() != 0 or _function_modes() != 0 or _autocast()
+            or _transforms() is not None or _tracing() or _forward_ad._current_level >= 0 or _profiling())
+
+
+class _Op:
+    """A ``torch.library.custom_op`` named wsl::`name` over `fn` (called through torch.ops.wsl as
+    any other), with the direct routes above for its own callers."""
+
+    def __init__(self, name: str, fn, mutates_args=()):
+        self._fn = fn
+        self._def = torch.library.custom_op(f"wsl::{name}", fn, mutates_args=mutates_args, device_types="cuda")
+        self._op = getattr(torch.ops.wsl, name).default
+        params = list(inspect.signature(fn).parameters.values())
+        self._tensors = tuple(i for i, q in enumerate(params) if q.annotation in ("torch.Tensor", "Optional[torch.Tensor]"))
+        self._mutates = tuple(i for i, q in enumerate(params) if q.name in mutates_args)
+        self._n = len(params)
+        self._function = None
+        functools.update_wrapper(self, fn)
+
+    def __call__(self, *args, **kwargs):
+        if _dispatcher_only() or kwargs or len(args) != self._n:
+            return self._op(*args, **kwargs)
+        recorded = False
+        grad = _grad_on()
+        for i in self._tensors:
+            t = args[i]
+            if t is None:
+                continue
+            if type(t) not in _PLAIN_TYPES or not t.is_cuda:
+                return self._op(*args)
+            if grad and t.requires_grad:
+                recorded = True
+        if recorded:
+            return self._function.apply(*args) if self._function is not None else self._op(*args)
+        for i in self._mutates:
+            if not args[i].is_inference():
+                torch.autograd.graph.increment_version(args[i])
+        return self._fn(*args)
+
+    def register_fake(self, fn):
+        return self._def.register_fake(fn)
+
+    def register_autograd(self, backward, setup_context) -> None:
+        self._def.register_autograd(backward, setup_context=setup_context)
+        impl = self._fn
+
+        def forward(ctx, *args):
+            setup_context(ctx, args, None)
+            return impl(*args)
+
+        self._function = type(f"Wsl_{self._fn.__name__}", (torch.autograd.Function,),
+                              {"forward": staticmethod(forward), "backward": staticmethod(backward)})
+
+
+def _custom_op(name: str, mutates_args=()):
+    return lambda fn: _Op(name, fn, mutates_args)
+
+
+_NO_GUARD = contextlib.nullcontext()
+
+
+def _on(dev: torch.device):
+    """A guard that makes `dev` the current device (nothing to do where it is)."""
+    return _NO_GUARD if torch.cuda.current_device() == dev.index else torch.cuda.device(dev)
+
+
+def _stream(dev: torch.device) -> int:
+    return torch._C._cuda_getCurrentRawStream(dev.index)
+
+
 _WS_MIN_BYTES = 16 << 20
 _workspaces: dict = {}
 # Workspaces that were replaced (grown, or dropped after a failed launch). A HIP graph
@@ -149,10 +241,10 @@ def _pad_rank(a: torch.Tensor, b: torch.Tensor, groups: int) -> tuple[torch.Tens
     K, rp = a.shape[1], (r + 7) // 8 * 8
     both = torch.empty(groups * rp * K + N * rp, dtype=torch.bfloat16, device=b.device)
     ap, bp = both[:groups * rp * K].view(groups * rp, K), both[groups * rp * K:].view(N, rp)
-    with torch.cuda.device(b.device):
+    with _on(b.device):
         rc = _native.lib().wsl_lora_pad_rank(a.data_ptr(), a.stride(0), b.data_ptr(), b.stride(0), groups, r, rp, K, N,
                                              ap.data_ptr(), bp.data_ptr(),
-                                             torch.cuda.current_stream(b.device).cuda_stream)
+                                             _stream(b.device))
     _native.check(rc, "wsl_lora_pad_rank")
     return ap, bp, rp
 
@@ -165,7 +257,7 @@ def _out_features(w: Optional[torch.Tensor], b: Optional[torch.Tensor]) -> int:
     raise ValueError("lora_linear needs w or (a, b)")
 
 
-@torch.library.custom_op("wsl::lora_linear", mutates_args=(), device_types="cuda")
+@_custom_op("lora_linear")
 def lora_linear_op(x: torch.Tensor, w: Optional[torch.Tensor], w_scale: Optional[torch.Tensor],
                    a: Optional[torch.Tensor], b: Optional[torch.Tensor],
                    scale: float) -> torch.Tensor:
@@ -210,9 +302,9 @@ def lora_linear_op(x: torch.Tensor, w: Optional[torch.Tensor], w_scale: Optional
         if _pads_rank(r, x2, K):
             a, b, r = _pad_rank(a, b, 1)
         ws_bytes = _native.workspace_bytes(M, N, K, r, w_dtype)
-        stream = torch.cuda.current_stream(dev).cuda_stream
+        stream = _stream(dev)
         ws = workspace(dev, stream, ws_bytes)
-        with torch.cuda.device(dev):
+        with _on(dev):
             rc = _native.lib().wsl_lora_linear_fwd(
                 x2.data_ptr(), x2.stride(0),
                 _dev_ptr(w), w.stride(0) if w is not None else 0, w_dtype, _dev_ptr(w_scale),
@@ -234,7 +326,7 @@ def _lora_linear_fake(x, w, w_scale, a, b, scale):
     return x.new_empty((*x.shape[:-1], N), dtype=torch.bfloat16)
 
 
-@torch.library.custom_op("wsl::lora_linear_bwd_input", mutates_args=(), device_types="cuda")
+@_custom_op("lora_linear_bwd_input")
 def lora_linear_bwd_input_op(gy: torch.Tensor, w: torch.Tensor, w_scale: Optional[torch.Tensor],
                              a: Optional[torch.Tensor], b: Optional[torch.Tensor], scale: float) -> torch.Tensor:
     """dx [M, K] = gy . W + scale * (gy . b) . a for bf16 gy [M, N], w [N, K] (bf16, or
@@ -279,9 +371,9 @@ def lora_linear_bwd_input_op(gy: torch.Tensor, w: torch.Tensor, w_scale: Optiona
                                                  ws_ptr, _dev_ptr(a), a.stride(0) if r else 0, _dev_ptr(b),
                                                  b.stride(0) if r else 0, dx.data_ptr(), K, M, N, K, r):
         if not fp8 and not (N % 64 == 0 and K % 4 == 0 and _rows16(gy2)):
-            stream = torch.cuda.current_stream(dev).cuda_stream
+            stream = _stream(dev)
             ws = workspace(dev, stream, _native.bwd_input_any_workspace_bytes(M, N, K, r))
-            with torch.cuda.device(dev):
+            with _on(dev):
                 rc = L.wsl_lora_linear_bwd_input_any(
                     gy2.data_ptr(), gy2.stride(0), w.data_ptr(), w.stride(0), _dev_ptr(a), a.stride(0) if r else 0,
                     _dev_ptr(b), b.stride(0) if r else 0, float(scale), dx.data_ptr(), K, M, N, K, r, ws.data_ptr(),
@@ -291,9 +383,9 @@ def lora_linear_bwd_input_op(gy: torch.Tensor, w: torch.Tensor, w_scale: Optiona
         wt = ((w.float() * w_scale[:, None]).to(torch.bfloat16) if fp8 else w).t().contiguous()
         return lora_linear_op(gy2, wt, None, b.t().contiguous() if r else None, a.t().contiguous() if r else None,
                               float(scale))
-    stream = torch.cuda.current_stream(dev).cuda_stream
+    stream = _stream(dev)
     ws = workspace(dev, stream, _native.bwd_input_workspace_bytes(M, N, K, r))
-    with torch.cuda.device(dev):
+    with _on(dev):
         rc = L.wsl_lora_linear_bwd_input(gy2.data_ptr(), gy2.stride(0), w.data_ptr(), w.stride(0), wdt, ws_ptr,
                                          _dev_ptr(a), a.stride(0) if r else 0, _dev_ptr(b), b.stride(0) if r else 0,
                                          float(scale), dx.data_ptr(), K, M, N, K, r, ws.data_ptr(), ws.numel(),
@@ -313,7 +405,7 @@ def _input_grad(gy2, w, w_scale, a, b, s):
     return lora_linear_bwd_input_op(gy2, w, w_scale if w.dtype == _FP8 else None, a, b, float(s))
 
 
-@torch.library.custom_op("wsl::lora_linear_weight_grads", mutates_args=(), device_types="cuda")
+@_custom_op("lora_linear_weight_grads")
 def lora_linear_weight_grads_op(x: torch.Tensor, gy: torch.Tensor, a: Optional[torch.Tensor],
                                 b: Optional[torch.Tensor], scale: float, need_w: bool, need_a: bool,
                                 need_b: bool) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
@@ -353,9 +445,9 @@ def lora_linear_weight_grads_op(x: torch.Tensor, gy: torch.Tensor, a: Optional[t
     dw = torch.empty((N, K), dtype=torch.bfloat16, device=dev) if need_w else None
     da = torch.empty((r, K), dtype=torch.bfloat16, device=dev) if need_a else None
     db = torch.empty((N, r), dtype=torch.bfloat16, device=dev) if need_b else None
-    stream = torch.cuda.current_stream(dev).cuda_stream
+    stream = _stream(dev)
     ws = workspace(dev, stream, _native.bwd_weights_workspace_bytes(M, N, K, r))
-    with torch.cuda.device(dev):
+    with _on(dev):
         rc = L.wsl_lora_linear_bwd_weights(
             x2.data_ptr(), x2.stride(0), gy2.data_ptr(), gy2.stride(0),
             _dev_ptr(a), a.stride(0) if r else 0, _dev_ptr(b), b.stride(0) if r else 0,
@@ -432,7 +524,7 @@ def _lora_linear_backward(ctx, gy):
 lora_linear_op.register_autograd(_lora_linear_backward, setup_context=_lora_linear_setup)
 
 
-@torch.library.custom_op("wsl::lora_linear_grouped", mutates_args=(), device_types="cuda")
+@_custom_op("lora_linear_grouped")
 def lora_linear_grouped_op(x: torch.Tensor, w: torch.Tensor, w_scale: Optional[torch.Tensor],
                            a: Optional[torch.Tensor], b: Optional[torch.Tensor], scale: float,
                            group_n: list[int]) -> torch.Tensor:
@@ -485,9 +577,9 @@ def lora_linear_grouped_op(x: torch.Tensor, w: torch.Tensor, w_scale: Optional[t
             a, b, r = _pad_rank(a, b, G)
         gn = _native.group_array(group_n)
         ws_bytes = _native.grouped_workspace_bytes(M, K, r, group_n, w_dtype)
-        stream = torch.cuda.current_stream(dev).cuda_stream
+        stream = _stream(dev)
         ws = workspace(dev, stream, ws_bytes)
-        with torch.cuda.device(dev):
+        with _on(dev):
             rc = _native.lib().wsl_lora_linear_grouped_fwd(
                 x2.data_ptr(), x2.stride(0),
                 w.data_ptr(), w.stride(0), w_dtype, _dev_ptr(w_scale),
@@ -508,7 +600,7 @@ def _lora_linear_grouped_fake(x, w, w_scale, a, b, scale, group_n):
     return x.new_empty((*x.shape[:-1], sum(int(n) for n in group_n)), dtype=torch.bfloat16)
 
 
-@torch.library.custom_op("wsl::lora_linear_bcast", mutates_args=(), device_types="cuda")
+@_custom_op("lora_linear_bcast")
 def lora_linear_bcast_op(x: torch.Tensor, w: torch.Tensor, w_scale: Optional[torch.Tensor],
                          a: Optional[torch.Tensor], b: Optional[torch.Tensor], scale: float, g: int,
                          n_groups: int) -> torch.Tensor:
@@ -559,9 +651,9 @@ def lora_linear_bcast_op(x: torch.Tensor, w: torch.Tensor, w_scale: Optional[tor
     if M > 0:
         if _pads_rank(r, x2, K):
             a, b, r = _pad_rank(a, b, G)
-        stream = torch.cuda.current_stream(dev).cuda_stream
+        stream = _stream(dev)
         ws = workspace(dev, stream, _native.bcast_workspace_bytes(M, N, K, r, G, w_dtype))
-        with torch.cuda.device(dev):
+        with _on(dev):
             rc = _native.lib().wsl_lora_linear_bcast_fwd(
                 x2.data_ptr(), x2.stride(0), w.data_ptr(), w.stride(0), w_dtype, _dev_ptr(w_scale),
                 _dev_ptr(a), a.stride(0) if a is not None else 0, _dev_ptr(b), b.stride(0) if b is not None else 0,
@@ -750,7 +842,7 @@ def lora_linear_grouped(x: torch.Tensor, ws, as_=None, bs=None, scale: float = 2
     return list(torch.split(y, group_n, dim=-1))
 
 
-@torch.library.custom_op("wsl::factorized_embedding", mutates_args=(), device_types="cuda")
+@_custom_op("factorized_embedding")
 def factorized_embedding_op(ids: torch.Tensor, emb: torch.Tensor, proj: torch.Tensor) -> torch.Tensor:
     """out[..., :] = emb[ids[...], :] . proj^T   (emb [V,k], proj [H,k], bf16)."""
     dev = _check_device(ids, emb, proj)
@@ -767,8 +859,8 @@ def factorized_embedding_op(ids: torch.Tensor, emb: torch.Tensor, proj: torch.Te
     flat = ids.reshape(-1).contiguous()
     out = torch.empty((flat.numel(), H), dtype=torch.bfloat16, device=dev)
     if flat.numel() > 0:
-        stream = torch.cuda.current_stream(dev).cuda_stream
-        with torch.cuda.device(dev):
+        stream = _stream(dev)
+        with _on(dev):
             rc = _native.lib().wsl_factorized_embedding_fwd(
                 flat.data_ptr(), flat.numel(), emb.data_ptr(), emb.stride(0), V, k,
                 proj.data_ptr(), proj.stride(0), H, out.data_ptr(), out.stride(0), stream)
@@ -866,10 +958,6 @@ def factorized_embedding(ids: torch.Tensor, emb: torch.Tensor, proj: torch.Tenso
 # ------------------------------------------------------------------------------------------
 # Decode-step ops of the weight-shared Qwen3 harness (include/wsl_decode.h). GPU only.
 # ------------------------------------------------------------------------------------------
-def _stream(dev: torch.device) -> int:
-    return torch.cuda.current_stream(dev).cuda_stream
-
-
 def _bf16_2d(t: torch.Tensor, name: str) -> torch.Tensor:
     if t.dtype != torch.bfloat16:
         raise TypeError(f"{name} must be bfloat16, got {t.dtype}")
@@ -896,7 +984,7 @@ def _rmsnorm_launch(x, weight, eps, residual):
     w = weight.to(torch.bfloat16).contiguous()
     out = torch.empty((x2.shape[0], dim), dtype=torch.bfloat16, device=dev)
     h = torch.empty_like(out) if residual is not None else None
-    with torch.cuda.device(dev):
+    with _on(dev):
         rc = _native.lib().wsl_rmsnorm_fwd(
             x2.data_ptr(), x2.stride(0), _dev_ptr(r2), r2.stride(0) if r2 is not None else 0,
             w.data_ptr(), float(eps), out.data_ptr(), out.stride(0),
@@ -905,7 +993,7 @@ def _rmsnorm_launch(x, weight, eps, residual):
     return out.view(x.shape), (h.view(x.shape) if h is not None else None)
 
 
-@torch.library.custom_op("wsl::rmsnorm", mutates_args=(), device_types="cuda")
+@_custom_op("rmsnorm")
 def rmsnorm_op(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
     """RMSNorm(x) * weight over the last dimension (bf16 in/out, fp32 arithmetic)."""
     return _rmsnorm_launch(x, weight, eps, None)[0]
@@ -916,7 +1004,7 @@ def _rmsnorm_fake(x, weight, eps):
     return x.new_empty(x.shape, dtype=torch.bfloat16)
 
 
-@torch.library.custom_op("wsl::add_rmsnorm", mutates_args=(), device_types="cuda")
+@_custom_op("add_rmsnorm")
 def add_rmsnorm_op(x: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor,
                    eps: float) -> tuple[torch.Tensor, torch.Tensor]:
     """(RMSNorm(h) * weight, h) with h = bf16(x + residual): the residual add of a block and
@@ -929,7 +1017,7 @@ def _add_rmsnorm_fake(x, residual, weight, eps):
     return x.new_empty(x.shape, dtype=torch.bfloat16), x.new_empty(x.shape, dtype=torch.bfloat16)
 
 
-@torch.library.custom_op("wsl::qk_norm_rope", mutates_args=("k_cache", "v_cache"), device_types="cuda")
+@_custom_op("qk_norm_rope", mutates_args=("k_cache", "v_cache"))
 def qk_norm_rope_op(qkv: torch.Tensor, q_norm_w: torch.Tensor, k_norm_w: torch.Tensor, eps: float,
                     rope: torch.Tensor, pos: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
                     n_heads: int, n_kv_heads: int) -> torch.Tensor:
@@ -946,7 +1034,7 @@ def qk_norm_rope_op(qkv: torch.Tensor, q_norm_w: torch.Tensor, k_norm_w: torch.T
     rope = rope.float().contiguous()
     pos = pos.to(torch.int64).contiguous()
     q = torch.empty((b, n_heads, hd), dtype=torch.bfloat16, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         rc = _native.lib().wsl_qk_norm_rope_fwd(
             q2.data_ptr(), q2.stride(0), b, n_heads, n_kv_heads, hd, qw.data_ptr(), kw.data_ptr(), float(eps),
             rope.data_ptr(), pos.data_ptr(), q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), L, _stream(dev))
@@ -959,7 +1047,7 @@ def _qk_norm_rope_fake(qkv, q_norm_w, k_norm_w, eps, rope, pos, k_cache, v_cache
     return qkv.new_empty((k_cache.shape[0], n_heads, k_cache.shape[3]), dtype=torch.bfloat16)
 
 
-@torch.library.custom_op("wsl::decode_attention", mutates_args=(), device_types="cuda")
+@_custom_op("decode_attention")
 def decode_attention_op(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, pos: torch.Tensor,
                         scale: float) -> torch.Tensor:
     """softmax(q . K^T * scale) . V over cache positions 0..pos; q [b, n_heads, hd],
@@ -972,7 +1060,7 @@ def decode_attention_op(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.T
     out = torch.empty((b, nh * hd), dtype=torch.bfloat16, device=dev)
     nbytes = _native.lib().wsl_decode_attention_workspace_bytes(b, nh, nkv, hd, L)
     part = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=dev)  # partial softmax records
-    with torch.cuda.device(dev):
+    with _on(dev):
         rc = _native.lib().wsl_decode_attention_fwd(
             q.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), b, nh, nkv, hd, L, pos.data_ptr(),
             float(scale), out.data_ptr(), part.data_ptr(), part.numel(), _stream(dev))
@@ -985,14 +1073,14 @@ def _decode_attention_fake(q, k_cache, v_cache, pos, scale):
     return q.new_empty((q.shape[0], q.shape[1] * q.shape[2]), dtype=torch.bfloat16)
 
 
-@torch.library.custom_op("wsl::swiglu", mutates_args=(), device_types="cuda")
+@_custom_op("swiglu")
 def swiglu_op(gate_up: torch.Tensor) -> torch.Tensor:
     """silu(g) * u for gate_up = [g | u] along the last dimension."""
     dev = _check_device(gate_up)
     ffn = gate_up.shape[-1] // 2
     g2 = _bf16_2d(gate_up, "gate_up")
     out = torch.empty((g2.shape[0], ffn), dtype=torch.bfloat16, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         rc = _native.lib().wsl_swiglu_fwd(g2.data_ptr(), g2.stride(0), g2.shape[0], ffn, out.data_ptr(),
                                           out.stride(0), _stream(dev))
     _native.check(rc, "wsl_swiglu_fwd", decode=True)
@@ -1024,7 +1112,7 @@ def _check_prompt(rows: int, k_cache: torch.Tensor, v_cache: torch.Tensor, rope:
     return seq
 
 
-@torch.library.custom_op("wsl::kv_norm_rope", mutates_args=("k_cache", "v_cache"), device_types="cuda")
+@_custom_op("kv_norm_rope", mutates_args=("k_cache", "v_cache"))
 def kv_norm_rope_op(k: torch.Tensor, v: torch.Tensor, k_norm_w: torch.Tensor, eps: float, rope: torch.Tensor,
                     k_cache: torch.Tensor, v_cache: torch.Tensor) -> None:
     """k [b * seq, n_kv_heads * hd] (normed, rotated) and v into the caches [b, n_kv_heads, L, hd]
@@ -1037,7 +1125,7 @@ def kv_norm_rope_op(k: torch.Tensor, v: torch.Tensor, k_norm_w: torch.Tensor, ep
         raise ValueError(f"k {tuple(k2.shape)}, v {tuple(v2.shape)} and k_norm_w {tuple(k_norm_w.shape)} do not match "
                          f"{nkv} heads of {hd}")
     kw = k_norm_w.to(torch.bfloat16).contiguous()
-    with torch.cuda.device(dev):
+    with _on(dev):
         rc = _native.lib().wsl_kv_norm_rope_fwd(
             k2.data_ptr(), k2.stride(0), v2.data_ptr(), v2.stride(0), b, seq, nkv, hd, kw.data_ptr(), float(eps),
             rope.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), L, _stream(dev))
@@ -1049,7 +1137,7 @@ def _kv_norm_rope_fake(k, v, k_norm_w, eps, rope, k_cache, v_cache):
     return None
 
 
-@torch.library.custom_op("wsl::prefill_attention", mutates_args=(), device_types="cuda")
+@_custom_op("prefill_attention")
 def prefill_attention_op(q: torch.Tensor, q_norm_w: torch.Tensor, eps: float, rope: torch.Tensor,
                          k_cache: torch.Tensor, v_cache: torch.Tensor, n_heads: int, scale: float) -> torch.Tensor:
     """Causal attention of a prompt: q [b * seq, n_heads * hd] normed and rotated, against positions
@@ -1062,7 +1150,7 @@ def prefill_attention_op(q: torch.Tensor, q_norm_w: torch.Tensor, eps: float, ro
         raise ValueError(f"q {tuple(q2.shape)} and q_norm_w {tuple(q_norm_w.shape)} do not match {n_heads} heads of {hd}")
     qw = q_norm_w.to(torch.bfloat16).contiguous()
     out = torch.empty((q2.shape[0], n_heads * hd), dtype=torch.bfloat16, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         rc = _native.lib().wsl_prefill_attention_fwd(
             q2.data_ptr(), q2.stride(0), b, seq, n_heads, nkv, hd, qw.data_ptr(), float(eps), rope.data_ptr(),
             k_cache.data_ptr(), v_cache.data_ptr(), L, float(scale), out.data_ptr(), out.stride(0), _stream(dev))
@@ -1075,7 +1163,7 @@ def _prefill_attention_fake(q, q_norm_w, eps, rope, k_cache, v_cache, n_heads, s
     return q.new_empty((q.numel() // q.shape[-1], n_heads * k_cache.shape[3]), dtype=torch.bfloat16)
 
 
-@torch.library.custom_op("wsl::swiglu_pair", mutates_args=(), device_types="cuda")
+@_custom_op("swiglu_pair")
 def swiglu_pair_op(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
     """silu(gate) * up for two tensors of one shape."""
     dev = _check_device(gate, up)
@@ -1083,7 +1171,7 @@ def swiglu_pair_op(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
         raise ValueError(f"gate {tuple(gate.shape)} and up {tuple(up.shape)} differ")
     g2, u2 = _bf16_2d(gate, "gate"), _bf16_2d(up, "up")
     out = torch.empty(g2.shape, dtype=torch.bfloat16, device=dev)
-    with torch.cuda.device(dev):
+    with _on(dev):
         rc = _native.lib().wsl_swiglu_pair_fwd(g2.data_ptr(), g2.stride(0), u2.data_ptr(), u2.stride(0), g2.shape[0],
                                                g2.shape[1], out.data_ptr(), out.stride(0), _stream(dev))
     _native.check(rc, "wsl_swiglu_pair_fwd", decode=True)
@@ -1095,7 +1183,7 @@ def _swiglu_pair_fake(gate, up):
     return gate.new_empty(gate.shape, dtype=torch.bfloat16)
 
 
-@torch.library.custom_op("wsl::argmax_rows", mutates_args=(), device_types="cuda")
+@_custom_op("argmax_rows")
 def argmax_rows_op(x: torch.Tensor) -> torch.Tensor:
     """int64 index of the largest element of each row (first on ties, NaN largest)."""
     dev = _check_device(x)
@@ -1108,7 +1196,7 @@ def argmax_rows_op(x: torch.Tensor) -> torch.Tensor:
     lib = _native.lib()
     stream = _stream(dev)
     ws = workspace(dev, stream, lib.wsl_argmax_rows_workspace_bytes(x2.shape[0], x2.shape[1]), kind="argmax")
-    with torch.cuda.device(dev):
+    with _on(dev):
         rc = lib.wsl_argmax_rows_fwd(x2.data_ptr(), x2.stride(0), x2.shape[0], x2.shape[1], out.data_ptr(),
                                      ws.data_ptr(), ws.numel(), stream)
     if rc == _native.WSL_E_LAUNCH:
@@ -1122,7 +1210,7 @@ def _argmax_rows_fake(x):
     return x.new_empty(x.shape[:-1], dtype=torch.int64)
 
 
-@torch.library.custom_op("wsl::decode_attention_step", mutates_args=("k_cache", "v_cache"), device_types="cuda")
+@_custom_op("decode_attention_step", mutates_args=("k_cache", "v_cache"))
 def decode_attention_step_op(qkv: torch.Tensor, q_norm_w: torch.Tensor, k_norm_w: torch.Tensor, eps: float,
                              rope: torch.Tensor, pos: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
                              n_heads: int, n_kv_heads: int, scale: float) -> torch.Tensor:
@@ -1144,7 +1232,7 @@ def decode_attention_step_op(qkv: torch.Tensor, q_norm_w: torch.Tensor, k_norm_w
     stream = _stream(dev)
     ws = workspace(dev, stream, lib.wsl_decode_attention_step_workspace_bytes(b, n_heads, n_kv_heads, hd, L),
                    kind="attention")
-    with torch.cuda.device(dev):
+    with _on(dev):
         rc = lib.wsl_decode_attention_step_fwd(
             q2.data_ptr(), q2.stride(0), b, n_heads, n_kv_heads, hd, qw.data_ptr(), kw.data_ptr(), float(eps),
             rope.data_ptr(), pos.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), L, float(scale),
@@ -1166,7 +1254,7 @@ def tied_head_argmax_supported(M: int, N: int, K: int) -> bool:
     return bool(_native.lib().wsl_tied_head_argmax_supported(M, N, K))
 
 
-@torch.library.custom_op("wsl::tied_head_argmax", mutates_args=(), device_types="cuda")
+@_custom_op("tied_head_argmax")
 def tied_head_argmax_op(z: torch.Tensor, emb: torch.Tensor) -> torch.Tensor:
     """Greedy token of the tied head: argmax over n of bf16(z[m] . emb[n]) for every row of z
     [M, k] (M <= 64), without writing the [M, vocab] logits (include/wsl_decode.h)."""
@@ -1183,7 +1271,7 @@ def tied_head_argmax_op(z: torch.Tensor, emb: torch.Tensor) -> torch.Tensor:
     lib = _native.lib()
     stream = _stream(dev)
     ws = workspace(dev, stream, lib.wsl_tied_head_argmax_workspace_bytes(M), kind="head_argmax")
-    with torch.cuda.device(dev):
+    with _on(dev):
         rc = lib.wsl_tied_head_argmax_fwd(z2.data_ptr(), z2.stride(0), emb.data_ptr(), emb.stride(0), V, K, M,
                                           out.data_ptr(), ws.data_ptr(), ws.numel(), stream)
     if rc == _native.WSL_E_LAUNCH:
@@ -1202,7 +1290,7 @@ def lora_linear_fused_supported(M: int, N: int, K: int, r: int, fuse: int) -> bo
     return bool(_native.lib().wsl_lora_linear_fused_supported(M, N, K, r, fuse))
 
 
-@torch.library.custom_op("wsl::lora_linear_fused", mutates_args=(), device_types="cuda")
+@_custom_op("lora_linear_fused")
 def lora_linear_fused_op(x: torch.Tensor, norm_w: Optional[torch.Tensor], eps: float, w: torch.Tensor,
                          a: Optional[torch.Tensor], b: Optional[torch.Tensor], scale: float,
                          residual: Optional[torch.Tensor], fuse: int) -> torch.Tensor:
@@ -1224,7 +1312,7 @@ def lora_linear_fused_op(x: torch.Tensor, norm_w: Optional[torch.Tensor], eps: f
     y = torch.empty((M, ny), dtype=torch.bfloat16, device=dev)
     stream = _stream(dev)
     ws = workspace(dev, stream, _native.workspace_bytes(M, N, K, r, _native.WSL_DTYPE_BF16))
-    with torch.cuda.device(dev):
+    with _on(dev):
         rc = _native.lib().wsl_lora_linear_fused_fwd(
             x2.data_ptr(), x2.stride(0), _dev_ptr(nw), float(eps), w.data_ptr(), w.stride(0),
             _dev_ptr(a), a.stride(0) if a is not None else 0, _dev_ptr(b), b.stride(0) if b is not None else 0,
@@ -1311,9 +1399,9 @@ def lora_linear_chain(stages, M: int) -> None:
     need = ctypes.c_size_t(0)
     _native.check(L.wsl_lora_linear_chain_workspace_bytes(M, len(stages), arr, ctypes.byref(need)),
                   "wsl_lora_linear_chain_workspace_bytes")
-    stream = torch.cuda.current_stream(dev).cuda_stream
+    stream = _stream(dev)
     ws = workspace(dev, stream, int(need.value), kind="chain")
-    with torch.cuda.device(dev):
+    with _on(dev):
         rc = L.wsl_lora_linear_chain_fwd(M, len(stages), arr, ws.data_ptr(), ws.numel(), stream)
     if rc == _native.WSL_E_LAUNCH:
         _retire((dev.index, stream, "chain"))
@@ -1324,12 +1412,12 @@ def chain_status(dev: Optional[torch.device] = None) -> bool:
     """True when a chain launch on the current stream's workspace gave up a stage wait since
     the last call (the sticky failure word, then cleared); synchronizes the stream."""
     dev = dev or torch.device("cuda", torch.cuda.current_device())
-    stream = torch.cuda.current_stream(dev).cuda_stream
+    stream = _stream(dev)
     ws = _workspaces.get((dev.index, stream, "chain"))
     if ws is None:
         return False
     failed = ctypes.c_int32(0)
-    with torch.cuda.device(dev):
+    with _on(dev):
         _native.check(_native.lib().wsl_lora_linear_chain_status(ws.data_ptr(), stream, ctypes.byref(failed)),
                       "wsl_lora_linear_chain_status")
     return bool(failed.value)
