@@ -400,12 +400,13 @@ prefill_kernel(const uint16_t* __restrict__ x, int64_t ldx,
   uint32_t aoff = 0;
   if constexpr (RB > 0) aoff = (uint32_t)(min(wave * 8 + (lane >> 3), r - 1) * lda * 2 + fill_chunk(lane, wave) * 16);
   // fp8 W: BN rows x 64 B per K tile, 16 fp8 per chunk
-  constexpr int W8C = (W8 && !WT) ? C::BN * 4 / NT : 1;  // chunks per thread
+  constexpr int W8N = C::BN * 4;                                       // chunks per K tile
+  constexpr int W8C = (W8 && !WT) ? (W8N + NT - 1) / NT : 1;  // per thread (the 192-wide tile's last: half of them)
   const uint8_t* w8row[W8C];
   if constexpr (W8 && !WT) {
 #pragma unroll
     for (int i = 0; i < W8C; ++i) {
-      const int id = i * NT + tid;
+      const int id = min(i * NT + tid, W8N - 1);
       w8row[i] = reinterpret_cast<const uint8_t*>(w) + (int64_t)map_row(min(n0 + (id >> 2), N - 1), wmap) * ldw + (id & 3) * 16;
     }
   }
@@ -530,6 +531,7 @@ prefill_kernel(const uint16_t* __restrict__ x, int64_t ldx,
 #pragma unroll
       for (int i = 0; i < W8C; ++i) {
         const int id = i * NT + tid;
+        if (W8N % NT != 0 && id >= W8N) break;
         const int row = id >> 2, c = (id & 3) * 2;
         u32x4_t lo, hi;
         fp8x16_to_bf16x16(w8stage[i], lo, hi);
