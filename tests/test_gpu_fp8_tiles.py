@@ -1,4 +1,7 @@
-"""fp8 base weights decoded onto the bf16 matrix cores, on the tiles the planner takes."""
+"""fp8 base weights decoded onto the bf16 matrix cores, on every tile the planner takes (128 x 128
+on the deep ring, split in K or not, and two to a CU; 128 x 256, 256 x 192, 256 x 256), with ragged
+M and N, T in the K loop and from the pre-pass, grouped and shared-base rows; and every code decodes
+exactly."""
 import sys
 
 import pytest
@@ -28,8 +31,19 @@ def inputs(gpu, M, N, K, r, seed, groups=1):
 
 CASES = [
     # M, N, K, r, the planner's tile
+    (65, 512, 64, 0, (128, 128)),       # one K tile, deep ring
+    (300, 1500, 128, 40, (128, 128)),   # two K tiles
+    (70, 1000, 1088, 0, (128, 128)),    # 17 K tiles: no even split
+    (130, 1000, 256, 16, (128, 128)),   # as many K tiles as ring buffers, an N tail
+    (333, 1536, 320, 64, (128, 128)),   # two rank blocks
+    (333, 6144, 448, 128, (128, 128)),  # T from the pre-pass
+    (2700, 2900, 128, 8, (128, 128)),   # more tiles than CUs: two-buffer ring
+    (4096, 2048, 192, 32, (128, 256)),
+    (3900, 2040, 448, 128, (128, 256)),
     (2700, 3072, 128, 16, (256, 192)),   # 768 chunks of codes a K tile for 512 threads
     (1024, 12288, 256, 128, (256, 192)),
+    (8192, 2048, 192, 16, (256, 256)),
+    (8100, 2040, 256, 128, (256, 256)),
 ]
 
 
@@ -47,3 +61,89 @@ def test_fp8_tiles(gpu, wsl_opts, M, N, K, r, tile):
         ref += (x.double() @ a.double().t()) @ b.double().t()
     assert rel(y, ref) <= TOL
     assert torch.equal(y, ops.lora_linear_op(x, q, sc, a, b, 1.0))
+
+
+SPLITS = [
+    # M, N, K, r, splits
+    (65, 512, 1024, 0, 2),
+    (100, 1000, 4096, 16, 8),           # an N tail
+    (333, 4096, 4096, 64, 2),           # two rank blocks
+    (129, 1024, 8192, 128, 16),         # T from the pre-pass, applied by the first split
+    (80, 4096, 12288, 256, 8),
+]
+
+
+@pytest.mark.parametrize("M,N,K,r,splits", SPLITS)
+def test_fp8_splits_of_k(gpu, wsl_opts, M, N, K, r, splits):
+    """The in-launch split-K form on codes: the planner's split count, equal to the unsplit launch
+    within the bar, repeatable, its counters back at zero under graph replays."""
+    from weightshared_torchtitan_amd import ops
+    _say(f"[fp8 split-K] M={M} N={N} K={K} r={r}")
+    pl = ops.plan(M, K, r, [N], fp8=True)
+    assert pl["path"] == "prefill_splitk" and pl["k_splits"] == splits
+    x, q, sc, a, b = inputs(gpu, M, N, K, r, M + N + r)
+    y = ops.lora_linear_op(x, q, sc, a, b, 1.0)
+    ref = x.double() @ (q.double() * sc.double()[:, None]).t()
+    if r:
+        ref += (x.double() @ a.double().t()) @ b.double().t()
+    assert rel(y, ref) <= TOL
+    s = torch.cuda.Stream()
+    s.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(s):
+        ops.lora_linear_op(x, q, sc, a, b, 1.0)
+    s.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=s):
+        out = ops.lora_linear_op(x, q, sc, a, b, 1.0)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, y) and torch.equal(ops.lora_linear_op(x, q, sc, a, b, 1.0), y)
+    wsl_opts(prefill_split=-1, fp8_prefill=1)
+    assert ops.plan(M, K, r, [N], fp8=True)["path"] == "prefill"
+    assert rel(ops.lora_linear_op(x, q, sc, a, b, 1.0), ref) <= TOL
+
+
+def test_fp8_grouped_and_shared_base_rows(gpu, wsl_opts):
+    from weightshared_torchtitan_amd import ops
+    wsl_opts(fp8_prefill=1)
+    M, K, r, gn = 300, 1024, 128, [512, 256, 256]
+    assert ops.plan(M, K, r, gn, fp8=True)["path"] == "prefill_splitk"
+    x, q, sc, a, b = inputs(gpu, M, sum(gn), K, r, 3, groups=3)
+    y = ops.lora_linear_grouped_op(x, q, sc, a, b, 1.0, gn)
+    n0 = 0
+    for j, n in enumerate(gn):
+        ref = x.double() @ (q[n0:n0 + n].double() * sc[n0:n0 + n].double()[:, None]).t() \
+            + (x.double() @ a[j * r:(j + 1) * r].double().t()) @ b[n0:n0 + n].double().t()
+        assert rel(y[:, n0:n0 + n], ref) <= TOL
+        n0 += n
+    base_n, g = 128, 2  # 256 wide projections on a base of 128 rows, two templates
+    y = ops.lora_linear_bcast_op(x, q[:base_n], sc[:base_n], a, b[:768], 1.0, g, 3)
+    c, d = torch.arange(256, device=gpu), base_n // g
+    rows = c // (2 * d) * d + c % d
+    for j in range(3):
+        ref = x.double() @ (q[rows].double() * sc[rows].double()[:, None]).t() \
+            + (x.double() @ a[j * r:(j + 1) * r].double().t()) @ b[j * 256:(j + 1) * 256].double().t()
+        assert rel(y[:, j * 256:(j + 1) * 256], ref) <= TOL
+
+
+@pytest.mark.parametrize("M", [80, 4096])
+def test_every_code_decodes_exactly(gpu, wsl_opts, M):
+    """Row n of W holds code n in column n % 128 alone: y picks it out."""
+    from weightshared_torchtitan_amd import ops
+    wsl_opts(fp8_prefill=1)
+    codes = torch.arange(256, dtype=torch.uint8, device=gpu)
+    W = torch.zeros(256, 128, dtype=torch.uint8, device=gpu)
+    W[torch.arange(256), torch.arange(256) % 128] = codes
+    W = W.view(torch.float8_e4m3fn)
+    x = torch.zeros(M, 128, device=gpu, dtype=torch.bfloat16)
+    m = torch.arange(M, device=gpu)
+    x[m, m % 128] = 1.0
+    y = ops.lora_linear_op(x, W, torch.ones(256, device=gpu), None, None, 0.0)
+    want = codes.view(torch.float8_e4m3fn).float()
+    for half in (0, 1):
+        got = y[:128 if M >= 128 else M].float()
+        k = torch.arange(got.shape[0], device=gpu)
+        v, w = got[k, k + 128 * half], want[k + 128 * half]
+        assert torch.equal(v.isnan(), w.isnan()) and torch.equal(v[~w.isnan()], w[~w.isnan()])

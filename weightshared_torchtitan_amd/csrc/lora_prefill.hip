@@ -158,6 +158,17 @@ __device__ __forceinline__ void direct_fill(char* lds_tile, int grp, const void*
   __builtin_amdgcn_global_load_lds(src, (lds_void_t*)(lds_tile + grp * 1024), 16, 0, 0);
 }
 
+// Eight OCP e4m3 codes -> eight bf16 (exact): gfx950's packed conversion with scale 1.
+typedef __bf16 bf16x2v_t __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ u32x4_t fp8x8_decode(uint32_t q0, uint32_t q1) {
+  const bf16x2v_t a = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(q0, 1.f, false);
+  const bf16x2v_t b = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(q0, 1.f, true);
+  const bf16x2v_t c = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(q1, 1.f, false);
+  const bf16x2v_t d = __builtin_amdgcn_cvt_scalef32_pk_bf16_fp8(q1, 1.f, true);
+  return u32x4_t{__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b), __builtin_bit_cast(uint32_t, c),
+                 __builtin_bit_cast(uint32_t, d)};
+}
+
 // s_waitcnt vmcnt(0) with expcnt/lgkmcnt left unconstrained (gfx9 encoding).
 __device__ __forceinline__ void wait_vm0() { __builtin_amdgcn_s_waitcnt(0x0f70); }
 // s_waitcnt vmcnt(N), N < 64
@@ -248,14 +259,19 @@ prefill_kernel(const uint16_t* __restrict__ x, int64_t ldx,
   constexpr bool WDIRECT = HAS_W && WDT == kBF16;
   constexpr bool LORA = RB > 0 || EXT_T;
   constexpr int NT = C::NT;
+  // Deep ring with an fp8 W (the split-K form): the ring holds W's codes ([BN][64] bytes a K tile, filled one K
+  // tile ahead of x's); each K tile is decoded once into one of two bf16 W tiles past the ring.
+  constexpr bool W8R = W8 && !WT && C::NS > 2;
   constexpr int AB = RB * 32 * ROWB;         // rank-A slice of a K tile
-  constexpr int STAGE = C::XB + C::WB + AB;  // one of the two ring buffers
+  constexpr int WBX = W8R ? C::BN * BK : C::WB;
+  constexpr int STAGE = C::XB + WBX + AB;    // one of the ring buffers
+  constexpr int WDEC = C::NS * STAGE;        // W8R: the decoded tiles
   constexpr int OS = C::BN * 2 + 16;          // LDS row stride of the staged output tile
   // PER: T of the strip's row block, [BM m][r ranks] bf16, past the ring (rows of 64 bytes
   // for r <= 32, 128 for r <= 64); the staged output tile stays within the ring
   constexpr int TROW = (PER && RB == 1) ? 64 : ROWB;
   constexpr int TREG = PER ? C::BM * TROW : 0;
-  constexpr int RING = C::NS * STAGE + TREG;
+  constexpr int RING = C::NS * STAGE + TREG + (W8R ? 2 * C::WB : 0);
   constexpr int LDS_BYTES = (RING > C::BM * OS) ? RING : C::BM * OS;
   static_assert(LDS_BYTES <= 160 * 1024, "LDS budget");
   static_assert(!PER || C::BM * OS <= C::NS * STAGE, "staged output clear of the T region");
@@ -265,8 +281,8 @@ prefill_kernel(const uint16_t* __restrict__ x, int64_t ldx,
   __shared__ __attribute__((aligned(1024))) char lds[LDS_BYTES];
   static_assert(!SPLIT || (WDT == kBF16 && HAS_W && RB == 0 && !EXT_T && !GATHER), "split-K is a plain bf16 GEMM");
   static_assert(!TN || (WDT == kBF16 && HAS_W && RB == 0 && !EXT_T && !GATHER), "token-major operands: plain bf16 GEMM");
-  static_assert(!RED || (WDT == kBF16 && HAS_W && !EXT_T && !GATHER && !SPLIT && !TN), "in-launch split-K: bf16 W");
-  static_assert(C::NS == 2 || (!W8 && !TN && !GATHER), "deep ring: bf16 W and x as they lie");
+  static_assert(!RED || (HAS_W && !WT && (W8 || !EXT_T) && !GATHER && !SPLIT && !TN), "in-launch split-K: W as it lies");
+  static_assert(C::NS == 2 || (!(W8 && WT) && !TN && !GATHER), "deep ring: x and W as they lie");
   static_assert(!WT || (HAS_W && !TN && !GATHER && !SPLIT && !RED && C::BN % 128 == 0 &&
                         (WDT == kBF16 || (C::NS == 2 && (64 * C::BN / 16) % C::NT == 0))),
                 "token-major W': x as it lies, 128-column multiples (fp8: two-buffer ring)");
@@ -276,7 +292,7 @@ prefill_kernel(const uint16_t* __restrict__ x, int64_t ldx,
   if constexpr (RED) {
     const int64_t kofs = (int64_t)blockIdx.y * K;
     x += kofs;
-    w = reinterpret_cast<const uint16_t*>(w) + kofs;
+    w = reinterpret_cast<const char*>(w) + kofs * (W8 ? 1 : 2);
     if constexpr (RB > 0) a_arg += kofs;
   }
   if constexpr (SPLIT) {
@@ -401,15 +417,53 @@ prefill_kernel(const uint16_t* __restrict__ x, int64_t ldx,
   if constexpr (RB > 0) aoff = (uint32_t)(min(wave * 8 + (lane >> 3), r - 1) * lda * 2 + fill_chunk(lane, wave) * 16);
   // fp8 W: BN rows x 64 B per K tile, 16 fp8 per chunk
   constexpr int W8N = C::BN * 4;                                       // chunks per K tile
-  constexpr int W8C = (W8 && !WT) ? (W8N + NT - 1) / NT : 1;  // per thread (the 192-wide tile's last: half of them)
+  constexpr int W8C = (W8 && !WT && !W8R) ? (W8N + NT - 1) / NT : 1;  // per thread (192 wide: half have a last one)
   const uint8_t* w8row[W8C];
-  if constexpr (W8 && !WT) {
+  if constexpr (W8 && !WT && !W8R) {
 #pragma unroll
     for (int i = 0; i < W8C; ++i) {
       const int id = min(i * NT + tid, W8N - 1);
       w8row[i] = reinterpret_cast<const uint8_t*>(w) + (int64_t)map_row(min(n0 + (id >> 2), N - 1), wmap) * ldw + (id & 3) * 16;
     }
   }
+
+  // W8R: fill q of this wave writes lane i's 16 codes at 1024 q + 16 i: chunk i % 4 of row
+  // 16 q + i / 4, in order (each lane decodes the chunk it filled, read back linearly).
+  constexpr int W8Q = W8R ? C::BN / 16 / C::NW : 1;  // fills per wave
+  static_assert(!W8R || (C::BN / 16) % C::NW == 0, "whole fills per wave");
+  const char* w8base = reinterpret_cast<const char*>(w) + (W8R ? (int64_t)wrow0 * ldw : 0);
+  uint32_t w8off[W8Q];
+  if constexpr (W8R) {
+#pragma unroll
+    for (int i = 0; i < W8Q; ++i) {
+      const int row = (wave * W8Q + i) * 16 + (lane >> 2);
+      w8off[i] = (uint32_t)((map_row(min(n0 + row, N - 1), wmap) - wrow0) * ldw + (lane & 3) * 16);
+    }
+  }
+  auto issue_w8 = [&](char* dst, int k0) {
+    if constexpr (W8R) {
+#pragma unroll
+      for (int i = 0; i < W8Q; ++i) direct_fill(dst, wave * W8Q + i, w8base + k0 + opaque(w8off[i]));
+    }
+  };
+  // A lane's codes at `raw`, and half of each chunk decoded into the bf16 W tile `par`.
+  u32x4_t w8v[W8Q];
+  auto read_w8 = [&](const char* raw) {
+    if constexpr (W8R) {
+#pragma unroll
+      for (int i = 0; i < W8Q; ++i) w8v[i] = lds_read16(raw, (wave * W8Q + i) * 1024 + lane * 16);
+    }
+  };
+  auto decode_w8 = [&](int half, int par) {
+    if constexpr (W8R) {
+      char* dst = lds + WDEC + par * C::WB;
+#pragma unroll
+      for (int i = 0; i < W8Q; ++i) {
+        const int row = (wave * W8Q + i) * 16 + (lane >> 2), c = (lane & 3) * 2 + half;
+        lds_write16(dst, lds_off(row, c), fp8x8_decode(w8v[i][2 * half], w8v[i][2 * half + 1]));
+      }
+    }
+  };
 
   // TN fills: wave fill q covers LDS bytes [1024 q, 1024 q + 1024) of a [64][cols] tile, lane i
   // the 16 bytes at 1024 q + 16 i: row (1024 q + 16 i) / (2 cols), physical chunk s, which
@@ -426,7 +480,7 @@ prefill_kernel(const uint16_t* __restrict__ x, int64_t ldx,
   auto issue = [&](int stage, int k0) {
     char* sx = lds + stage * STAGE;
     char* sw = sx + C::XB;
-    char* sa = sw + C::WB;
+    char* sa = sw + WBX;
     if constexpr (TN) {
       constexpr int QX = 64 * C::BM * 2 / 1024 / C::NW, QW = 64 * C::BN * 2 / 1024 / C::NW;
 #pragma unroll
@@ -483,7 +537,7 @@ prefill_kernel(const uint16_t* __restrict__ x, int64_t ldx,
         w8t[i] = ld_global_16(reinterpret_cast<const uint8_t*>(w) + (int64_t)(k0 + row) * ldw + col);
         w8s[i] = w_scale[k0 + row];
       }
-    } else if constexpr (W8) {
+    } else if constexpr (W8 && !W8R) {
 #pragma unroll
       for (int i = 0; i < W8C; ++i) w8stage[i] = ld_global_16(w8row[i] + k0);
     }
@@ -526,7 +580,7 @@ prefill_kernel(const uint16_t* __restrict__ x, int64_t ldx,
         lds_write16(sw, row * C::BN * 2 + (((c16 * 2) ^ sw4) << 4), u32x4_t{o[0], o[1], o[2], o[3]});
         lds_write16(sw, row * C::BN * 2 + (((c16 * 2 + 1) ^ sw4) << 4), u32x4_t{o[4], o[5], o[6], o[7]});
       }
-    } else if constexpr (W8) {
+    } else if constexpr (W8 && !W8R) {
       char* sw = lds + stage * STAGE + C::XB;
 #pragma unroll
       for (int i = 0; i < W8C; ++i) {
@@ -594,10 +648,10 @@ prefill_kernel(const uint16_t* __restrict__ x, int64_t ldx,
     const uint2 lo = lds_read_tr8(tile, off), hi = lds_read_tr8(tile, off + 4 * cols * 2);
     return u32x4_t{lo.x, lo.y, hi.x, hi.y};
   };
-  auto frag_load = [&](auto do_t, int stage, int kk, Frags& f) {
+  auto frag_load = [&](auto do_t, int stage, int kk, Frags& f, int par = 0) {
     const char* sx = lds + stage * STAGE;
-    const char* sw = sx + C::XB;
-    const char* sa = sw + C::WB;
+    const char* sw = W8R ? lds + WDEC + par * C::WB : sx + C::XB;
+    const char* sa = sx + C::XB + WBX;
     if constexpr (TN) {
 #pragma unroll
       for (int j = 0; j < C::MJ; ++j) f.x[j] = tn_frag(sx, C::BM, wm * C::TM + j * 32, kk);
@@ -745,28 +799,45 @@ prefill_kernel(const uint16_t* __restrict__ x, int64_t ldx,
   // K tile waiting one fill's latency (about 1.2 us per 128 x 128 x 64 tile at M = 256).
   auto run_k_deep = [&](auto do_t, auto cls) {
     constexpr int NS = C::NS;
-    constexpr int PT = C::NXI + (WDIRECT ? C::NWI : 0);  // fills per K tile of every wave (waves < NAI add one)
+    // fills per K tile of every wave (waves < NAI add one)
+    constexpr int PT = C::NXI + (WDIRECT ? C::NWI : W8R ? W8Q : 0);
     const int pre = nk < NS ? nk : NS;
-    for (int q = 0; q < pre; ++q) issue(q, q * BK);
+    // W8R: a K tile's fills bring the next one's codes (the last K tile's again at the end), so
+    // that they have landed while its predecessor is multiplied; K tile 0's go where K tile 1
+    // will be decoded.
+    auto issue_kt = [&](int stage, int kt) {
+      issue(stage, kt * BK);
+      issue_w8(lds + stage * STAGE + C::XB, min(kt + 1, nk - 1) * BK);
+    };
+    issue_w8(lds + WDEC + C::WB, 0);
+    for (int q = 0; q < pre; ++q) issue_kt(q, q);
     if constexpr (LORA) {
       if (nk < NS) issue_b(lora_b, 0);  // buffer nk is never filled with a K tile
     }
     if (nk >= NS) wait_vm<(NS - 1) * PT>();  // tile 0 has landed
     else wait_vm0();
+    read_w8(lds + WDEC + C::WB);
+    decode_w8(0, 0);
+    decode_w8(1, 0);
     ring_barrier();
     WSL_STAMP(srec, 1);
     Frags cur;
-    frag_load(t_at(do_t, cls, K0{}), 0, 0, cur);
+    frag_load(t_at(do_t, cls, K0{}), 0, 0, cur, 0);
     int buf = 0;
     for (int kt = 0; kt < nk; ++kt) {
       const int nbuf = buf + 1 == NS ? 0 : buf + 1;
+      // W8R: the next K tile's codes (this lane's own fill), decoded between this tile's first k
+      // steps, off the path from the wait to the barrier; the other bf16 tile's readers are behind
+      // the last barrier. (After the last K tile: the last tile's codes again, never read.)
+      read_w8(lds + buf * STAGE + C::XB);
       for_ct<0, KK - 1>([&](auto kc) {
         using KN = std::integral_constant<int, decltype(kc)::value + 1>;
         Frags nxt;
-        frag_load(t_at(do_t, cls, KN{}), buf, KN::value, nxt);
+        frag_load(t_at(do_t, cls, KN{}), buf, KN::value, nxt, kt & 1);
         frag_mma(t_at(do_t, cls, kc), cur);
         interleave(t_at(do_t, cls, kc), t_at(do_t, cls, KN{}));
         cur = nxt;
+        if constexpr (W8R && decltype(kc)::value < 2) decode_w8(decltype(kc)::value, (kt + 1) & 1);
       });
       if (kt + 1 < nk) {
         if (kt + NS - 1 < nk) wait_vm<(NS - 2) * PT>();  // tile kt+1 has landed
@@ -774,12 +845,12 @@ prefill_kernel(const uint16_t* __restrict__ x, int64_t ldx,
         ring_barrier();  // all fragments of tile kt are read; tile kt+1 visible
       }
       Frags nxt;
-      frag_load(t_at(do_t, cls, K0{}), nbuf, 0, nxt);
+      frag_load(t_at(do_t, cls, K0{}), nbuf, 0, nxt, (kt + 1) & 1);
       frag_mma(t_at(do_t, cls, KL{}), cur);
       interleave(t_at(do_t, cls, KL{}), t_at(do_t, cls, K0{}));
       cur = nxt;
       if (kt + NS < nk) {
-        issue(buf, (kt + NS) * BK);
+        issue_kt(buf, kt + NS);
       } else if constexpr (LORA) {
         if (kt + NS == nk) issue_b(lora_b, 0);  // buffer `buf` is lora_b
       }
@@ -948,7 +1019,8 @@ prefill_kernel(const uint16_t* __restrict__ x, int64_t ldx,
         }
       }
     }
-    const int nrc = (r + 63) / 64;
+    // RED with T from the pre-pass: the whole of T, so one split applies it
+    const int nrc = RED && EXT_T && blockIdx.y != 0 ? 0 : (r + 63) / 64;
     for (int rc = 0; rc < nrc; ++rc) {
       const int rk0 = rc * 64;
       if (rc > 0) issue_b(sb, rk0);
@@ -1457,20 +1529,33 @@ int rank_splits(int64_t M, int64_t K, int64_t r) {
   return 1;
 }
 
-// T[m][k] = bf16(s * sum_q part[q][m][k]), q in order: 8 consecutive ranks per thread.
+// T[m][k] = bf16(s * sum_q part[q][m][k]), q in order: 4 consecutive ranks per thread, eight
+// splits' loads in flight (one at a time, the sum of 14 splits of 333 x 384 was a chain of 14
+// round trips, 6.4 us).
 __global__ void __launch_bounds__(256)
 rank_reduce_kernel(const float* __restrict__ part, int splits, int64_t slice, float s,
                    uint16_t* __restrict__ t) {
-  const int64_t e = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 8;
+  const int64_t e = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
   if (e >= slice) return;
-  f32x4_t lo = *reinterpret_cast<const f32x4_t*>(part + e);
-  f32x4_t hi = *reinterpret_cast<const f32x4_t*>(part + e + 4);
-  for (int q = 1; q < splits; ++q) {
-    lo += *reinterpret_cast<const f32x4_t*>(part + q * slice + e);
-    hi += *reinterpret_cast<const f32x4_t*>(part + q * slice + e + 4);
+  const f32x4_t* p = reinterpret_cast<const f32x4_t*>(part + e);
+  const int64_t sv = slice / 4;
+  f32x4_t a = p[0];
+  int q = 1;
+  for (; q + 8 <= splits; q += 8) {
+    f32x4_t v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v[u] = p[(q + u) * sv];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) a += v[u];
   }
-  *reinterpret_cast<u32x4_t*>(t + e) = u32x4_t{pack_bf16x2(s * lo[0], s * lo[1]), pack_bf16x2(s * lo[2], s * lo[3]),
-                                               pack_bf16x2(s * hi[0], s * hi[1]), pack_bf16x2(s * hi[2], s * hi[3])};
+  f32x4_t v[7];
+#pragma unroll
+  for (int u = 0; u < 7; ++u)
+    if (q + u < splits) v[u] = p[(q + u) * sv];
+#pragma unroll
+  for (int u = 0; u < 7; ++u)
+    if (q + u < splits) a += v[u];
+  *reinterpret_cast<uint2*>(t + e) = uint2{pack_bf16x2(s * a[0], s * a[1]), pack_bf16x2(s * a[2], s * a[3])};
 }
 
 }  // namespace
@@ -1581,11 +1666,22 @@ constexpr int kRedMaxSplits = 16;
 constexpr int kRedMinTiles = 8;  // 1.7B layer at M = 129-256: 8 K tiles per split 7-8 % ahead of 4
 constexpr size_t kRedPartBytes = (size_t)24 << 20;
 
+size_t align256(size_t v) { return (v + 255) & ~(size_t)255; }
+
 // Bytes of one (tile, split) record: 8 waves x 64 lanes x 16 words (the output partial).
 size_t red_record_bytes() { return (size_t)CfgDeep::NW * 64 * 8 * (CfgDeep::NI * CfgDeep::MJ * 8); }
 
+// Workspace bytes of the form with an fp8 W: the pre-pass region (`pre`: ranks above RIN; rt, the
+// ranks of all groups), then the records; 0 (the form not taken) above the records' budget, so
+// that it never needs more than the no-allocation scratch has.
+size_t red_fp8_bytes(int64_t M, int64_t N, int64_t K, int64_t rt, bool pre, int splits) {
+  const size_t b = (pre && rt > 0 ? align256(rank_prepass_bytes(M, K, rt)) : 0) +
+                   (size_t)(((M + 127) / 128) * ((N + 127) / 128) * splits) * red_record_bytes();
+  return b <= kRedPartBytes ? b : 0;
+}
+
 int red_splits(int64_t M, int64_t N, int64_t K, int w_dtype, bool has_w, bool gather) {
-  if (!has_w || gather || w_dtype != kBF16 || M < 1) return 0;
+  if (!has_w || gather || M < 1) return 0;
   const int64_t nk = K / BK;
   const int64_t tiles = ((M + 127) / 128) * ((N + 127) / 128);
   if (tiles > kRedMaxTiles) return 0;
@@ -1605,11 +1701,45 @@ int red_splits(int64_t M, int64_t N, int64_t K, int w_dtype, bool has_w, bool ga
   return s > 1 ? s : 0;
 }
 
+// An fp8 W (8B shapes, graphs of 20 launches, us, the unsplit launch before): 80 x 4096 x 12288
+// 139.7 -> 37.4 at r = 16, 147.1 -> 49.1 at r = 128 (pre-pass included); 333 x 4096 x 4096 51.9 ->
+// 37.2 and 62.2 -> 47.1; 600 x 1024 x 4096 51.7 -> 24.5; 80 x 12288 x 4096 50.2 -> 36.3. The splits
+// run on the deep ring, W's codes in the ring and each K tile decoded once (W8R). Unsplit
+// launches stay on the two-buffer ring: their loop is bound by the LDS (the decode's reads and
+// writes beside the fragments'), and the deep ring ran 333 x 6144 x 4096 at 48.4 against 48.0 us
+// (57.6 against 52.0 with a rank block). Decoding at the fragments instead, which reads half the
+// LDS bytes, was slower still (52.3-55.6): every wave then converts the rows it shares.
+//
+// The split count a call takes (0: not the in-launch split-K form): red_splits where the form
+// covers its rank (up to 64 in the K loop; an fp8 W also with T from the pre-pass), its groups end
+// on whole tiles, an fp8 W does not go to the fp8 matrix cores, and the workspace has the records.
+int red_splits_of(const LoraArgs& p) {
+  if (p.w == nullptr || p.gather != nullptr || !groups_fit(p, 128)) return 0;
+  const bool fp8 = p.w_dtype == kFP8;
+  if (p.r > RIN && !fp8) return 0;
+  if (fp8 && fp8_matrix_cores(p)) return 0;
+  const int s = red_splits(p.M, p.N, p.K, p.w_dtype, true, false);
+  return s > 0 && (!fp8 || red_fp8_bytes(p.M, p.N, p.K, p.r * p.groups, p.r > RIN, s) > 0) ? s : 0;
+}
+
 namespace {
 hipError_t launch_red(const LoraArgs& p, int splits) {
   LoraArgs q = p;
   q.K = p.K / splits;
   uint64_t* part = reinterpret_cast<uint64_t*>(p.ws);
+  if (p.w_dtype == kFP8) {
+    if (p.r > RIN) {  // T from the pre-pass, applied by split 0
+      const int64_t rt = p.r * p.groups;
+      uint16_t* t = reinterpret_cast<uint16_t*>(p.ws);
+      const hipError_t e = rank_prepass(p, t);
+      if (e != hipSuccess) return e;
+      part = reinterpret_cast<uint64_t*>(reinterpret_cast<char*>(p.ws) + align256(rank_prepass_bytes(p.M, p.K, rt)));
+      return launch_cfg<CfgDeep, kFP8, true, 0, true, false, false, false, true>(q, t, rt, splits, part, p.red_cnt);
+    }
+    if (p.r == 0) return launch_cfg<CfgDeep, kFP8, true, 0, false, false, false, false, true>(q, nullptr, 0, splits, part, p.red_cnt);
+    if (p.r <= 32) return launch_cfg<CfgDeep, kFP8, true, 1, false, false, false, false, true>(q, nullptr, 0, splits, part, p.red_cnt);
+    return launch_cfg<CfgDeep, kFP8, true, 2, false, false, false, false, true>(q, nullptr, 0, splits, part, p.red_cnt);
+  }
   if (p.r == 0) return launch_cfg<CfgDeep, kBF16, true, 0, false, false, false, false, true>(q, nullptr, 0, splits, part, p.red_cnt);
   if (p.r <= 32) return launch_cfg<CfgDeep, kBF16, true, 1, false, false, false, false, true>(q, nullptr, 0, splits, part, p.red_cnt);
   return launch_cfg<CfgDeep, kBF16, true, 2, false, false, false, false, true>(q, nullptr, 0, splits, part, p.red_cnt);
@@ -1733,8 +1863,11 @@ hipError_t launch_medium(const LoraArgs& p, int splits) {
 // With the in-launch split-K form possible (which `r`, the ranks of all groups, does not
 // decide) its records are covered as well.
 size_t prefill_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t r, int w_dtype) {
-  if (w_dtype == kFP8)
-    return (r > 0 ? rank_prepass_bytes(M, K, r) : 0) + prefill_fp8_workspace_bytes(M, K, 2);
+  if (w_dtype == kFP8) {
+    const size_t b = (r > 0 ? rank_prepass_bytes(M, K, r) : 0) + prefill_fp8_workspace_bytes(M, K, 2);
+    const int s = red_splits(M, N, K, w_dtype, true, false);  // r: the ranks of all groups, so with the pre-pass or not
+    return s > 0 ? std::max({b, red_fp8_bytes(M, N, K, r, true, s), red_fp8_bytes(M, N, K, r, false, s)}) : b;
+  }
   size_t b = r > 32 ? rank_prepass_bytes(M, K, r) : 0;
   const int ms = medium_splits(M, N, K, r, w_dtype, true, false);
   if (ms > 0) {
@@ -1769,7 +1902,7 @@ hipError_t rank_prepass(const LoraArgs& p, uint16_t* t) {
     hipError_t e = launch_cfg<CfgDeep, kBF16, true, 0, false, false, true>(q, nullptr, 0, splits);
     if (e != hipSuccess) return e;
     const int64_t slice = p.M * rt;
-    rank_reduce_kernel<<<dim3((unsigned)((slice / 8 + 255) / 256)), dim3(256), 0, p.stream>>>(part, splits, slice, p.scale, t);
+    rank_reduce_kernel<<<dim3((unsigned)((slice / 4 + 255) / 256)), dim3(256), 0, p.stream>>>(part, splits, slice, p.scale, t);
     return hipGetLastError();
   }
   return launch_rank<kBF16, true>(q, nullptr, 0);
@@ -1860,15 +1993,14 @@ PrefillPlan plan_prefill(const LoraArgs& p) {
   } else {
     // The in-launch split-K form runs 128 x 128 tiles that compute their group's T, so every
     // group end must fall on a tile boundary.
-    const int rs = (has_w && p.w_dtype == kBF16 && p.r <= RIN && p.red_cnt != nullptr && groups_fit(p, 128))
-                       ? red_splits(p.M, p.N, p.K, p.w_dtype, true, false)
-                       : 0;
+    const int rs = p.red_cnt != nullptr ? red_splits_of(p) : 0;
     const int ms = (rs == 0 && has_w && p.w_dtype == kBF16) ? medium_splits(p.M, p.N, p.K, rt, p.w_dtype, true, false)
                                                              : 0;
     if (rs > 0) {
       pl.form = WSL_PATH_PREFILL_SPLITK;
       pl.tile_m = pl.tile_n = 128;
-      pl.rank_blocks = p.r == 0 ? 0 : p.r <= 32 ? 1 : 2;
+      pl.prepass = p.r > RIN;
+      pl.rank_blocks = p.r == 0 || pl.prepass ? 0 : p.r <= 32 ? 1 : 2;
       pl.splits = rs;
       pl.workgroups = tiles128 * rs;
       return pl;

@@ -288,6 +288,7 @@ bool grouped_one_launch(const wsl::LoraArgs& p) {
   // tiles, so a group may sum K in another order than its single call (within the bar). That
   // form's 128 x 128 tiles compute their group's T, so its group ends must fall on multiples
   // of 128; where they do not, the groups go one by one (each may still take the form).
+  if (p.w_dtype == WSL_DTYPE_FP8_E4M3) return wsl::prefill_groups_supported(p);  // no medium form; split-K runs whole
   const auto medium = [&](int64_t n, int64_t rt) {
     if (p.r <= 64 && wsl::red_splits(p.M, n, p.K, p.w_dtype, p.w != nullptr, false) > 0) return 0;
     return wsl::medium_splits(p.M, n, p.K, rt, p.w_dtype, p.w != nullptr, false);

@@ -179,6 +179,8 @@ int medium_splits(int64_t M, int64_t N, int64_t K, int64_t rt, int w_dtype, bool
 // K splits of the prefill path's in-launch split-K form over 128 x 128 tiles (0: not taken;
 // it also needs a rank of at most 64 per group).
 int red_splits(int64_t M, int64_t N, int64_t K, int w_dtype, bool has_w, bool gather);
+// The same for a call, its groups and its rank included.
+int red_splits_of(const LoraArgs& p);
 // Plain bf16 products over a long contiguous K (csrc/lora_prefill.hip) and the rank
 // pre-pass T = bf16(s x . A^T), for the weight gradients (csrc/lora_backward.hip).
 int product_splits(int64_t M, int64_t N, int64_t nk, bool divides);
