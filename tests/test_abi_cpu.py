@@ -677,3 +677,11 @@ def test_plan_rank_33_to_64_takes_the_prepass_for_wider_tiles(M, K, r, groups, p
     assert p["rank_blocks"] == (0 if prepass else (1 if r <= 32 else 2))
     if prepass:  # the size query covers the pre-pass's T and split partials
         assert N.grouped_workspace_bytes(M, K, r, groups, N.WSL_DTYPE_BF16) >= 65536 + 2 * M * r * len(groups) * 2
+
+
+@pytest.mark.parametrize("dt", [0, 1, 2])
+@pytest.mark.parametrize("r", [0, 8, 50, 256])
+def test_workspace_bytes_without_rows(r, dt):
+    """A call of no rows needs no scratch beyond the counters; the query divided by its row tiles."""
+    assert N.workspace_bytes(0, 256, 4096, r, dt) == 65536
+    assert N.grouped_workspace_bytes(0, 4096, min(r, 64), (256, 128), dt) == 65536

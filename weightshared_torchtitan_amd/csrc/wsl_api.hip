@@ -138,7 +138,7 @@ size_t decode_data(int64_t M, int64_t N, int64_t K, int64_t r, int w_dtype, int 
 }
 size_t generic_data(int64_t M, int64_t r) { return (size_t)(M * r * 2); }
 size_t prefill_data(int64_t M, int64_t N, int64_t K, int64_t r, int w_dtype) {
-  return wsl::prefill_workspace_bytes(M, N, K, r, w_dtype);
+  return M > 0 ? wsl::prefill_workspace_bytes(M, N, K, r, w_dtype) : 0;  // the plans divide by the row tiles
 }
 
 // Upper bound over the paths a problem of this size can take (the path also depends on
