@@ -261,6 +261,31 @@ int wsl_lora_linear_bwd_input(const void* gy, int64_t ldg, const void* w, int64_
                               void* workspace, size_t workspace_bytes, void* stream);
 
 /*
+ * Every gradient of wsl_lora_linear_bcast_fwd (bf16 W): with gy [M, n_groups * N], gy_b [M, base_n]
+ * its columns summed by the base row they read, U = scale * gy . Bd and T = scale * x . A^T (bf16,
+ * Bd block-diagonal over the groups),
+ *
+ *   dx [M, K] = gy_b . W + U . A          dw [base_n, K] = gy_b^T . x
+ *   da [n_groups * r, K] = U^T . x        db [n_groups * N, r], group j's rows gy_j^T . T_j
+ *
+ * all dense; a NULL output is left out. _supported returns 1 for the layouts taken: K, base_n and
+ * n_groups * N multiples of 64, base_n / g and r of 8, n_groups * r <= WSL_MAX_RANK, x, gy, w and
+ * a 16-byte aligned with leading dimensions multiples of 8; the others return WSL_E_SHAPE, and a
+ * caller composes the single-projection gradients. Replaces torch autograd's backward of the
+ * composition (torchtitan/models/llama3/model/model.py:111-145, 189-192, 239-256, 381-398).
+ */
+int wsl_lora_linear_bcast_bwd_supported(const void* x, int64_t ldx, const void* gy, int64_t ldg, const void* w,
+                                        int64_t ldw, const void* a, int64_t lda, const void* b, int64_t ldb,
+                                        int64_t M, int64_t N, int64_t K, int64_t r, int64_t base_n, int64_t g,
+                                        int32_t n_groups);
+int wsl_lora_linear_bcast_bwd_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t r, int64_t base_n,
+                                              int32_t n_groups, size_t* bytes);
+int wsl_lora_linear_bcast_bwd(const void* x, int64_t ldx, const void* gy, int64_t ldg, const void* w, int64_t ldw,
+                              const void* a, int64_t lda, const void* b, int64_t ldb, float scale, int64_t M,
+                              int64_t N, int64_t K, int64_t r, int64_t base_n, int64_t g, int32_t n_groups, void* dx,
+                              void* dw, void* da, void* db, void* workspace, size_t workspace_bytes, void* stream);
+
+/*
  * wsl_lora_linear_bwd_input for a bf16 W in any layout (any N, K, r up to WSL_MAX_RANK, any
  * leading dimensions, element-aligned pointers), on bounds-checked matrix-core tiles that read W
  * and A where they lie. Workspace (256-byte aligned): bf16(scale * gy . B) [M, r].

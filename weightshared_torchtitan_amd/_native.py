@@ -50,6 +50,9 @@ EXPORTED = (
     "wsl_lora_linear_bwd_input_supported",
     "wsl_lora_linear_bwd_input_workspace_bytes",
     "wsl_lora_linear_bwd_input",
+    "wsl_lora_linear_bcast_bwd_supported",
+    "wsl_lora_linear_bcast_bwd_workspace_bytes",
+    "wsl_lora_linear_bcast_bwd",
     "wsl_lora_linear_bwd_input_any_workspace_bytes",
     "wsl_lora_linear_bwd_input_any",
     "wsl_lora_pad_rank",
@@ -240,6 +243,16 @@ def _declare(lib: ctypes.CDLL) -> None:
         _c_vp, ctypes.c_size_t,          # workspace, bytes
         _c_vp,                           # stream
     ]
+    operands = [_c_vp, _c_i64] * 5  # x, gy, w, a, b with their leading dimensions
+    sizes = [_c_i64] * 6 + [ctypes.c_int32]  # M, N, K, r, base_n, g, n_groups
+    lib.wsl_lora_linear_bcast_bwd_supported.restype = ctypes.c_int
+    lib.wsl_lora_linear_bcast_bwd_supported.argtypes = operands + sizes
+    lib.wsl_lora_linear_bcast_bwd_workspace_bytes.restype = ctypes.c_int
+    lib.wsl_lora_linear_bcast_bwd_workspace_bytes.argtypes = [_c_i64] * 5 + [ctypes.c_int32, ctypes.POINTER(ctypes.c_size_t)]
+    lib.wsl_lora_linear_bcast_bwd.restype = ctypes.c_int
+    lib.wsl_lora_linear_bcast_bwd.argtypes = operands + [ctypes.c_float] + sizes + [
+        _c_vp, _c_vp, _c_vp, _c_vp,      # dx, dw, da, db
+        _c_vp, ctypes.c_size_t, _c_vp]   # workspace, bytes, stream
     lib.wsl_lora_linear_bwd_input_any_workspace_bytes.restype = ctypes.c_int
     lib.wsl_lora_linear_bwd_input_any_workspace_bytes.argtypes = [_c_i64, _c_i64, _c_i64, _c_i64,
                                                                   ctypes.POINTER(ctypes.c_size_t)]
@@ -409,6 +422,13 @@ def bwd_input_workspace_bytes(M: int, N: int, K: int, r: int) -> int:
     out = ctypes.c_size_t(0)
     check(lib().wsl_lora_linear_bwd_input_workspace_bytes(M, N, K, r, ctypes.byref(out)),
           "wsl_lora_linear_bwd_input_workspace_bytes")
+    return int(out.value)
+
+
+def bcast_bwd_workspace_bytes(M: int, N: int, K: int, r: int, base_n: int, n_groups: int) -> int:
+    out = ctypes.c_size_t(0)
+    check(lib().wsl_lora_linear_bcast_bwd_workspace_bytes(M, N, K, r, base_n, n_groups, ctypes.byref(out)),
+          "wsl_lora_linear_bcast_bwd_workspace_bytes")
     return int(out.value)
 
 

@@ -399,4 +399,203 @@ hipError_t launch_weight_grads(const LoraArgs& p, const void* gy, int64_t ldg, v
   return e;
 }
 
+// ---- Shared-base backward ----
+// One base W [base_n, K] under `groups` projections of N columns, output column c of each on base
+// row c' = map_row(c) (RowMap). With gy_b [M, base_n] the sums of gy's columns by base row and Bd
+// the block-diagonal [G N, G r] form of B,
+//
+//   dX = gy_b . W + U . A      U = bf16(s gy . Bd)     dW = gy_b^T . x
+//   dA = U^T . x               dB_j = gy_j^T . T_j     T = bf16(s x . A^T)
+//
+// U is computed once for dX and dA. Kernels of this part: the column sums (one read of gy), and the
+// factors in the layouts that the products take (Bd^T and A^T, one launch); dB's diagonal blocks
+// are picked out as the token splits of the [G N, G r] product are summed. As torch operators
+// (casts, a 5-d sum, block copies, transposes, a separate delta product and its addition) this
+// work was 22 launches and 125 of 307 us of the backward at M = 4096, q|k|v on 2048 x 2048, r = 32;
+// forward and backward there 433 -> 305 us (dX's delta joins its base product's accumulators, so
+// dX is rounded once, not three times), 436 -> 107 us on small sizes, which the launches bounded.
+namespace {
+// gyb[m][n] = bf16(sum of gy[m][c] over the columns c of every group whose base row is n), groups
+// then heads in order; eight consecutive base rows per thread (the template width D is a multiple
+// of 8, so they are consecutive columns in every head). Bound by reading gy.
+__global__ void __launch_bounds__(256) fold_columns_kernel(const uint16_t* __restrict__ gy, int64_t ldg, int64_t M,
+                                                          int base_n, int N, int groups, RowMap wmap,
+                                                          uint16_t* __restrict__ gyb) {
+  const int per = base_n / 8;
+  const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int64_t m = idx / per;
+  if (m >= M) return;
+  const int n = (int)(idx % per) * 8;
+  // base row n of template n / D is column (n / D) S + h D + n % D of head h, h < S / D
+  const int c0 = n / wmap.D * wmap.S + n % wmap.D, heads = wmap.S / wmap.D;
+  float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  for (int j = 0; j < groups; ++j)
+    for (int h = 0; h < heads; ++h) {
+      const u32x4_t v = ld_global_16(gy + m * ldg + (int64_t)j * N + c0 + h * wmap.D);
+#pragma unroll
+      for (int e = 0; e < 8; ++e) acc[e] += bf16_bits_to_f32((v[e >> 1] >> ((e & 1) * 16)) & 0xffffu);
+    }
+  u32x4_t o;
+#pragma unroll
+  for (int q = 0; q < 4; ++q) o[q] = pack_bf16x2(acc[2 * q], acc[2 * q + 1]);
+  *reinterpret_cast<u32x4_t*>(gyb + m * base_n + n) = o;
+}
+
+// bt [G r, G N] = Bd^T (zeros off the diagonal blocks) and at [K, G r] = A^T, one element a thread.
+__global__ void __launch_bounds__(256) bcast_factors_kernel(const uint16_t* __restrict__ a, int64_t lda,
+                                                           const uint16_t* __restrict__ b, int64_t ldb, int64_t K,
+                                                           int64_t N, int64_t r, int groups,
+                                                           uint16_t* __restrict__ bt, uint16_t* __restrict__ at) {
+  const int64_t gr = groups * r, gn = groups * N, nb = gr * gn;
+  const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (e < nb) {
+    const int64_t q = e / gn, c = e % gn;
+    bt[e] = c / N == q / r ? b[c * ldb + q % r] : 0;
+  } else if (e - nb < K * gr) {
+    const int64_t k = (e - nb) / gr, q = (e - nb) % gr;
+    at[e - nb] = a[q * lda + k];
+  }
+}
+
+// db[c][q] = bf16(sum over the splits of part[s][c][(c / N) r + q]), splits in order: four
+// consecutive ranks per thread.
+__global__ void __launch_bounds__(256) diag_sum_kernel(const float* __restrict__ part, int splits, int64_t gn, int64_t N,
+                                                      int64_t r, int64_t gr, uint16_t* __restrict__ db) {
+  const int64_t e = ((int64_t)blockIdx.x * 256 + threadIdx.x) * 4;
+  if (e >= gn * r) return;
+  const int64_t c = e / r, q = e % r;
+  const f32x4_t v = sum_splits(part + c * gr + c / N * r + q, gn * gr, splits);
+  *reinterpret_cast<uint2*>(db + e) = uint2{pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3])};
+}
+
+struct BcastPlan {
+  int sw, sb, sa;  // token splits of the dW, dB and dA products
+  size_t off_gyb, off_bt, off_at, off_u, off_t, off_part, total;
+};
+BcastPlan make_bcast_plan(int64_t M, int64_t N, int64_t K, int64_t r, int64_t base_n, int groups) {
+  BcastPlan L{};
+  const int64_t nk = (M + 63) / 64, gn = groups * N, gr = groups * r;
+  L.sw = product_splits(base_n, K, nk, false);
+  L.sb = r > 0 ? product_splits(gn, gr, nk, false) : 1;
+  L.sa = r > 0 ? product_splits(gr, K, nk, false) : 1;
+  size_t off = 0;
+  L.off_gyb = off; off = a256(off + (size_t)M * base_n * 2);
+  L.off_bt = off;  off = a256(off + (size_t)(gr * gn) * 2);
+  L.off_at = off;  off = a256(off + (size_t)(K * gr) * 2);
+  L.off_u = off;   off = a256(off + (r > 0 ? rank_prepass_bytes(M, gn, gr) : 0));
+  L.off_t = off;   off = a256(off + (r > 0 ? rank_prepass_bytes(M, K, gr) : 0));
+  L.off_part = off;
+  size_t part = (size_t)L.sw * base_n * K;
+  part = std::max({part, (size_t)(L.sb * gn * gr), (size_t)(L.sa * gr * K)});
+  L.total = a256(off + part * 4);
+  return L;
+}
+}  // namespace
+
+bool bcast_bwd_supported(const LoraArgs& p, const void* gy, int64_t ldg) {
+  const int64_t gn = p.groups * p.N, gr = p.groups * p.r, base_n = p.wrows, lim = (int64_t)1 << 22;
+  if (p.M < 1 || p.M > lim - 2048 || gn > lim || p.K > lim || p.ldx > lim || ldg > lim || p.ldw > lim || p.lda > lim)
+    return false;
+  if (p.K % 64 != 0 || gn % 64 != 0 || base_n % 64 != 0 || p.wmap.D % 8 != 0 || p.r % 8 != 0 || gr > WSL_MAX_RANK)
+    return false;
+  if (p.w == nullptr || p.w_dtype != kBF16 || !al16(p.w) || p.ldw % 8 != 0) return false;
+  if (!al16(p.x) || p.ldx % 8 != 0 || !al16(gy) || ldg % 8 != 0) return false;
+  if (p.r > 0 && (!al16(p.a) || p.lda % 8 != 0)) return false;  // b goes through its rearranged copy
+  return p.M * base_n / 8 / 256 < 0x7fffffff;
+}
+
+size_t bcast_bwd_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t r, int64_t base_n, int groups) {
+  return make_bcast_plan(M, N, K, r, base_n, groups).total;
+}
+
+hipError_t launch_bcast_bwd(const LoraArgs& p, const void* gy, int64_t ldg, void* dx, void* dw, void* da, void* db) {
+  const int64_t M = p.M, K = p.K, N = p.N, r = p.r, base_n = p.wrows;
+  const int64_t gn = p.groups * N, gr = p.groups * r;
+  const hipStream_t st = p.stream;
+  const BcastPlan L = make_bcast_plan(M, N, K, r, base_n, p.groups);
+  char* ws = reinterpret_cast<char*>(p.ws);
+  uint16_t* gyb = reinterpret_cast<uint16_t*>(ws + L.off_gyb);
+  uint16_t* bt = reinterpret_cast<uint16_t*>(ws + L.off_bt);
+  uint16_t* at = reinterpret_cast<uint16_t*>(ws + L.off_at);
+  uint16_t* U = reinterpret_cast<uint16_t*>(ws + L.off_u);
+  uint16_t* T = reinterpret_cast<uint16_t*>(ws + L.off_t);
+  float* part = reinterpret_cast<float*>(ws + L.off_part);
+  const int64_t nkt = (M + 63) / 64;
+  hipError_t e = hipSuccess;
+  LoraArgs base = p;  // a plain problem of this stream; its operands are set per product
+  base.groups = 1; base.wmap = RowMap{}; base.gather = nullptr; base.gather_rows = 0;
+
+  // part[s] [rows, cols] = the token splits of xa^T . wb; how many there are
+  auto token_product = [&](const void* xa, int64_t ldxa, int64_t rows, const void* wb, int64_t ldwb, int64_t cols,
+                           int splits, int* used, void* direct) -> hipError_t {
+    LoraArgs q = base;
+    q.x = xa; q.ldx = ldxa; q.w = wb; q.ldw = ldwb; q.M = rows; q.N = cols; q.yscale = 1.f;
+    const int64_t kt = (nkt + splits - 1) / splits;
+    q.K = kt * 64;
+    *used = (int)((nkt + kt - 1) / kt);
+    if (direct != nullptr && *used == 1) {
+      q.y = direct; q.ldy = cols;
+      *used = 0;
+      return launch_product_tn(q, M, nullptr, 1);
+    }
+    return launch_product_tn(q, M, part, *used);
+  };
+  auto sum_to = [&](int splits, int64_t rows, int64_t cols, void* dst) {
+    const int64_t n4 = rows * cols / 4;
+    split_sum_kernel<<<dim3((unsigned)((n4 + 255) / 256)), dim3(256), 0, st>>>(
+        part, splits, rows, cols, 1.f, reinterpret_cast<uint16_t*>(dst), cols, 1);
+    return hipGetLastError();
+  };
+
+  const void* gb = gy;  // gy by base row
+  int64_t ldgb = ldg;
+  if ((dx != nullptr || dw != nullptr) && !(p.groups == 1 && base_n == N)) {
+    const int64_t blocks = (M * (base_n / 8) + 255) / 256;
+    fold_columns_kernel<<<dim3((unsigned)blocks), dim3(256), 0, st>>>(reinterpret_cast<const uint16_t*>(gy), ldg, M,
+                                                                     (int)base_n, (int)N, p.groups, p.wmap, gyb);
+    e = hipGetLastError();
+    gb = gyb;
+    ldgb = base_n;
+  }
+  if (e == hipSuccess && r > 0 && (dx != nullptr || da != nullptr)) {
+    const int64_t blocks = (gr * gn + K * gr + 255) / 256;
+    bcast_factors_kernel<<<dim3((unsigned)blocks), dim3(256), 0, st>>>(
+        reinterpret_cast<const uint16_t*>(p.a), p.lda, reinterpret_cast<const uint16_t*>(p.b), p.ldb, K, N, r,
+        p.groups, bt, at);
+    e = hipGetLastError();
+    if (e == hipSuccess) {
+      LoraArgs q = base;
+      q.x = gy; q.ldx = ldg; q.K = gn; q.a = bt; q.lda = gn; q.r = gr;
+      e = rank_prepass(q, U);
+    }
+  }
+  if (e == hipSuccess && dx != nullptr) {
+    LoraArgs q = base;
+    q.x = gb; q.ldx = ldgb; q.K = base_n; q.N = K; q.wrows = 0;
+    q.a = bt; q.lda = gn; q.b = at; q.ldb = gr; q.r = gr; q.y = dx; q.ldy = K;
+    e = launch_prefill_wt(q, r > 0 ? U : nullptr, gr);
+  }
+  int s = 0;
+  if (e == hipSuccess && dw != nullptr) {
+    e = token_product(gb, ldgb, base_n, p.x, p.ldx, K, L.sw, &s, dw);
+    if (e == hipSuccess && s > 0) e = sum_to(s, base_n, K, dw);
+  }
+  if (e == hipSuccess && r > 0 && da != nullptr) {
+    e = token_product(U, gr, gr, p.x, p.ldx, K, L.sa, &s, nullptr);
+    if (e == hipSuccess) e = sum_to(s, gr, K, da);
+  }
+  if (e == hipSuccess && r > 0 && db != nullptr) {
+    LoraArgs q = base;
+    q.r = gr;
+    e = rank_prepass(q, T);
+    if (e == hipSuccess) e = token_product(gy, ldg, gn, T, gr, gr, L.sb, &s, nullptr);
+    if (e == hipSuccess) {
+      diag_sum_kernel<<<dim3((unsigned)((gn * r / 4 + 255) / 256)), dim3(256), 0, st>>>(
+          part, s, gn, N, r, gr, reinterpret_cast<uint16_t*>(db));
+      e = hipGetLastError();
+    }
+  }
+  return e;
+}
+
 }  // namespace wsl

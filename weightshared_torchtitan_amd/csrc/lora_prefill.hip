@@ -2053,18 +2053,16 @@ hipError_t launch_wt_rank(const LoraArgs& q, const uint16_t* tg, int64_t ldt) {
 // The forward's tile forms (tiles by how they fill the CUs, persistent strips, the three-
 // and four-buffer rings), without the 192-wide tile (the token-major W' tile needs whole
 // 128-column chunks). Ranks above 64 take T = s dY . B from the rank pre-pass in the
-// workspace. An fp8 W is decoded through registers with each row's scale (bf16(code *
-// scale), the values of the dequantised W) into the same token-major tiles (two-buffer
-// ring, no strips).
-hipError_t launch_prefill_wt(const LoraArgs& q_in) {
+// workspace; a caller that has T passes it (tg [M, r], row stride ldt). An fp8 W is decoded
+// through registers with each row's scale (bf16(code * scale), the values of the dequantised
+// W) into the same token-major tiles (two-buffer ring, no strips).
+hipError_t launch_prefill_wt(const LoraArgs& q_in, const uint16_t* tg, int64_t ldt) {
   LoraArgs q = q_in;
   q.gather_rows = q.K;  // every reduction row of W' is in range: no clamping in its fills
-  const uint16_t* tg = nullptr;
-  int64_t ldt = 0;
   // T from the pre-pass above RIN, and for ranks 33-64 where it frees a tile wider than
   // 128 x 128 (as the forward's prepass_rank)
-  bool pre = q.r > RIN;
-  if (!pre && q.r > 32) {
+  bool pre = tg == nullptr && q.r > RIN;
+  if (tg == nullptr && !pre && q.r > 32) {
     const Tile t = pick_tiles(q, (int)q.w_dtype, true, 0, true, false, true).tile;
     pre = t != Tile::kSmall && t != Tile::kDeep;
   }

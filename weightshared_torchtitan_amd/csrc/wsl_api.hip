@@ -576,6 +576,74 @@ int wsl_lora_linear_bcast_fwd(const void* x, int64_t ldx, const void* w, int64_t
   return run_grouped(p, n_groups, gn, true, workspace, workspace_bytes);
 }
 
+// The arguments of a shared-base backward as launch_bcast_bwd takes them; false for sizes or
+// pointers that no call may have.
+static bool bcast_bwd_args(const void* x, int64_t ldx, const void* gy, int64_t ldg, const void* w, int64_t ldw,
+                           const void* a, int64_t lda, const void* b, int64_t ldb, float scale, int64_t M, int64_t N,
+                           int64_t K, int64_t r, int64_t base_n, int64_t g, int32_t n_groups, void* stream,
+                           wsl::LoraArgs* out) {
+  if (n_groups < 1 || n_groups > WSL_MAX_GROUPS || base_n < 1 || g < 1 || N < 1 || N % base_n != 0 || base_n % g != 0)
+    return false;
+  if (M < 1 || K < 1 || r < 0 || r > WSL_MAX_RANK || N > ((int64_t)1 << 30) || K > ((int64_t)1 << 30)) return false;
+  if (x == nullptr || gy == nullptr || w == nullptr || (r > 0 && (a == nullptr || b == nullptr))) return false;
+  if (ldx < K || ldg < N * n_groups || ldw < K || (r > 0 && (lda < K || ldb < r))) return false;
+  wsl::LoraArgs p = make_args(x, ldx, w, ldw, WSL_DTYPE_BF16, nullptr, a, lda, b, ldb, scale, nullptr, 0, M, N, K, r,
+                              stream);
+  p.groups = n_groups;
+  p.wmap.P = (int)N;
+  p.wmap.S = (int)(N / g);
+  p.wmap.D = (int)(base_n / g);
+  p.wrows = base_n;
+  *out = p;
+  return wsl::bcast_bwd_supported(p, gy, ldg);
+}
+
+int wsl_lora_linear_bcast_bwd_supported(const void* x, int64_t ldx, const void* gy, int64_t ldg, const void* w,
+                                        int64_t ldw, const void* a, int64_t lda, const void* b, int64_t ldb,
+                                        int64_t M, int64_t N, int64_t K, int64_t r, int64_t base_n, int64_t g,
+                                        int32_t n_groups) {
+  wsl::LoraArgs p;
+  return bcast_bwd_args(x, ldx, gy, ldg, w, ldw, a, lda, b, ldb, 1.f, M, N, K, r, base_n, g, n_groups, nullptr, &p) ? 1 : 0;
+}
+
+int wsl_lora_linear_bcast_bwd_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t r, int64_t base_n,
+                                              int32_t n_groups, size_t* bytes) {
+  clear_err();
+  if (bytes == nullptr) return fail(WSL_E_INVALID_ARG, "bytes must not be NULL");
+  const int rc = validate_sizes(M, N, K, r, WSL_DTYPE_BF16);
+  if (rc != WSL_OK) return rc;
+  if (n_groups < 1 || n_groups > WSL_MAX_GROUPS || base_n < 1 || base_n > N)
+    return fail(WSL_E_SHAPE, "need 1 <= n_groups <= %d and 1 <= base_n <= N", WSL_MAX_GROUPS);
+  *bytes = layout_bytes(M > 0 ? wsl::bcast_bwd_workspace_bytes(M, N, K, r, base_n, n_groups) : 0);
+  return WSL_OK;
+}
+
+int wsl_lora_linear_bcast_bwd(const void* x, int64_t ldx, const void* gy, int64_t ldg, const void* w, int64_t ldw,
+                              const void* a, int64_t lda, const void* b, int64_t ldb, float scale, int64_t M,
+                              int64_t N, int64_t K, int64_t r, int64_t base_n, int64_t g, int32_t n_groups, void* dx,
+                              void* dw, void* da, void* db, void* workspace, size_t workspace_bytes, void* stream) {
+  clear_err();
+  if (dx == nullptr && dw == nullptr && da == nullptr && db == nullptr) return WSL_OK;
+  if (r == 0 && (da != nullptr || db != nullptr)) return fail(WSL_E_INVALID_ARG, "da and db need r > 0");
+  wsl::LoraArgs p;
+  if (!bcast_bwd_args(x, ldx, gy, ldg, w, ldw, a, lda, b, ldb, scale, M, N, K, r, base_n, g, n_groups, stream, &p))
+    return fail(WSL_E_SHAPE, "layout not taken (see wsl_lora_linear_bcast_bwd_supported)");
+  if (((uintptr_t)dx & 15) || ((uintptr_t)dw & 15) || ((uintptr_t)da & 15) || ((uintptr_t)db & 15))
+    return fail(WSL_E_ALIGN, "the gradients must be 16-byte aligned");
+  const size_t need = wsl::bcast_bwd_workspace_bytes(M, N, K, r, base_n, n_groups);
+  if (workspace == nullptr || workspace_bytes < layout_bytes(need))
+    return fail(WSL_E_WORKSPACE, "workspace of %zu bytes required (got %zu)", layout_bytes(need), workspace_bytes);
+  if ((uintptr_t)workspace & 255) return fail(WSL_E_ALIGN, "workspace must be 256-byte aligned");
+  const int rc = check_device();
+  if (rc != WSL_OK) return rc;
+  const size_t half = half_of(workspace_bytes);
+  p.ws = reinterpret_cast<char*>(workspace) + wsl::kCounterBytes + half;
+  p.ws_bytes = half;
+  const hipError_t e = wsl::launch_bcast_bwd(p, gy, ldg, dx, dw, da, db);
+  if (e != hipSuccess) return fail(WSL_E_LAUNCH, "kernel launch failed: %s", hipGetErrorString(e));
+  return WSL_OK;
+}
+
 int wsl_lora_linear_bwd_weights_supported(const void* x, int64_t ldx, const void* gy, int64_t ldg, const void* a,
                                           int64_t lda, const void* b, int64_t ldb, int64_t M, int64_t N, int64_t K,
                                           int64_t r) {

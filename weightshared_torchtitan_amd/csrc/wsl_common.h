@@ -199,10 +199,16 @@ hipError_t launch_weight_grads(const LoraArgs& p, const void* gy, int64_t ldg, v
 // dY [M, N], w = W [N, K], a = A [r, K], b = B [N, r], y = dX [M, K]; p.N and p.K are the
 // linear's), which transposes A and B into the workspace (csrc/lora_backward.hip).
 bool prefill_wt_supported(const LoraArgs& q);
-hipError_t launch_prefill_wt(const LoraArgs& q);
+hipError_t launch_prefill_wt(const LoraArgs& q, const uint16_t* tg = nullptr, int64_t ldt = 0);
 bool bwd_input_supported(const LoraArgs& p);
 size_t bwd_input_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t r);
 hipError_t launch_bwd_input(const LoraArgs& p);
+// Every gradient of a shared-base call (p: x [M, K], w [wrows, K], a [groups r, K], b [groups N, r]
+// with p.N one group's width and p.wmap its column map; gy [M, groups N]), null outputs left out
+// (csrc/lora_backward.hip).
+bool bcast_bwd_supported(const LoraArgs& p, const void* gy, int64_t ldg);
+size_t bcast_bwd_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t r, int64_t base_n, int groups);
+hipError_t launch_bcast_bwd(const LoraArgs& p, const void* gy, int64_t ldg, void* dx, void* dw, void* da, void* db);
 
 // fp8 matrix-core prefill path (csrc/lora_prefill_fp8.hip): T from the rank pre-pass, the
 // activation codes and per-token scales in `scratch` (prefill_fp8_workspace_bytes).

@@ -671,6 +671,59 @@ def _lora_linear_bcast_fake(x, w, w_scale, a, b, scale, g, n_groups):
     return x.new_empty((*x.shape[:-1], int(n_groups) * N), dtype=torch.bfloat16)
 
 
+@_custom_op("lora_linear_bcast_grads")
+def lora_linear_bcast_grads_op(x: torch.Tensor, gy: torch.Tensor, w: torch.Tensor, a: Optional[torch.Tensor],
+                               b: Optional[torch.Tensor], scale: float, g: int, n_groups: int, need_x: bool,
+                               need_w: bool, need_a: bool,
+                               need_b: bool) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
+    """(dx [M, K], dw, da, db) of wsl::lora_linear_bcast, each only when asked for (else an empty
+    tensor), for x [M, K] and gy [M, n_groups * N] (wsl_lora_linear_bcast_bwd; raises for the layouts
+    it does not take: see bcast_grads_supported)."""
+    dev = _check_device(x, gy, w, a, b)
+    M, K = x.shape
+    base_n, N, r = w.shape[0], gy.shape[1] // n_groups, b.shape[1] if b is not None else 0
+    mk = lambda need, *s: x.new_empty(s if need else 0)  # noqa: E731
+    dx, dw, da, db = mk(need_x, M, K), mk(need_w, base_n, K), mk(need_a, n_groups * r, K), mk(need_b, n_groups * N, r)
+    ptr = lambda t, need: t.data_ptr() if need else None  # noqa: E731
+    # a view into storage that does not start on 16 bytes goes through a copy
+    x, gy, w = (t if _rows16(t) else t.clone(memory_format=torch.contiguous_format) for t in (x, gy, w))
+    if r and not _rows16(a):
+        a = a.clone(memory_format=torch.contiguous_format)
+    stream = _stream(dev)
+    ws = workspace(dev, stream, _native.bcast_bwd_workspace_bytes(M, N, K, r, base_n, n_groups))
+    with _on(dev):
+        rc = _native.lib().wsl_lora_linear_bcast_bwd(
+            x.data_ptr(), x.stride(0), gy.data_ptr(), gy.stride(0), w.data_ptr(), w.stride(0), _dev_ptr(a),
+            a.stride(0) if r else 0, _dev_ptr(b), b.stride(0) if r else 0, float(scale), M, N, K, r, base_n, int(g),
+            n_groups, ptr(dx, need_x), ptr(dw, need_w), ptr(da, need_a), ptr(db, need_b), ws.data_ptr(), ws.numel(),
+            stream)
+    _native.check(rc, "wsl_lora_linear_bcast_bwd")
+    return dx, dw, da, db
+
+
+@lora_linear_bcast_grads_op.register_fake
+def _lora_linear_bcast_grads_fake(x, gy, w, a, b, scale, g, n_groups, need_x, need_w, need_a, need_b):
+    mk = lambda need, *s: x.new_empty(s if need else (0,))  # noqa: E731
+    r = b.shape[1] if b is not None else 0
+    return (mk(need_x, *x.shape), mk(need_w, *w.shape), mk(need_a, n_groups * r, x.shape[1]),
+            mk(need_b, gy.shape[1], r))
+
+
+def bcast_grads_supported(x, gy, w, a, b, g: int, n_groups: int) -> bool:
+    """Whether wsl::lora_linear_bcast_grads takes these operands: row-major bf16 on the tile grid, rows
+    whole 16-byte pieces apart (from sizes, types and strides only, so that tracing decides alike)."""
+    ts = [t for t in (x, gy, w, a, b) if t is not None]
+    if any(t.dtype != torch.bfloat16 or t.dim() != 2 or t.stride(1) != 1 or t.stride(0) < t.shape[1] for t in ts):
+        return False
+    M, K = x.shape
+    base_n, G, r = w.shape[0], n_groups, b.shape[1] if b is not None else 0
+    N = gy.shape[1] // G
+    return (M >= 1 and K % 64 == 0 and base_n % 64 == 0 and G * N % 64 == 0 and base_n // g % 8 == 0 and r % 8 == 0
+            and G <= _native.WSL_MAX_GROUPS and G * r <= _native.WSL_MAX_RANK
+            and max(M + 2048, G * N, K, *(t.stride(0) for t in ts)) <= 1 << 22
+            and all(t.stride(0) % 8 == 0 and t.storage_offset() % 8 == 0 for t in ((x, gy, w, a) if r else (x, gy, w))))
+
+
 def _lora_linear_bcast_setup(ctx, inputs, output):
     x, w, w_scale, a, b, scale, g, n_groups = inputs
     ctx.save_for_backward(x, w, w_scale, a, b)
@@ -684,11 +737,12 @@ def _lora_linear_bcast_backward(ctx, gy):
     base(c) = (c / (hpg D)) D + c % D, so W's gradient gathers them: with gy_b [M, base_n]
     the sum of gy over the groups and the heads of each template,
 
-        dx = gy_b . W + scale * (gy . Bd) . a       two launches of the fused kernel
+        dx = gy_b . W + scale * (gy . Bd) . a
         dW = gy_b^T . x
         da = scale * (gy . Bd)^T . x,   db_j = scale * gy_j^T . (x . a_j^T)
 
-    (Bd: b block-diagonal over the groups). The reference differentiates broadcast_add's
+    (Bd: b block-diagonal over the groups), in one wsl::lora_linear_bcast_grads call where it takes the
+    layout, else composed from the single-projection gradients. The reference differentiates broadcast_add's
     expand and the separate projections (torchtitan/models/llama3/model/model.py:111-145,
     381-398); these are the same sums."""
     x, w, w_scale, a, b, scale = *ctx.saved_tensors, ctx.scale
@@ -703,6 +757,14 @@ def _lora_linear_bcast_backward(ctx, gy):
     D = base_n // g
     hpg = N // base_n
     x2 = x.reshape(-1, K)
+    if M > 0 and bcast_grads_supported(x2, gy2, w, a, b, g, G):
+        has_r = b is not None and b.shape[1] > 0
+        needs = (need_x, need_w, has_r and need_a, has_r and need_b)
+        if not any(needs):
+            return (None,) * 8
+        dx, dw, da, db = (t if n else None for t, n in zip(
+            lora_linear_bcast_grads_op(x2, gy2, w, a if has_r else None, b if has_r else None, s, g, G, *needs), needs))
+        return dx.reshape(x.shape) if need_x else None, dw, None, da, db, None, None, None
     gyb = gy2.float().view(M, G, g, hpg, D).sum(dim=(1, 3)).reshape(M, base_n).to(torch.bfloat16)
     has_lora = a is not None and b is not None and b.shape[1] > 0
     r = b.shape[1] if has_lora else 0
