@@ -183,6 +183,7 @@ bool al16(const void* q) { return (reinterpret_cast<uintptr_t>(q) & 15u) == 0; }
 // union of both routes' buffers.
 struct Plan {
   int sw;          // token splits of the dW product
+  bool sw_big;     // dW over 256 x 256 tiles
   int sb, sa;      // token route: token splits of the dB and dA products
   int sdb, sda;    // dW route: splits of dB = s dW . A^T (over K) and dA = s B^T . dW (over N)
   size_t off_t, off_u, off_bt, off_dwc, off_dwt, off_part, total;
@@ -191,7 +192,9 @@ struct Plan {
 Plan make_plan(int64_t M, int64_t N, int64_t K, int64_t r) {
   Plan L{};
   const int64_t nk = (M + 63) / 64;
-  L.sw = product_splits(N, K, nk, false);
+  const TnSplit tw = product_tn_splits(N, K, nk);
+  L.sw = tw.splits;
+  L.sw_big = tw.big;
   L.sb = r > 0 ? product_splits(N, r, nk, false) : 1;
   L.sa = r > 0 ? product_splits(r, K, nk, false) : 1;
   L.sdb = r > 0 ? product_splits(N, r, K / 64, true) : 1;
@@ -362,7 +365,7 @@ hipError_t launch_weight_grads(const LoraArgs& p, const void* gy, int64_t ldg, v
     } else {
       LoraArgs q = p;
       q.x = gy; q.ldx = ldg; q.w = p.x; q.ldw = p.ldx; q.M = N; q.N = K; q.K = per;
-      e = launch_product_tn(q, M, part, sw);
+      e = launch_product_tn(q, M, part, sw, L.sw_big);
       if (e == hipSuccess) {
         dw_reduce_kernel<<<dim3((unsigned)(K / TT), (unsigned)(N / TT)), dim3(256), 0, st>>>(
             part, sw, N, K, reinterpret_cast<uint16_t*>(dw), lddw, vec_ok(dw, lddw) ? 1 : 0,
@@ -470,12 +473,15 @@ __global__ void __launch_bounds__(256) diag_sum_kernel(const float* __restrict__
 
 struct BcastPlan {
   int sw, sb, sa;  // token splits of the dW, dB and dA products
+  bool sw_big;     // dW's over 256 x 256 tiles
   size_t off_gyb, off_bt, off_at, off_u, off_t, off_part, total;
 };
 BcastPlan make_bcast_plan(int64_t M, int64_t N, int64_t K, int64_t r, int64_t base_n, int groups) {
   BcastPlan L{};
   const int64_t nk = (M + 63) / 64, gn = groups * N, gr = groups * r;
-  L.sw = product_splits(base_n, K, nk, false);
+  const TnSplit tw = product_tn_splits(base_n, K, nk);
+  L.sw = tw.splits;
+  L.sw_big = tw.big;
   L.sb = r > 0 ? product_splits(gn, gr, nk, false) : 1;
   L.sa = r > 0 ? product_splits(gr, K, nk, false) : 1;
   size_t off = 0;
@@ -527,7 +533,7 @@ hipError_t launch_bcast_bwd(const LoraArgs& p, const void* gy, int64_t ldg, void
 
   // part[s] [rows, cols] = the token splits of xa^T . wb; how many there are
   auto token_product = [&](const void* xa, int64_t ldxa, int64_t rows, const void* wb, int64_t ldwb, int64_t cols,
-                           int splits, int* used, void* direct) -> hipError_t {
+                           int splits, bool big, int* used, void* direct) -> hipError_t {
     LoraArgs q = base;
     q.x = xa; q.ldx = ldxa; q.w = wb; q.ldw = ldwb; q.M = rows; q.N = cols; q.yscale = 1.f;
     const int64_t kt = (nkt + splits - 1) / splits;
@@ -538,7 +544,7 @@ hipError_t launch_bcast_bwd(const LoraArgs& p, const void* gy, int64_t ldg, void
       *used = 0;
       return launch_product_tn(q, M, nullptr, 1);
     }
-    return launch_product_tn(q, M, part, *used);
+    return launch_product_tn(q, M, part, *used, big);
   };
   auto sum_to = [&](int splits, int64_t rows, int64_t cols, void* dst) {
     const int64_t n4 = rows * cols / 4;
@@ -577,18 +583,18 @@ hipError_t launch_bcast_bwd(const LoraArgs& p, const void* gy, int64_t ldg, void
   }
   int s = 0;
   if (e == hipSuccess && dw != nullptr) {
-    e = token_product(gb, ldgb, base_n, p.x, p.ldx, K, L.sw, &s, dw);
+    e = token_product(gb, ldgb, base_n, p.x, p.ldx, K, L.sw, L.sw_big, &s, dw);
     if (e == hipSuccess && s > 0) e = sum_to(s, base_n, K, dw);
   }
   if (e == hipSuccess && r > 0 && da != nullptr) {
-    e = token_product(U, gr, gr, p.x, p.ldx, K, L.sa, &s, nullptr);
+    e = token_product(U, gr, gr, p.x, p.ldx, K, L.sa, false, &s, nullptr);
     if (e == hipSuccess) e = sum_to(s, gr, K, da);
   }
   if (e == hipSuccess && r > 0 && db != nullptr) {
     LoraArgs q = base;
     q.r = gr;
     e = rank_prepass(q, T);
-    if (e == hipSuccess) e = token_product(gy, ldg, gn, T, gr, gr, L.sb, &s, nullptr);
+    if (e == hipSuccess) e = token_product(gy, ldg, gn, T, gr, gr, L.sb, false, &s, nullptr);
     if (e == hipSuccess) {
       diag_sum_kernel<<<dim3((unsigned)((gn * r / 4 + 255) / 256)), dim3(256), 0, st>>>(
           part, s, gn, N, r, gr, reinterpret_cast<uint16_t*>(db));

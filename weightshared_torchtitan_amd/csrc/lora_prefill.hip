@@ -477,17 +477,40 @@ prefill_kernel(const uint16_t* __restrict__ x, int64_t ldx,
     const int64_t t = min((int64_t)(k0 + row), tok_rem - 1);
     direct_fill(tile, q, src + t * ld + f);
   };
+  // A whole K tile's lane offsets from its first row (64 rows of at most 2^22 elements: 32 bits);
+  // only the last, partial K tile takes the clamped rows of tn_fill.
+  constexpr int TQX = TN ? 64 * C::BM * 2 / 1024 / C::NW : 1, TQW = TN ? 64 * C::BN * 2 / 1024 / C::NW : 1;
+  uint32_t tnx[TQX], tnw[TQW];
+  if constexpr (TN) {
+    auto tn_off = [&](int cols, int q, int64_t ld, int col0, int ncols) {
+      const int row = (q * 1024 + lane * 16) / (cols * 2);
+      const int c = (lane % (cols / 8)) ^ ((row & 3) << 2);
+      return (uint32_t)((row * ld + min(col0 + c * 8, ncols - 8)) * 2);
+    };
+#pragma unroll
+    for (int i = 0; i < TQX; ++i) tnx[i] = tn_off(C::BM, wave * TQX + i, ldx, m0, M);
+#pragma unroll
+    for (int i = 0; i < TQW; ++i) tnw[i] = tn_off(C::BN, wave * TQW + i, ldw, n0, N);
+  }
   auto issue = [&](int stage, int k0) {
     char* sx = lds + stage * STAGE;
     char* sw = sx + C::XB;
     char* sa = sw + WBX;
     if constexpr (TN) {
-      constexpr int QX = 64 * C::BM * 2 / 1024 / C::NW, QW = 64 * C::BN * 2 / 1024 / C::NW;
+      if (tok_rem - k0 >= BK) {  // the same for every wave
+        const char* xk = reinterpret_cast<const char*>(x) + (int64_t)k0 * ldx * 2;
+        const char* wk = reinterpret_cast<const char*>(w) + (int64_t)k0 * ldw * 2;
 #pragma unroll
-      for (int i = 0; i < QX; ++i) tn_fill(sx, C::BM, wave * QX + i, x, ldx, m0, M, k0);
+        for (int i = 0; i < TQX; ++i) direct_fill(sx, wave * TQX + i, xk + opaque(tnx[i]));
 #pragma unroll
-      for (int i = 0; i < QW; ++i)
-        tn_fill(sw, C::BN, wave * QW + i, reinterpret_cast<const uint16_t*>(w), ldw, n0, N, k0);
+        for (int i = 0; i < TQW; ++i) direct_fill(sw, wave * TQW + i, wk + opaque(tnw[i]));
+        return;
+      }
+#pragma unroll
+      for (int i = 0; i < TQX; ++i) tn_fill(sx, C::BM, wave * TQX + i, x, ldx, m0, M, k0);
+#pragma unroll
+      for (int i = 0; i < TQW; ++i)
+        tn_fill(sw, C::BN, wave * TQW + i, reinterpret_cast<const uint16_t*>(w), ldw, n0, N, k0);
       return;
     }
 #pragma unroll
@@ -1944,12 +1967,42 @@ hipError_t launch_product(const LoraArgs& p, float* part, int splits) {
   return launch_cfg<CfgSmall, kBF16, true, 0, false, false, true>(q, nullptr, 0, splits);
 }
 
+// Token splits of a weight gradient [M, N] over nk K tiles, and their tile. A 128 x 128 tile
+// reads 1.5 KB of fragments from LDS for each MFMA and a 256 x 256 tile half of that, so the
+// small tile runs at the LDS's rate: 0.7 us of a CU for each of its K tiles beside another
+// workgroup, 0.92 alone, against 1.85 for four times the work on the large one. Few large tiles
+// therefore pay for more splits, whose fp32 partials are written and read once (about 7 TB/s):
+// the cheaper of the two by these figures. dW with its reduce, 128 x 128 against 256 x 256:
+// 16384 tokens x 2048 x 2048 215 (unsplit) against 130 us (4 splits), 8192 x 1024 x 3072 77 (4)
+// against 68 (5), 4096 x 2048 x 2048 60 (unsplit) against 55 (4). Where the large tiles fill
+// the CUs alone (192 or more) the product is not split.
+TnSplit product_tn_splits(int64_t M, int64_t N, int64_t nk) {
+  const TnSplit small{product_splits(M, N, nk, false), false};
+  const int64_t tb = ((M + 255) / 256) * ((N + 255) / 256), ts = ((M + 127) / 128) * ((N + 127) / 128);
+  if (M < 256 || N < 256 || tb >= 192) return small;
+  auto cost = [&](int64_t tiles, int splits, double per_tile) {
+    const double partials = splits > 1 ? 8.0 * splits * M * N / 7e6 : 0.0;
+    return ((tiles * splits + 255) / 256) * ((nk + splits - 1) / splits) * per_tile + partials;
+  };
+  double best = cost(ts, small.splits, ts * small.splits > 256 ? 0.7 : 0.92);
+  TnSplit pick = small;
+  for (int s = 2; s <= kMaxProductSplits && s <= nk / kMinSplitTiles; ++s) {
+    const double c = cost(tb, s, 1.85);
+    if (c < 0.97 * best) {
+      best = c;
+      pick = TnSplit{s, true};
+    }
+  }
+  return pick;
+}
+
 // Token-major products (the weight gradients): x' from p.x [tokens][M] (row stride ldx),
 // W' from p.w [tokens][N] (ldw), bf16, M and N multiples of 8, 16-byte aligned rows;
 // `tokens` rows in all, p.K per split (a multiple of BK; every split starts below `tokens`).
 // part == nullptr (splits 1): bf16 y' (p.y, p.ldy, p.yscale) over 256 x 256 tiles when they
-// fill the CUs, else 128 x 128; otherwise unscaled fp32 partials [splits][M][N] over 128 x 128.
-hipError_t launch_product_tn(const LoraArgs& p, int64_t tokens, float* part, int splits) {
+// fill the CUs, else 128 x 128; otherwise unscaled fp32 partials [splits][M][N] over 128 x 128
+// tiles, or 256 x 256 with `big`.
+hipError_t launch_product_tn(const LoraArgs& p, int64_t tokens, float* part, int splits, bool big) {
   LoraArgs q = p;
   q.w_dtype = kBF16; q.w_scale = nullptr; q.a = nullptr; q.lda = 0; q.b = nullptr; q.ldb = 0; q.r = 0;
   q.groups = 1; q.gather = nullptr; q.gather_rows = tokens; q.wmap = RowMap{}; q.wrows = q.N;
@@ -1959,6 +2012,7 @@ hipError_t launch_product_tn(const LoraArgs& p, int64_t tokens, float* part, int
     return launch_cfg<CfgSmall, kBF16, true, 0, false, false, false, true>(q, nullptr, 0);
   }
   q.y = part; q.ldy = q.N;
+  if (big) return launch_cfg<CfgBig, kBF16, true, 0, false, false, true, true>(q, nullptr, 0, splits);
   return launch_cfg<CfgSmall, kBF16, true, 0, false, false, true, true>(q, nullptr, 0, splits);
 }
 
