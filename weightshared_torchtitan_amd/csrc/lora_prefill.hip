@@ -242,8 +242,14 @@ __device__ __forceinline__ void for_ct(F&& f) {
 // computes the classes it has not seen from x and A in global memory (the same k steps in
 // the same order: the same bits), so the launch ends whatever the residency; the last
 // tile to pass (red_cnt[2 rbg + 1]) returns both counters to zero.
+//
+// SHARE: a shared base computed once. The tile is BN rows of W (N = base rows, T of every group
+// from the pre-pass, group j's at column j r of tg); its accumulators are kept, and each of the
+// tpw output copies (group j, head h) is their sum with T_j . B^T of its own B rows, stored at the
+// columns that read these base rows (the inverse of wmap: base row n of a template D wide is column
+// j P + (n / D) S + h D + n % D). r % 16 == 0, D % 8 == 0.
 template <class C, int WDT, bool HAS_W, int RB, bool EXT_T, bool GATHER, bool SPLIT = false, bool TN = false,
-          bool RED = false, bool PER = false, bool WT = false, bool SKT = false>
+          bool RED = false, bool PER = false, bool WT = false, bool SKT = false, bool SHARE = false>
 __global__ void __launch_bounds__(C::NT, 1)
 prefill_kernel(const uint16_t* __restrict__ x, int64_t ldx,
                const int64_t* __restrict__ gidx, int64_t grows,
@@ -288,6 +294,8 @@ prefill_kernel(const uint16_t* __restrict__ x, int64_t ldx,
                 "token-major W': x as it lies, 128-column multiples (fp8: two-buffer ring)");
   static_assert(!SKT || (WDT == kBF16 && HAS_W && RB == 1 && !EXT_T && !GATHER && !SPLIT && !TN && !RED && !PER && !WT),
                 "shared T: one in-loop rank block, bf16 W, one tile per workgroup");
+  static_assert(!SHARE || (WDT == kBF16 && HAS_W && RB == 0 && EXT_T && !GATHER && !SPLIT && !TN && !RED && !PER && !WT),
+                "shared base: bf16 W, T from the pre-pass");
   int64_t tok_rem = grows;  // TN: K rows from this workgroup's first one to the end (>= 1)
   if constexpr (RED) {
     const int64_t kofs = (int64_t)blockIdx.y * K;
@@ -385,13 +393,14 @@ prefill_kernel(const uint16_t* __restrict__ x, int64_t ldx,
   }
   // W rows by output column (mapped for the shared-base forms, whose W is small enough for
   // 32-bit offsets from its start)
-  const int wrow0 = wmap.P == 0 ? n0 : 0;
+  const int wrow0 = SHARE || wmap.P == 0 ? n0 : 0;
   const char* wbase = reinterpret_cast<const char*>(w) + (WDIRECT ? (int64_t)wrow0 * ldw * 2 : 0);
   uint32_t woff[C::NWI];
 #pragma unroll
   for (int i = 0; i < C::NWI; ++i) {
     const int row = (wave * C::NWI + i) * 8 + (lane >> 3);
-    woff[i] = (uint32_t)((map_row(min(n0 + row, N - 1), wmap) - wrow0) * ldw * 2 + fill_chunk(lane, wave * C::NWI + i) * 16);
+    const int wr = min(n0 + row, N - 1);
+    woff[i] = (uint32_t)(((SHARE ? wr : map_row(wr, wmap)) - wrow0) * ldw * 2 + fill_chunk(lane, wave * C::NWI + i) * 16);
   }
   // WT: the W' tile's direct fills, [64 k][BN] as the TN operands lie: fill q of this wave
   // writes lane i's 16 bytes at 1024 q + 16 i of the tile, row (1024 q + 16 i) / (2 BN), and
@@ -773,7 +782,7 @@ prefill_kernel(const uint16_t* __restrict__ x, int64_t ldx,
       issue(1, BK);
       load_w8(BK);
     }
-    if constexpr (LORA) {
+    if constexpr (LORA && !SHARE) {
       if (nk == 1) issue_b(lora_b, 0);
     }
     Frags cur;
@@ -807,7 +816,7 @@ prefill_kernel(const uint16_t* __restrict__ x, int64_t ldx,
         if (kt + 2 < nk) {
           issue(buf, (kt + 2) * BK);
           load_w8((kt + 2) * BK);
-        } else if constexpr (LORA) {
+        } else if constexpr (LORA && !SHARE) {
           issue_b(lora_b, 0);  // kt + 2 == nk: buffer `buf` is lora_b
         }
       }
@@ -834,7 +843,7 @@ prefill_kernel(const uint16_t* __restrict__ x, int64_t ldx,
     };
     issue_w8(lds + WDEC + C::WB, 0);
     for (int q = 0; q < pre; ++q) issue_kt(q, q);
-    if constexpr (LORA) {
+    if constexpr (LORA && !SHARE) {
       if (nk < NS) issue_b(lora_b, 0);  // buffer nk is never filled with a K tile
     }
     if (nk >= NS) wait_vm<(NS - 1) * PT>();  // tile 0 has landed
@@ -874,7 +883,7 @@ prefill_kernel(const uint16_t* __restrict__ x, int64_t ldx,
       cur = nxt;
       if (kt + NS < nk) {
         issue_kt(buf, kt + NS);
-      } else if constexpr (LORA) {
+      } else if constexpr (LORA && !SHARE) {
         if (kt + NS == nk) issue_b(lora_b, 0);  // buffer `buf` is lora_b
       }
       buf = nbuf;
@@ -908,6 +917,112 @@ prefill_kernel(const uint16_t* __restrict__ x, int64_t ldx,
     issue_b(lora_b, 0);
   }
   WSL_STAMP(srec, 2);
+
+  if constexpr (SHARE) {
+    // One copy after another, 64 ranks at a time: the next chunk's T and B fills are in flight while
+    // a finished copy is staged and stored. LDS: the staged output, B's chunk, T's chunk.
+    constexpr int SB = (C::BM * OS + 1023) / 1024 * 1024, ST = SB + C::WB;
+    static_assert(ST + C::XB <= LDS_BYTES, "shared base: LDS areas");
+    const int heads = wmap.S / wmap.D, nrc = (r + 63) / 64;
+    auto out_col = [&](int n) { return n / wmap.D * wmap.S + n % wmap.D; };  // of group 0, head 0
+    int bcol[C::NBI];
+#pragma unroll
+    for (int i = 0; i < C::NBI; ++i) bcol[i] = out_col(min(n0 + (wave * C::NBI + i) * 8 + (lane >> 3), N - 1));
+    // Fills of ranks rk0 .. rk0 + 63 of copy cp (ranks from r on: in-range values of no k step)
+    auto issue_tb = [&](int cp, int rk0) {
+      const int j = cp / heads, c0 = j * wmap.P + (cp - j * heads) * wmap.D;
+      const uint16_t* tj_ = tg_arg + j * r;
+#pragma unroll
+      for (int i = 0; i < C::NBI; ++i) {
+        const int kr = rk0 + fill_chunk(lane, wave * C::NBI + i) * 8;
+        direct_fill(lds + SB, wave * C::NBI + i, bm + (int64_t)(c0 + bcol[i]) * ldb + (kr < r ? kr : 0));
+      }
+#pragma unroll
+      for (int i = 0; i < C::NXI; ++i) {
+        const int fill = wave * C::NXI + i, kr = rk0 + fill_chunk(lane, fill) * 8;
+        const int m = min(m0 + fill * 8 + (lane >> 3), M - 1);
+        direct_fill(lds + ST, fill, tj_ + (int64_t)m * ldt + (kr < r ? kr : 0));
+      }
+    };
+    constexpr int CPR = C::BN / 8, IT = C::BM * CPR / NT;
+    static_assert(NT % CPR == 0 && C::BM * CPR % NT == 0, "a thread stores one column chunk");
+    const bool a16 = ((reinterpret_cast<uintptr_t>(y) & 15u) == 0) && ((ldy & 7) == 0);
+    const bool whole = a16 && m0 + C::BM <= M && n0 + C::BN <= N;
+    const int nst = n0 + tid % CPR * 8;         // this thread's base rows in the store
+    const int yc = out_col(min(nst, N - 8));    // N % 8 == 0
+    issue_tb(0, 0);
+    for (int cp = 0; cp < tpw; ++cp) {
+      f32x16_t out[C::NI][C::MJ];
+#pragma unroll
+      for (int i = 0; i < C::NI; ++i)
+#pragma unroll
+        for (int j = 0; j < C::MJ; ++j) out[i][j] = acc[i][j];
+      for (int rc = 0; rc < nrc; ++rc) {
+        // this chunk has landed; a whole tile's IT stores of the last copy, issued after it, may be out
+        asm volatile("" ::: "memory");
+        if (whole && cp > 0 && rc == 0) wait_vm<IT>();
+        else wait_vm0();
+        ring_barrier();
+        const int nkk = min(4, (r - rc * 64) / 16);
+        for (int kk = 0; kk < nkk; ++kk) {
+          const int c = kk * 2 + lh;
+          bf16x8_t tf[C::MJ], bf[C::NI];
+#pragma unroll
+          for (int j = 0; j < C::MJ; ++j) tf[j] = as_bf16x8(lds_read16(lds + ST, lds_off(wm * C::TM + j * 32 + l32, c)));
+#pragma unroll
+          for (int i = 0; i < C::NI; ++i) bf[i] = as_bf16x8(lds_read16(lds + SB, lds_off(wn * C::TN + i * 32 + l32, c)));
+#pragma unroll
+          for (int i = 0; i < C::NI; ++i)
+#pragma unroll
+            for (int j = 0; j < C::MJ; ++j)
+              out[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bf[i], tf[j], out[i][j], 0, 0, 0);
+        }
+        ring_barrier();  // T and B are read
+        if (rc + 1 < nrc) issue_tb(cp, (rc + 1) * 64);
+      }
+      if (cp + 1 < tpw) issue_tb(cp + 1, 0);
+#pragma unroll
+      for (int j = 0; j < C::MJ; ++j) {
+        const int mr = wm * C::TM + j * 32 + l32;
+#pragma unroll
+        for (int i = 0; i < C::NI; ++i)
+#pragma unroll
+          for (int g = 0; g < 4; ++g) {
+            const f32x16_t& cc = out[i][j];
+            uint2 v;
+            v.x = pack_bf16x2(yscale * cc[g * 4 + 0], yscale * cc[g * 4 + 1]);
+            v.y = pack_bf16x2(yscale * cc[g * 4 + 2], yscale * cc[g * 4 + 3]);
+            *reinterpret_cast<uint2*>(lds + mr * OS + (wn * C::TN + i * 32 + g * 8 + lh * 4) * 2) = v;
+          }
+      }
+      ring_barrier();  // staged (the next copy is staged after the next chunk's barrier, these reads done)
+      const int j = cp / heads;
+      uint16_t* yp = y + j * wmap.P + (cp - j * heads) * wmap.D + yc;
+      u32x4_t v[IT];
+#pragma unroll
+      for (int i = 0; i < IT; ++i)
+        v[i] = *reinterpret_cast<const u32x4_t*>(lds + (i * NT + tid) / CPR * OS + tid % CPR * 16);
+      if (whole) {
+#pragma unroll
+        for (int i = 0; i < IT; ++i)
+          store_y16(v[i], reinterpret_cast<u32x4_t*>(yp + (int64_t)(m0 + (i * NT + tid) / CPR) * ldy));
+        continue;
+      }
+#pragma unroll
+      for (int i = 0; i < IT; ++i) {
+        const int m = m0 + (i * NT + tid) / CPR;
+        if (m >= M || nst >= N) continue;
+        uint16_t* dst = yp + (int64_t)m * ldy;
+        if (a16) {
+          store_y16(v[i], reinterpret_cast<u32x4_t*>(dst));
+        } else {
+          reinterpret_cast<uint2*>(dst)[0] = uint2{v[i][0], v[i][1]};
+          reinterpret_cast<uint2*>(dst)[1] = uint2{v[i][2], v[i][3]};
+        }
+      }
+    }
+    return;
+  }
 
   if constexpr (SKT) {
     // Shared T: publish this tile's class, wait for every class of the row block, sum them
@@ -1303,19 +1418,19 @@ bool groups_fit(const LoraArgs& p, int bn) {
 }
 
 template <class C, int WDT, bool HAS_W, int RB, bool EXT_T, bool GATHER, bool SPLIT = false, bool TN = false,
-          bool RED = false, bool PER = false, bool WT = false, bool SKT = false>
+          bool RED = false, bool PER = false, bool WT = false, bool SKT = false, bool SHARE = false>
 hipError_t launch_cfg(const LoraArgs& p, const uint16_t* tg, int64_t ldt, int splits = 1,
                       uint64_t* red_part = nullptr, unsigned* red_cnt = nullptr, int tpw = 1, int skt_spin = 0) {
   const int tiles_m = (int)((p.M + C::BM - 1) / C::BM);
   const int tiles_n = (int)((p.N + C::BN - 1) / C::BN);
-  prefill_kernel<C, WDT, HAS_W, RB, EXT_T, GATHER, SPLIT, TN, RED, PER, WT, SKT>
+  prefill_kernel<C, WDT, HAS_W, RB, EXT_T, GATHER, SPLIT, TN, RED, PER, WT, SKT, SHARE>
       <<<dim3(tiles_m * tiles_n / (PER ? tpw : 1), splits), dim3(C::NT), 0, p.stream>>>(
       reinterpret_cast<const uint16_t*>(p.x), p.ldx, p.gather, p.gather_rows, p.w, p.ldw, p.w_scale,
       reinterpret_cast<const uint16_t*>(p.a), p.lda, tg, ldt,
       reinterpret_cast<const uint16_t*>(p.b), p.ldb, p.scale, p.yscale,
       reinterpret_cast<uint16_t*>(p.y), p.ldy, (int)p.M, (int)p.N, (int)p.K, (int)p.r, tiles_m, tiles_n,
       group_end(p, 0), group_end(p, 1), group_end(p, 2), p.groups > 1 ? p.r * p.lda : 0,
-      (p.groups > 1 && tg != nullptr) ? (int)p.r : 0, p.wmap, red_part, red_cnt, PER ? tpw : 1, skt_spin);
+      (p.groups > 1 && tg != nullptr) ? (int)p.r : 0, p.wmap, red_part, red_cnt, PER || SHARE ? tpw : 1, skt_spin);
   return hipGetLastError();
 }
 
@@ -2131,6 +2246,44 @@ hipError_t launch_prefill_wt(const LoraArgs& q_in, const uint16_t* tg, int64_t l
   return launch_wt_rank<kBF16>(q, tg, ldt);
 }
 
+// ---- Shared base computed once (the SHARE form) ----
+// The output copies (groups x heads of a template) of a shared-base call whose tiles hold base rows,
+// or 0 where every output column computes its base row anew. A launch over the output columns is
+// bound by its MFMAs, of which all but one copy's base products repeat; computed once, the call
+// pays a pre-pass for T and a serial walk over the copies in each tile's tail instead (about 10 us
+// and 2 us a copy). Graphs of 10 launches, over the columns against once, at the multiply-adds
+// saved: 8.6 G (2^33, the line): 4096 tokens, 2048 -> 2 x 1024: 39.3 / 35.5 us, 8192, 1024 -> 2 x
+// 1024, rank 128: 56.9 / 47.4, 1024, 2048 -> 3 x 2048: 34.8 / 33.5; half of that: 28.0 / 31.6,
+// 26.0 / 32.3, 21.4 / 22.7; above: 4096, 2048 -> 3 x 2048: 125.7 / 57.0, 16384, 2048 -> 2 x 4096
+// over 2048: 439 / 192. K below 1024 leaves too little per copy (512: 43.4 / 43.7).
+int shared_base_copies(const LoraArgs& p) {
+  if (p.wmap.P == 0 || p.w == nullptr || p.w_dtype != kBF16 || p.r == 0 || p.r % 16 != 0 || p.wmap.D % 8 != 0) return 0;
+  const int64_t copies = p.N / p.wrows;
+  if (copies < 2 || p.K < 1024 || (copies - 1) * p.M * p.wrows < ((int64_t)1 << 33) / p.K) return 0;
+  if (rank_prepass_bytes(p.M, p.K, p.r * p.groups) > p.ws_bytes) return 0;
+  return (int)copies;
+}
+
+namespace {
+hipError_t launch_shared_base(const LoraArgs& p, int copies) {
+  uint16_t* t = reinterpret_cast<uint16_t*>(p.ws);
+  const hipError_t e = rank_prepass(p, t);
+  if (e != hipSuccess) return e;
+  LoraArgs q = p;
+  q.N = p.wrows;
+  q.groups = 1;
+  // 128 x 128 tiles while they are one wave, else 128 x 256, whose registers hold the kept
+  // accumulators and a copy's (a 256 x 256 tile's would not fit)
+  const int64_t small = ((q.M + 127) / 128) * ((q.N + 127) / 128);
+  const int64_t ldt = p.r * p.groups;
+  if (small <= 256)
+    return launch_cfg<CfgDeep, kBF16, true, 0, true, false, false, false, false, false, false, false, true>(
+        q, t, ldt, 1, nullptr, nullptr, copies);
+  return launch_cfg<CfgTall3, kBF16, true, 0, true, false, false, false, false, false, false, false, true>(
+      q, t, ldt, 1, nullptr, nullptr, copies);
+}
+}  // namespace
+
 hipError_t launch_prefill(const LoraArgs& p) {
   if (p.gather != nullptr) {
     // factorized embedding: gathered x rows, bf16 base, no LoRA term
@@ -2150,6 +2303,8 @@ hipError_t launch_prefill(const LoraArgs& p) {
   }
   if (pl.form == WSL_PATH_PREFILL_SPLITK) return launch_red(p, pl.splits);
   if (pl.form == WSL_PATH_PREFILL_MEDIUM) return launch_medium(p, pl.splits);
+  const int copies = shared_base_copies(p);
+  if (copies > 0) return launch_shared_base(p, copies);
   const uint16_t* tg = nullptr;
   int64_t ldt = 0;
   if (pl.prepass) {

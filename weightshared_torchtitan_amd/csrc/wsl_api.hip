@@ -2,6 +2,7 @@
 // device check, and dispatch to the prefill / decode / generic kernels.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdarg>
 #include <cstdio>
 #include <atomic>
@@ -542,7 +543,11 @@ int wsl_lora_linear_bcast_workspace_bytes(int64_t M, int64_t N, int64_t K, int64
   }
   int64_t gn[WSL_MAX_GROUPS];
   for (int g = 0; g < n_groups; ++g) gn[g] = N;
-  return wsl_lora_linear_grouped_workspace_bytes(M, K, r, n_groups, gn, w_dtype, bytes);
+  const int rc = wsl_lora_linear_grouped_workspace_bytes(M, K, r, n_groups, gn, w_dtype, bytes);
+  // every group's T where the base is computed once; with less the call computes it per column
+  if (rc == WSL_OK && M > 0 && r > 0)
+    *bytes = std::max(*bytes, layout_bytes(wsl::rank_prepass_bytes(M, K, r * n_groups)));
+  return rc;
 }
 
 int wsl_lora_linear_bcast_fwd(const void* x, int64_t ldx, const void* w, int64_t ldw, int32_t w_dtype_in,
