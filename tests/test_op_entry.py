@@ -130,3 +130,32 @@ def test_calls_follow_the_current_stream(gpu):
         y = ops.lora_linear_op(x, w, None, a, b, 2.0)
     s.synchronize()
     assert ops._stream(x.device) == torch.cuda.current_stream().cuda_stream and torch.equal(y, want)
+
+
+def test_fused_prompt_needs_plain_norms():
+    """The prompt kernels stand for RMSNorm.forward: a norm that does anything else keeps the model
+    on its modules."""
+    from weightshared_torchtitan_amd.qwen3_shared import RMSNorm, SharedQwen3, SharedQwen3Args
+
+    class Other(RMSNorm):
+        pass
+
+    m = SharedQwen3(SharedQwen3Args(dim=64, n_layers=2, n_unique_blocks=1, n_heads=1, n_kv_heads=1, head_dim=64,
+                                    hidden_dim=64, vocab_size=64, embed_rank=64, lora_rank=8, max_seq_len=16))
+    assert m._norms_plain()
+    at = m.base_blocks[0].attention
+    for other in (Other(64, 1e-6), torch.nn.Identity()):
+        kept, at.q_norm = at.q_norm, other
+        assert not m._norms_plain()
+        at.q_norm = kept
+    m.norm.forward = lambda x: x
+    assert not m._norms_plain()
+    del m.norm.forward
+    for register in (at.k_norm.register_forward_hook, torch.nn.modules.module.register_module_forward_hook):
+        h = register(lambda *_: None)
+        assert not m._norms_plain()
+        h.remove()
+    h = torch.nn.modules.module.register_module_forward_pre_hook(lambda *_: None)
+    assert not m._norms_plain()
+    h.remove()
+    assert m._norms_plain()
