@@ -13,7 +13,6 @@ import torch
 
 from weightshared_torchtitan_amd import ops
 
-pytestmark = pytest.mark.gpu
 U = 2.0 ** -8
 
 
@@ -51,6 +50,7 @@ def _check(got, want, names="dx dw da db".split()):
         assert bool((err <= tol).all()), (name, float((err / tol).max()))
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("M,N,K,r,base_n,g,G", [
     (1, 128, 64, 8, 64, 1, 1),         # one row, one group
     (63, 64, 128, 16, 64, 2, 3),       # N = base_n, below one token tile
@@ -76,6 +76,7 @@ def test_bcast_grads(gpu, M, N, K, r, base_n, g, G):
     _check(no_lora[:2], _oracle(*host[:3], *zero, 2.0, g, G)[:2])
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("case", ["strided", "offset", "template 4", "rank 12", "K off", "K off rank"])
 def test_bcast_backward_routes(gpu, case):
     """The op's backward over layouts: rows 16 bytes apart in wider buffers, storage off 16 bytes, and
@@ -108,3 +109,58 @@ def test_bcast_backward_routes(gpu, case):
         v, tol = want[0]
         want[0] = (v, 3 * tol)
     _check(got, want)
+
+
+def _wrong():
+    """Name -> operands that do not belong together, and whether the factors' gradients are asked for."""
+    M, N, K, r, base_n, G = 24, 128, 64, 8, 64, 2
+    good = dict(zip(("x", "gy", "w", "a", "b"), _operands(M, N, K, r, base_n, G, seed=1)), g=2, n_groups=G)
+    z = lambda *s: torch.zeros(*s, dtype=torch.bfloat16)  # noqa: E731
+    for name, change in {
+        "gy rows": {"gy": z(M - 1, G * N)}, "gy columns": {"gy": z(M, G * N - 1)}, "N": {"gy": z(M, G * 96)},
+        "w columns": {"w": z(base_n, K - 8)}, "a rows": {"a": z(r, K)}, "a columns": {"a": z(G * r, K - 8)},
+        "b rows": {"b": z(N, r)}, "a alone": {"b": None}, "b alone": {"a": None}, "no factors": {"a": None, "b": None},
+        "rank 0": {"a": z(0, K), "b": z(G * N, 0)}, "template": {"g": 3}, "no template": {"g": 0},
+        "no group": {"n_groups": 0}, "groups": {"n_groups": 5}, "3-d": {"x": z(2, M // 2, K)},
+        **{f"{n} type": {n: good[n].float()} for n in ("x", "gy", "w", "a", "b")},
+    }.items():
+        yield name, {**good, **change}
+
+
+@pytest.mark.parametrize("name,args", _wrong(), ids=lambda v: v if isinstance(v, str) else "")
+def test_operands_that_do_not_match_are_refused(name, args):
+    with pytest.raises((TypeError, ValueError)):
+        ops._bcast_grads_operands(**args, need_ab=True)
+
+
+@pytest.mark.gpu
+def test_bcast_grads_op_checks_its_operands(gpu):
+    for name, args in _wrong():
+        print(f"[bcast grads] refused: {name}", flush=True)
+        x, gy, w, a, b = (args[n].to(gpu) if args[n] is not None else None for n in ("x", "gy", "w", "a", "b"))
+        for op in (ops.lora_linear_bcast_grads_op, torch.ops.wsl.lora_linear_bcast_grads):
+            with pytest.raises((TypeError, ValueError)):
+                op(x, gy, w, a, b, 2.0, args["g"], args["n_groups"], True, True, True, True)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("which", range(5))
+@pytest.mark.parametrize("layout", ["columns apart", "transposed", "overlapping"])
+def test_bcast_grads_takes_any_strides(gpu, which, layout):
+    """An operand with columns apart, transposed, or with rows that overlap gives the gradients of its values."""
+    M, N, K, r, base_n, g, G = 65, 128, 128, 16, 64, 2, 2
+    print(f"[bcast grads] operand {which} {layout}", flush=True)
+    host = list(_operands(M, N, K, r, base_n, G, seed=3))
+    dev = [t.to(gpu) for t in host]
+    t = dev[which]
+    if layout == "columns apart":
+        buf = torch.full((t.shape[0], 2 * t.shape[1]), float("nan"), dtype=t.dtype, device=gpu)
+        buf[:, ::2] = t
+        dev[which] = buf[:, ::2]
+    elif layout == "transposed":
+        dev[which] = t.t().contiguous().t()
+    else:  # row i + 1 starts 8 elements after row i
+        line = t.flatten()[:8 * (t.shape[0] - 1) + t.shape[1]].contiguous()
+        dev[which] = line.as_strided(t.shape, (8, 1))
+        host[which] = dev[which].cpu()
+    _check(ops.lora_linear_bcast_grads_op(*dev, 2.0, g, G, True, True, True, True), _oracle(*host, 2.0, g, G))

@@ -671,15 +671,43 @@ def _lora_linear_bcast_fake(x, w, w_scale, a, b, scale, g, n_groups):
     return x.new_empty((*x.shape[:-1], int(n_groups) * N), dtype=torch.bfloat16)
 
 
+def _bcast_grads_operands(x, gy, w, a, b, g: int, n_groups: int, need_ab: bool):
+    """x, gy, w, a and b of lora_linear_bcast_grads with contiguous rows, after every check of their
+    types and sizes against one another: the C entry sees pointers and row strides only."""
+    ts = [t for t in (x, gy, w, a, b) if t is not None]
+    if any(t.dtype != torch.bfloat16 for t in ts):
+        raise TypeError(f"x, grad_y, w, a and b must be bfloat16, got {[t.dtype for t in ts]}")
+    x, gy, w = _row_major(x, "x"), _row_major(gy, "grad_y"), _row_major(w, "w")
+    (M, K), base_n, G = x.shape, w.shape[0], n_groups
+    if not 1 <= G <= _native.WSL_MAX_GROUPS:
+        raise ValueError(f"n_groups must be in [1, {_native.WSL_MAX_GROUPS}], got {G}")
+    if gy.shape[0] != M or gy.shape[1] % G != 0 or w.shape[1] != K:
+        raise ValueError(f"x {tuple(x.shape)}, grad_y {tuple(gy.shape)} and w {tuple(w.shape)} do not match {G} groups")
+    N = gy.shape[1] // G
+    if base_n < 1 or g < 1 or N < 1 or N % base_n != 0 or base_n % g != 0:
+        raise ValueError(f"broadcast needs N % base_n == 0 and base_n % g == 0 (N {N}, base_n {base_n}, g {g})")
+    if (a is None) != (b is None):
+        raise ValueError("a and b must be given together")
+    if a is not None:
+        a, b = _row_major(a, "a"), _row_major(b, "b")
+        if a.shape != (G * b.shape[1], K) or b.shape[0] != G * N:
+            raise ValueError(f"LoRA shapes a {tuple(a.shape)}, b {tuple(b.shape)} do not match {G} groups, K={K}, N={N}")
+    if need_ab and (b is None or b.shape[1] == 0):
+        raise ValueError("da and db need a and b of rank 1 or more")
+    return x, gy, w, a, b
+
+
 @_custom_op("lora_linear_bcast_grads")
 def lora_linear_bcast_grads_op(x: torch.Tensor, gy: torch.Tensor, w: torch.Tensor, a: Optional[torch.Tensor],
                                b: Optional[torch.Tensor], scale: float, g: int, n_groups: int, need_x: bool,
                                need_w: bool, need_a: bool,
                                need_b: bool) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]:
     """(dx [M, K], dw, da, db) of wsl::lora_linear_bcast, each only when asked for (else an empty
-    tensor), for x [M, K] and gy [M, n_groups * N] (wsl_lora_linear_bcast_bwd; raises for the layouts
-    it does not take: see bcast_grads_supported)."""
+    tensor), for x [M, K] and gy [M, n_groups * N] (wsl_lora_linear_bcast_bwd; operands whose rows
+    do not lie as it reads them go through a copy, sizes it does not take raise: see
+    bcast_grads_supported)."""
     dev = _check_device(x, gy, w, a, b)
+    x, gy, w, a, b = _bcast_grads_operands(x, gy, w, a, b, g, n_groups, need_a or need_b)
     M, K = x.shape
     base_n, N, r = w.shape[0], gy.shape[1] // n_groups, b.shape[1] if b is not None else 0
     mk = lambda need, *s: x.new_empty(s if need else 0)  # noqa: E731
