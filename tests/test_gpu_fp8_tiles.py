@@ -105,6 +105,38 @@ def test_fp8_splits_of_k(gpu, wsl_opts, M, N, K, r, splits):
     assert rel(ops.lora_linear_op(x, q, sc, a, b, 1.0), ref) <= TOL
 
 
+@pytest.mark.parametrize("M,N,K,r", [(65, 512, 1024, 16), (100, 1000, 4096, 8), (333, 4096, 4096, 64),
+                                     (200, 1024, 4096, 40)])
+def test_fp8_splits_keep_parts_of_t_that_cancel(gpu, wsl_opts, M, N, K, r):
+    """T = x . A^T whose halves of K, in different splits, nearly cancel. The operands are small
+    multiples of powers of two, so every sum is exact in fp32 in any order, and the error is T's
+    rounding (at most one, u = 2^-8 of |T|) and y's: u |y| + u (1 + u) sum |T| |B|."""
+    from weightshared_torchtitan_amd import ops
+    _say(f"[fp8 split-K, cancelling T] M={M} N={N} K={K} r={r}")
+    pl = ops.plan(M, K, r, [N], fp8=True)
+    assert pl["path"] == "prefill_splitk" and pl["k_splits"] % 2 == 0 and not pl["rank_prepass"]
+    g = torch.Generator(device="cuda").manual_seed(r)
+    ints = lambda n, *s: torch.randint(-n, n + 1, s, device=gpu, generator=g)  # noqa: E731
+    v, e = ints(16, M, K // 2), ints(1, M, K // 2) * (ints(8, M, K // 2) == 0)
+    x = (torch.cat([v, e - v], 1) / 8).bfloat16()
+    a = (ints(16, r, K // 2) / 64).repeat(1, 2).bfloat16()
+    b = (ints(16, N, r) / 64).bfloat16()
+    W = torch.zeros(N, K, device=gpu).to(torch.float8_e4m3fn)
+    y = ops.lora_linear_op(x, W, torch.ones(N, device=gpu), a, b, 2.0).double()
+    t = 2.0 * x.double() @ a.double().t()
+    want = t @ b.double().t()
+    parts = 2.0 * x[:, :K // 2].double() @ a[:, :K // 2].double().t()
+    assert float(parts.abs().mean()) > 16 * float(t.abs().mean())
+    u = 2.0 ** -8
+    tol = u * want.abs() + u * (1 + u) * t.abs() @ b.double().abs().t()
+    assert bool(((y - want).abs() <= tol).all()), float(((y - want).abs() / tol.clamp_min(1e-30)).max())
+    x[3, 5] = float("inf")  # the terms of an infinite part of T are itself and zeros
+    W = torch.ones(N, K, device=gpu).to(torch.float8_e4m3fn)
+    got = ops.lora_linear_op(x, W, torch.ones(N, device=gpu), a, b, 2.0)
+    ref = (2.0 * x.double() @ a.double().t()) @ b.double().t() + x.double() @ W.double().t()
+    assert torch.equal(got.isnan(), ref.isnan()) and torch.equal(got.isinf(), ref.isinf())
+
+
 def test_fp8_grouped_and_shared_base_rows(gpu, wsl_opts):
     from weightshared_torchtitan_amd import ops
     wsl_opts(fp8_prefill=1)
