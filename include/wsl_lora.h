@@ -297,13 +297,22 @@ int wsl_lora_linear_bwd_input_any(const void* gy, int64_t ldg, const void* w, in
                                   void* stream);
 
 /*
- * LoRA factors of a rank that the tiled kernels do not take (off 8), padded with zeros: a
- * [n_groups * r, K] -> a_out [n_groups * r_padded, K] (each group's rows followed by zero rows),
- * b [N, r] -> b_out [N, r_padded], both outputs dense. A LoRA linear with the padded factors is
- * that with the original ones.
+ * LoRA factors of a rank that the tiled kernels do not take (off 8) at the next rank they do:
+ * a [n_groups * r, K] -> a_out [n_groups * r_padded, K], b [N, r] -> b_out [N, r_padded], both
+ * outputs dense.
+ *
+ * wsl_lora_pad_rank fills up with zeros. The gradients of the padded factors are those of the
+ * original ones in the first r ranks. A product through them is that through the original ones on
+ * finite operands; an infinity in x (or gy) makes its row NaN (Inf . 0).
+ * wsl_lora_spread_rank repeats ranks instead (rank q is rank q % r of A, the columns of B shared
+ * among the copies in powers of two), and products keep their infinities: what
+ * y = x . W^T + s (x . A^T) . B^T and dx = gy . W + s (gy . B) . A take. The shares are exact unless
+ * a column of B reaches the subnormal range.
  */
 int wsl_lora_pad_rank(const void* a, int64_t lda, const void* b, int64_t ldb, int32_t n_groups, int64_t r,
                       int64_t r_padded, int64_t K, int64_t N, void* a_out, void* b_out, void* stream);
+int wsl_lora_spread_rank(const void* a, int64_t lda, const void* b, int64_t ldb, int32_t n_groups, int64_t r,
+                         int64_t r_padded, int64_t K, int64_t N, void* a_out, void* b_out, void* stream);
 
 /*
  * Factorized embedding:  out[t, :] = E[ids[t], :] . P^T      (k -> hidden)

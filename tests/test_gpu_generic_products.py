@@ -1,7 +1,7 @@
 """The products for layouts off the tiled kernels (csrc/lora_generic.hip) at the edges of their
 tiles (64 x 64 over k steps of 128; 128 x 128 over 64 where those fill the chip), with odd
 strides and unaligned pointers, forward and every gradient against plain torch in float64; and
-ranks off 8 on grid shapes, which the ops pad with zeros onto the tiled kernels."""
+ranks off 8 on grid shapes, which the ops bring to the next multiple of 8 for the tiled kernels."""
 import sys
 
 import pytest
@@ -117,6 +117,34 @@ def test_generic_fp8_base(gpu, M, N, K, r):
     y = ops.lora_linear_op(x, q, sc, a, b, 1.0)
     ref = x.double() @ (q.double() * sc.double()[:, None]).t() + (x.double() @ a.double().t()) @ b.double().t()
     assert rel(y, ref) <= TOL
+
+
+@pytest.mark.parametrize("r", [1, 2, 3, 5, 7, 12, 63])
+@pytest.mark.parametrize("M,N,K", [(4, 256, 512), (70, 512, 1024), (200, 384, 256), (2050, 512, 128), (70, 100, 104)])
+def test_infinities_stay_infinities_at_ranks_off_8(gpu, M, N, K, r):
+    """A row of x (or grad_y) with an infinity: each output is the infinity or NaN that its own terms
+    sum to (the decode, split-K, tiled, pre-pass and generic forms). Positive factors at the
+    infinity's column, so that the low-rank term is +Inf and half of the base products agree."""
+    from weightshared_torchtitan_amd import ops
+    _say(f"[infinities, rank off 8] M={M} N={N} K={K} r={r}")
+    x, w, a, b, gy = inputs(gpu, M, N, K, r, 11 + r)
+    a, b = a.abs() + 2.0 ** -6, b.abs() + 2.0 ** -6
+    x[2, 7] = gy[1, 5] = float("inf")
+    X, W, A, B, G = (t.double().cpu() for t in (x, w, a, b, gy))
+    wide = torch.cat([b, b.flip(0)])  # two groups: their own factors, one base twice
+    got = [(ops.lora_linear_op(x, w, None, a, b, 2.0), X @ W.t() + 2.0 * (X @ A.t()) @ B.t()),
+           (ops.lora_linear_op(x, None, None, a, b, 2.0), 2.0 * (X @ A.t()) @ B.t()),
+           (ops.lora_linear_bwd_input_op(gy, w, None, a, b, 2.0), G @ W + 2.0 * (G @ B) @ A),
+           (ops.lora_linear_grouped_op(x, torch.cat([w, w]), None, torch.cat([a, a]), wide, 2.0, [N, N]),
+            torch.cat([X @ W.t() + 2.0 * (X @ A.t()) @ f.t() for f in (B, B.flip(0))], 1)),
+           (ops.lora_linear_bcast_op(x, w, None, torch.cat([a, a]), wide, 2.0, 1, 2),
+            torch.cat([X @ W.t() + 2.0 * (X @ A.t()) @ f.t() for f in (B, B.flip(0))], 1))]
+    for y, ref in got:
+        y = y.double().cpu()
+        assert bool(ref.isinf().any()) and torch.equal(y.isnan(), ref.isnan())
+        assert torch.equal(y == float("inf"), ref == float("inf")) and torch.equal(y.isfinite(), ref.isfinite())
+        ok = ref.isfinite()
+        assert rel(y[ok], ref[ok]) <= TOL
 
 
 def test_nan_stays_in_its_rows_and_columns(gpu):

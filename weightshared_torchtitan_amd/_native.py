@@ -56,6 +56,7 @@ EXPORTED = (
     "wsl_lora_linear_bwd_input_any_workspace_bytes",
     "wsl_lora_linear_bwd_input_any",
     "wsl_lora_pad_rank",
+    "wsl_lora_spread_rank",
     "wsl_factorized_embedding_fwd",
     "wsl_last_error",
     "wsl_version",
@@ -266,11 +267,12 @@ def _declare(lib: ctypes.CDLL) -> None:
         _c_vp, ctypes.c_size_t,          # workspace, bytes
         _c_vp,                           # stream
     ]
-    lib.wsl_lora_pad_rank.restype = ctypes.c_int
-    lib.wsl_lora_pad_rank.argtypes = [
-        _c_vp, _c_i64, _c_vp, _c_i64,                  # a, lda, b, ldb
-        ctypes.c_int32, _c_i64, _c_i64, _c_i64, _c_i64,  # n_groups, r, r_padded, K, N
-        _c_vp, _c_vp, _c_vp]                           # a_out, b_out, stream
+    for pad in (lib.wsl_lora_pad_rank, lib.wsl_lora_spread_rank):
+        pad.restype = ctypes.c_int
+        pad.argtypes = [
+            _c_vp, _c_i64, _c_vp, _c_i64,                  # a, lda, b, ldb
+            ctypes.c_int32, _c_i64, _c_i64, _c_i64, _c_i64,  # n_groups, r, r_padded, K, N
+            _c_vp, _c_vp, _c_vp]                           # a_out, b_out, stream
     lib.wsl_decode_last_error.restype = ctypes.c_char_p
     lib.wsl_decode_last_error.argtypes = []
     lib.wsl_rmsnorm_fwd.restype = ctypes.c_int

@@ -449,6 +449,11 @@ hipError_t launch_weight_grads_generic(const LoraArgs& p, const void* gy, int64_
 }
 
 namespace {
+// SPREAD: rank q of a group's rp takes row q % r of A, and the copies of one rank share its column
+// of B in powers of two that sum to one (1; 1/2, 1/2; 1/2, 1/4, 1/4; ..). Zeros instead would make
+// T's padding Inf . 0 = NaN in a row of x that holds an infinity, and with it the whole row of y;
+// a copy's product with its share has the sign of the rank it copies, so y keeps its infinities.
+template <bool SPREAD>
 __global__ void __launch_bounds__(256) pad_rank_kernel(const uint16_t* __restrict__ a, int64_t lda,
                                                       const uint16_t* __restrict__ b, int64_t ldb, int64_t na,
                                                       int64_t nb, int64_t r, int64_t rp, int64_t K,
@@ -456,19 +461,25 @@ __global__ void __launch_bounds__(256) pad_rank_kernel(const uint16_t* __restric
   const int64_t e = (int64_t)blockIdx.x * 256 + threadIdx.x;
   if (e < na) {
     const int64_t row = e / K, k = e % K, j = row % rp;
-    a_out[e] = j < r ? a[(row / rp * r + j) * lda + k] : 0;
+    a_out[e] = SPREAD || j < r ? a[(row / rp * r + j % r) * lda + k] : 0;
   } else if (e - na < nb) {
-    const int64_t n = (e - na) / rp, j = (e - na) % rp;
-    b_out[e - na] = j < r ? b[n * ldb + j] : 0;
+    const int64_t n = (e - na) / rp, q = (e - na) % rp, j = q % r;
+    if (SPREAD) {
+      const int copy = (int)(q / r), last = (int)(rp / r) - (j < rp % r ? 0 : 1);
+      b_out[e - na] = f32_to_bf16_bits(ldexpf(bf16_bits_to_f32(b[n * ldb + j]), -min(copy + 1, last)));
+    } else {
+      b_out[e - na] = q < r ? b[n * ldb + j] : 0;
+    }
   }
 }
 }  // namespace
 
 hipError_t launch_pad_rank(const void* a, int64_t lda, const void* b, int64_t ldb, int groups, int64_t r, int64_t rp,
-                           int64_t K, int64_t N, void* a_out, void* b_out, hipStream_t st) {
+                           int64_t K, int64_t N, void* a_out, void* b_out, bool spread, hipStream_t st) {
   const int64_t na = groups * rp * K, nb = N * rp, blocks = (na + nb + 255) / 256;
   if (blocks > 0x7fffffff) return hipErrorInvalidValue;
-  pad_rank_kernel<<<dim3((unsigned)blocks), dim3(256), 0, st>>>(
+  const auto kernel = spread ? pad_rank_kernel<true> : pad_rank_kernel<false>;
+  kernel<<<dim3((unsigned)blocks), dim3(256), 0, st>>>(
       reinterpret_cast<const uint16_t*>(a), lda, reinterpret_cast<const uint16_t*>(b), ldb, na, nb, r, rp, K,
       reinterpret_cast<uint16_t*>(a_out), reinterpret_cast<uint16_t*>(b_out));
   return hipGetLastError();

@@ -808,8 +808,8 @@ int wsl_lora_linear_bwd_input_any(const void* gy, int64_t ldg, const void* w, in
   return WSL_OK;
 }
 
-int wsl_lora_pad_rank(const void* a, int64_t lda, const void* b, int64_t ldb, int32_t n_groups, int64_t r,
-                      int64_t r_padded, int64_t K, int64_t N, void* a_out, void* b_out, void* stream) {
+static int pad_rank(bool spread, const void* a, int64_t lda, const void* b, int64_t ldb, int32_t n_groups, int64_t r,
+                    int64_t r_padded, int64_t K, int64_t N, void* a_out, void* b_out, void* stream) {
   clear_err();
   if (n_groups < 1 || n_groups > WSL_MAX_GROUPS)
     return fail(WSL_E_SHAPE, "n_groups must be in [1, %d] (got %d)", WSL_MAX_GROUPS, (int)n_groups);
@@ -823,10 +823,20 @@ int wsl_lora_pad_rank(const void* a, int64_t lda, const void* b, int64_t ldb, in
     return fail(WSL_E_ALIGN, "pointers must be aligned to their element size");
   const int dc = check_device();
   if (dc != WSL_OK) return dc;
-  const hipError_t e = wsl::launch_pad_rank(a, lda, b, ldb, n_groups, r, r_padded, K, N, a_out, b_out,
+  const hipError_t e = wsl::launch_pad_rank(a, lda, b, ldb, n_groups, r, r_padded, K, N, a_out, b_out, spread,
                                             reinterpret_cast<hipStream_t>(stream));
   if (e != hipSuccess) return fail(WSL_E_LAUNCH, "kernel launch failed: %s", hipGetErrorString(e));
   return WSL_OK;
+}
+
+int wsl_lora_pad_rank(const void* a, int64_t lda, const void* b, int64_t ldb, int32_t n_groups, int64_t r,
+                      int64_t r_padded, int64_t K, int64_t N, void* a_out, void* b_out, void* stream) {
+  return pad_rank(false, a, lda, b, ldb, n_groups, r, r_padded, K, N, a_out, b_out, stream);
+}
+
+int wsl_lora_spread_rank(const void* a, int64_t lda, const void* b, int64_t ldb, int32_t n_groups, int64_t r,
+                         int64_t r_padded, int64_t K, int64_t N, void* a_out, void* b_out, void* stream) {
+  return pad_rank(true, a, lda, b, ldb, n_groups, r, r_padded, K, N, a_out, b_out, stream);
 }
 
 int wsl_lora_linear_fused_supported(int64_t M, int64_t N, int64_t K, int64_t r, int32_t fuse) {

@@ -259,10 +259,10 @@ hipError_t launch_weight_grads_generic(const LoraArgs& p, const void* gy, int64_
                                        void* da, int64_t ldda, void* db, int64_t lddb, int64_t r, uint16_t* t,
                                        uint16_t* u);
 hipError_t launch_bwd_input_generic(const LoraArgs& p, uint16_t* u);
-// a [groups * r, K] and b [N, r] with each group's rows of a and the columns of b padded with
-// zeros to rank rp: a_out [groups * rp, K], b_out [N, rp].
+// a [groups * r, K] and b [N, r] at rank rp: a_out [groups * rp, K], b_out [N, rp], with zeros past
+// each group's r ranks, or (spread) with copies that share the ranks they copy.
 hipError_t launch_pad_rank(const void* a, int64_t lda, const void* b, int64_t ldb, int groups, int64_t r, int64_t rp,
-                           int64_t K, int64_t N, void* a_out, void* b_out, hipStream_t st);
+                           int64_t K, int64_t N, void* a_out, void* b_out, bool spread, hipStream_t st);
 
 hipError_t launch_factorized_embedding(const int64_t* ids, int64_t n_ids, const void* emb,
                                        int64_t lde, int64_t vocab, int64_t k, const void* proj,

@@ -234,18 +234,20 @@ def _pads_rank(r: int, x: torch.Tensor, K: int) -> bool:
     return r % 8 != 0 and (r < 8 or (K % 64 == 0 and _rows16(x)))
 
 
-def _pad_rank(a: torch.Tensor, b: torch.Tensor, groups: int) -> tuple[torch.Tensor, torch.Tensor, int]:
-    """a [groups * r, K] and b [N, r] with zeros up to the next rank in multiples of 8, and that
-    rank (one launch): the same LoRA term, on factors whose rows the tiled kernels take."""
+def _pad_rank(a: torch.Tensor, b: torch.Tensor, groups: int,
+              spread: bool = True) -> tuple[torch.Tensor, torch.Tensor, int]:
+    """a [groups * r, K] and b [N, r] at the next rank in multiples of 8, and that rank (one launch):
+    the same LoRA term, on factors whose rows the tiled kernels take. `spread`: ranks repeated, for
+    products (they keep their infinities); else zeros, for the factors' own gradients."""
     N, r = b.shape
     K, rp = a.shape[1], (r + 7) // 8 * 8
     both = torch.empty(groups * rp * K + N * rp, dtype=torch.bfloat16, device=b.device)
     ap, bp = both[:groups * rp * K].view(groups * rp, K), both[groups * rp * K:].view(N, rp)
+    name = "wsl_lora_spread_rank" if spread else "wsl_lora_pad_rank"
     with _on(b.device):
-        rc = _native.lib().wsl_lora_pad_rank(a.data_ptr(), a.stride(0), b.data_ptr(), b.stride(0), groups, r, rp, K, N,
-                                             ap.data_ptr(), bp.data_ptr(),
-                                             _stream(b.device))
-    _native.check(rc, "wsl_lora_pad_rank")
+        rc = getattr(_native.lib(), name)(a.data_ptr(), a.stride(0), b.data_ptr(), b.stride(0), groups, r, rp, K, N,
+                                          ap.data_ptr(), bp.data_ptr(), _stream(b.device))
+    _native.check(rc, name)
     return ap, bp, rp
 
 
@@ -333,7 +335,7 @@ def lora_linear_bwd_input_op(gy: torch.Tensor, w: torch.Tensor, w_scale: Optiona
     float8_e4m3fn with w_scale [N] fp32: W = bf16(w * w_scale[:, None]) row by row),
     a [r, K] and b [N, r] as the forward takes them (a and b None: r = 0):
     wsl_lora_linear_bwd_input, the fused kernel reading w where it lies as the reduction rows
-    of its tiles. Ranks off 8 are padded with zeros. Layouts that entry point does not take (N off
+    of its tiles. Ranks off 8 are padded. Layouts that entry point does not take (N off
     the 64 grid, K off 8, unaligned rows) run on wsl_lora_linear_bwd_input_any, or, where the
     forward's tiled kernels take the transposed problem, the forward op on a copy of W^T."""
     dev = _check_device(gy, w, w_scale, a, b)
@@ -441,7 +443,7 @@ def lora_linear_weight_grads_op(x: torch.Tensor, gy: torch.Tensor, a: Optional[t
     L = _native.lib()
     r0 = r
     if _pads_rank(r, x2, K) and (r < 8 or (N % 64 == 0 and _rows16(gy2))):
-        a, b, r = _pad_rank(a, b, 1)
+        a, b, r = _pad_rank(a, b, 1, spread=False)
     dw = torch.empty((N, K), dtype=torch.bfloat16, device=dev) if need_w else None
     da = torch.empty((r, K), dtype=torch.bfloat16, device=dev) if need_a else None
     db = torch.empty((N, r), dtype=torch.bfloat16, device=dev) if need_b else None
