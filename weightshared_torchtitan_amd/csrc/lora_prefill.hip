@@ -1856,7 +1856,7 @@ int red_splits(int64_t M, int64_t N, int64_t K, int w_dtype, bool has_w, bool ga
 
 // An fp8 W (8B shapes, graphs of 20 launches, us, the unsplit launch before): 80 x 4096 x 12288
 // 139.7 -> 39.4 at r = 16, 147.1 -> 49.1 at r = 128 (pre-pass included); 333 x 4096 x 4096 51.9 ->
-// 37.4 and 62.2 -> 47.1; 600 x 1024 x 4096 51.7 -> 26.0; 80 x 12288 x 4096 50.2 -> 37.5. T's parts
+// 37.4 and 62.2 -> 47.1; 600 x 1024 x 4096 51.7 -> 26.0; 80 x 12288 x 4096 50.2 -> 36.1. T's parts
 // as three bf16 terms are 0.7-1.2 us of these at ranks 8-16, 1.5-2.2 at rank 64 (against one term
 // each, 38.5 -> 39.4 and 41.8 -> 44.0 at 80 x 4096 x 12288; the distance from 64-bit results
 // 1.685e-3 -> 1.664e-3 at rank 64, random inputs). The splits
