@@ -162,6 +162,44 @@ def test_model_forward_fused_matches_torch_ops_and_oracle(gpu, b, s, grouped, ca
             assert not x[:, :, :, s:].any()
 
 
+@pytest.mark.parametrize("what", ["norm", "q norm", "rope", "cache"])
+def test_model_forward_with_operands_off_16_bytes(gpu, what):
+    """Norm weights, a RoPE table or a cache in views that start off 16 bytes (a flat parameter buffer's,
+    say), which the kernels do not read: the forward runs on its modules, with the same results."""
+    from weightshared_torchtitan_amd.qwen3_shared import KVCache, SharedQwen3, SharedQwen3Args
+    _say(f"[model forward] {what} off 16 bytes")
+    a = SharedQwen3Args(dim=128, n_layers=2, n_unique_blocks=1, n_heads=2, n_kv_heads=1, head_dim=64, hidden_dim=128,
+                        vocab_size=300, embed_rank=64, lora_rank=8, max_seq_len=64)
+    m = SharedQwen3(a)
+    m.init_random(seed=2, std=0.05)
+    m = m.to(gpu).to(torch.bfloat16)
+    toks = torch.arange(40, device=gpu).view(2, 20)
+
+    def off(t):  # the same values one element into a buffer of their own
+        buf = torch.zeros(t.numel() + 1, dtype=t.dtype, device=t.device)
+        buf[1:] = t.flatten()
+        return buf[1:].view(t.shape)
+
+    with torch.no_grad():
+        m.prefill_fusion = False
+        cache = KVCache(a, 2, 24, gpu)
+        want = m(toks, cache), cache.k
+        m.prefill_fusion = True
+        cache = KVCache(a, 2, 24, gpu)
+        assert m._prefill_fused_ok(toks, cache)
+        blk = m.base_blocks[0]
+        if what == "cache":
+            cache.v = off(cache.v)
+        elif what == "rope":
+            m.rope = off(m.rope)
+        else:
+            norm = blk.ffn_norm if what == "norm" else blk.attention.q_norm
+            norm.weight = torch.nn.Parameter(off(norm.weight.detach()))
+        got = m(toks, cache)
+    assert not m._prefill_fused_ok(toks, cache)
+    assert torch.equal(got, want[0]) and torch.equal(cache.k, want[1])
+
+
 def test_opcheck_prompt_ops(gpu):
     from weightshared_torchtitan_amd import ops  # noqa: F401
     utils = ("test_schema", "test_faketensor", "test_aot_dispatch_dynamic")
