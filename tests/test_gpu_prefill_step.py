@@ -162,12 +162,13 @@ def test_model_forward_fused_matches_torch_ops_and_oracle(gpu, b, s, grouped, ca
             assert not x[:, :, :, s:].any()
 
 
-@pytest.mark.parametrize("what", ["norm", "q norm", "rope", "cache"])
-def test_model_forward_with_operands_off_16_bytes(gpu, what):
+@pytest.mark.parametrize("compiled", [False, True])
+@pytest.mark.parametrize("what", ["norm", "q norm", "k norm", "rope", "cache"])
+def test_model_forward_with_operands_off_16_bytes(gpu, what, compiled):
     """Norm weights, a RoPE table or a cache in views that start off 16 bytes (a flat parameter buffer's,
-    say), which the kernels do not read: the forward runs on its modules, with the same results."""
+    say) give what aligned ones give, eager and compiled into one graph."""
     from weightshared_torchtitan_amd.qwen3_shared import KVCache, SharedQwen3, SharedQwen3Args
-    _say(f"[model forward] {what} off 16 bytes")
+    _say(f"[model forward] {what} off 16 bytes, compiled={compiled}")
     a = SharedQwen3Args(dim=128, n_layers=2, n_unique_blocks=1, n_heads=2, n_kv_heads=1, head_dim=64, hidden_dim=128,
                         vocab_size=300, embed_rank=64, lora_rank=8, max_seq_len=64)
     m = SharedQwen3(a)
@@ -181,23 +182,23 @@ def test_model_forward_with_operands_off_16_bytes(gpu, what):
         return buf[1:].view(t.shape)
 
     with torch.no_grad():
-        m.prefill_fusion = False
-        cache = KVCache(a, 2, 24, gpu)
-        want = m(toks, cache), cache.k
-        m.prefill_fusion = True
         cache = KVCache(a, 2, 24, gpu)
         assert m._prefill_fused_ok(toks, cache)
+        want = m(toks, cache), cache.k, cache.v
+        cache = KVCache(a, 2, 24, gpu)
         blk = m.base_blocks[0]
         if what == "cache":
-            cache.v = off(cache.v)
+            cache.k, cache.v = off(cache.k), off(cache.v)
         elif what == "rope":
-            m.rope = off(m.rope)
+            m.rope = off(m.rope.float())
         else:
-            norm = blk.ffn_norm if what == "norm" else blk.attention.q_norm
+            norm = {"norm": blk.ffn_norm, "q norm": blk.attention.q_norm, "k norm": blk.attention.k_norm}[what]
             norm.weight = torch.nn.Parameter(off(norm.weight.detach()))
-        got = m(toks, cache)
-    assert not m._prefill_fused_ok(toks, cache)
-    assert torch.equal(got, want[0]) and torch.equal(cache.k, want[1])
+        assert m._prefill_fused_ok(toks, cache)
+        torch._dynamo.reset()
+        got = (torch.compile(m, backend="eager", fullgraph=True) if compiled else m)(toks, cache)
+    for x, y in zip((got, cache.k, cache.v), want):
+        assert torch.equal(x, y)
 
 
 def test_opcheck_prompt_ops(gpu):

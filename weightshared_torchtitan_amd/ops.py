@@ -1059,6 +1059,12 @@ def _bf16_2d(t: torch.Tensor, name: str) -> torch.Tensor:
     return t
 
 
+def _aligned(t: torch.Tensor) -> torch.Tensor:
+    """A contiguous tensor as it is, or a copy of it where it does not start on 16 bytes (a view into a
+    flat parameter buffer, say): the kernels read these in 16-byte pieces."""
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
 def _check_rope(rope: torch.Tensor, cache_len: int, head_dim: int) -> None:
     """The RoPE table must cover every cache position: [>= cache_len, 2 * head_dim] (cos
     then sin). The kernels index row `pos` of it for any pos < cache_len; a position at or
@@ -1073,7 +1079,7 @@ def _rmsnorm_launch(x, weight, eps, residual):
     dim = x.shape[-1]
     x2 = _bf16_2d(x, "x")
     r2 = _bf16_2d(residual, "residual") if residual is not None else None
-    w = weight.to(torch.bfloat16).contiguous()
+    w = _aligned(weight.to(torch.bfloat16).contiguous())
     out = torch.empty((x2.shape[0], dim), dtype=torch.bfloat16, device=dev)
     h = torch.empty_like(out) if residual is not None else None
     with _on(dev):
@@ -1216,12 +1222,17 @@ def kv_norm_rope_op(k: torch.Tensor, v: torch.Tensor, k_norm_w: torch.Tensor, ep
     if k2.shape != v2.shape or k2.shape[1] != nkv * hd or k_norm_w.shape != (hd,):
         raise ValueError(f"k {tuple(k2.shape)}, v {tuple(v2.shape)} and k_norm_w {tuple(k_norm_w.shape)} do not match "
                          f"{nkv} heads of {hd}")
-    kw = k_norm_w.to(torch.bfloat16).contiguous()
+    kw, table = _aligned(k_norm_w.to(torch.bfloat16).contiguous()), _aligned(rope)
+    kc, vc = _aligned(k_cache), _aligned(v_cache)
     with _on(dev):
         rc = _native.lib().wsl_kv_norm_rope_fwd(
             k2.data_ptr(), k2.stride(0), v2.data_ptr(), v2.stride(0), b, seq, nkv, hd, kw.data_ptr(), float(eps),
-            rope.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), L, _stream(dev))
+            table.data_ptr(), kc.data_ptr(), vc.data_ptr(), L, _stream(dev))
     _native.check(rc, "wsl_kv_norm_rope_fwd", decode=True)
+    if kc is not k_cache:
+        k_cache.copy_(kc)
+    if vc is not v_cache:
+        v_cache.copy_(vc)
 
 
 @kv_norm_rope_op.register_fake
@@ -1240,12 +1251,13 @@ def prefill_attention_op(q: torch.Tensor, q_norm_w: torch.Tensor, eps: float, ro
     seq = _check_prompt(q2.shape[0], k_cache, v_cache, rope)
     if q2.shape[1] != n_heads * hd or q_norm_w.shape != (hd,):
         raise ValueError(f"q {tuple(q2.shape)} and q_norm_w {tuple(q_norm_w.shape)} do not match {n_heads} heads of {hd}")
-    qw = q_norm_w.to(torch.bfloat16).contiguous()
+    qw, table = _aligned(q_norm_w.to(torch.bfloat16).contiguous()), _aligned(rope)
+    kc, vc = _aligned(k_cache), _aligned(v_cache)
     out = torch.empty((q2.shape[0], n_heads * hd), dtype=torch.bfloat16, device=dev)
     with _on(dev):
         rc = _native.lib().wsl_prefill_attention_fwd(
-            q2.data_ptr(), q2.stride(0), b, seq, n_heads, nkv, hd, qw.data_ptr(), float(eps), rope.data_ptr(),
-            k_cache.data_ptr(), v_cache.data_ptr(), L, float(scale), out.data_ptr(), out.stride(0), _stream(dev))
+            q2.data_ptr(), q2.stride(0), b, seq, n_heads, nkv, hd, qw.data_ptr(), float(eps), table.data_ptr(),
+            kc.data_ptr(), vc.data_ptr(), L, float(scale), out.data_ptr(), out.stride(0), _stream(dev))
     _native.check(rc, "wsl_prefill_attention_fwd", decode=True)
     return out
 

@@ -286,8 +286,7 @@ class SharedQwen3(nn.Module):
     def _prefill_fused_ok(self, tokens: torch.Tensor, cache: Optional[KVCache]) -> bool:
         """Whether this forward may take the fused prompt kernels: inference in bf16 on the GPU
         outside autocast, head sizes the attention kernel has, a contiguous cache that holds the
-        prompt, norm modules whose call is the kernels' arithmetic (the kernels do not call them), and
-        the 16-byte alignment of what the kernels read in place."""
+        prompt, and norm modules whose call is the kernels' arithmetic (the kernels do not call them)."""
         a = self.args
         if not self.prefill_fusion or torch.is_grad_enabled() or tokens.device.type != "cuda" \
                 or torch.is_autocast_enabled("cuda") or tokens.numel() == 0:
@@ -301,17 +300,7 @@ class SharedQwen3(nn.Module):
             if any(t.dtype != torch.bfloat16 or t.device != tokens.device or t.shape != shape or not t.is_contiguous()
                    for t in (cache.k, cache.v)) or s > cache.max_len:
                 return False
-        if not self._norms_plain() or any(p.dtype != torch.bfloat16 or p.device != tokens.device for p in self.parameters()):
-            return False
-        tracing = torch.compiler.is_compiling()  # no addresses then: storage counts as aligned
-        in_place = [m.weight for m in self._norms()] + [self.rope] + ([cache.k, cache.v] if cache is not None else [])
-        return all((t.storage_offset() * t.element_size() if tracing else t.data_ptr()) % 16 == 0 for t in in_place)
-
-    def _norms(self) -> list:
-        norms = [self.norm]
-        for blk in self.base_blocks:
-            norms += [blk.attention_norm, blk.ffn_norm, blk.attention.q_norm, blk.attention.k_norm]
-        return norms
+        return self._norms_plain() and all(p.dtype == torch.bfloat16 and p.device == tokens.device for p in self.parameters())
 
     def _norms_plain(self) -> bool:
         """Whether calling any norm of the model is RMSNorm.forward and nothing else: no other class
@@ -319,8 +308,11 @@ class SharedQwen3(nn.Module):
         every = torch.nn.modules.module
         if every._global_forward_hooks or every._global_forward_pre_hooks:
             return False
+        norms = [self.norm]
+        for blk in self.base_blocks:
+            norms += [blk.attention_norm, blk.ffn_norm, blk.attention.q_norm, blk.attention.k_norm]
         return all(type(m) is RMSNorm and "forward" not in m.__dict__ and not m._forward_hooks
-                   and not m._forward_pre_hooks for m in self._norms())
+                   and not m._forward_pre_hooks for m in norms)
 
     def _forward_fused(self, tokens: torch.Tensor, cache: Optional[KVCache], pk: Optional[dict]) -> torch.Tensor:
         """``forward`` with the prompt kernels of include/wsl_decode.h between the projections."""
