@@ -49,6 +49,62 @@ def test_tensors_off_the_gpu_and_subclasses_go_to_the_dispatcher(monkeypatch):
     assert ops.swiglu_op(gate_up=torch.zeros(2, 16, dtype=torch.bfloat16, device="meta")).shape == (2, 8)
 
 
+ALL_OPS = sorted(n for n in vars(ops) if n.endswith("_op") and not n.startswith("_"))
+
+
+@pytest.fixture(scope="module")
+def probe():
+    """An op made as the module's own are: a scaled copy, with a CUDA implementation and a gradient."""
+    def entry_probe(x: torch.Tensor, s: float, n: int, flag: bool, sizes: list[int]) -> torch.Tensor:
+        return x * s + n
+
+    op = ops._custom_op("entry_probe")(entry_probe)
+    op.register_fake(lambda x, s, n, flag, sizes: torch.empty_like(x))
+    op.register_autograd(lambda ctx, g: (g * ctx.s, None, None, None, None),
+                         setup_context=lambda ctx, inputs, output: setattr(ctx, "s", inputs[1]))
+    return op
+
+
+@pytest.mark.parametrize("name", ALL_OPS)
+def test_ops_are_custom_op_definitions(name):
+    """What torch.library takes and offers for a custom op it takes and offers for these."""
+    op = getattr(ops, name)
+    assert isinstance(op, torch.library.CustomOpDef)
+    for method in ("register_kernel", "register_fake", "register_vmap", "register_autograd", "register_autocast",
+                   "register_torch_dispatch", "set_kernel_enabled"):
+        assert callable(getattr(op, method))
+
+
+def test_torch_library_functions_take_the_ops(probe):
+    x = torch.arange(6.0)
+    torch.library.register_kernel(probe, "cpu", lambda x, s, n, flag, sizes: x * s + n)
+    assert probe._direct  # a CPU kernel leaves the CUDA one in its place
+    assert torch.equal(probe(x, 2.0, 1, False, [1]), 2 * x + 1)
+    torch.library.register_vmap(probe, lambda info, dims, x, *a: (probe(x, *a), dims[0]))
+    assert torch.equal(torch.func.vmap(lambda t: probe(t, 3.0, 0, True, [1, 2]))(x.view(2, 3)), 3 * x.view(2, 3))
+    y = x.clone().requires_grad_()
+    probe(y, 2.0, 1, False, []).sum().backward()
+    assert torch.equal(y.grad, torch.full_like(x, 2.0))
+    torch.library.opcheck(probe, (y, 2.0, 1, False, [1]))
+
+
+@pytest.mark.gpu
+def test_registered_kernels_and_formulas_have_the_last_word(gpu):
+    def entry_late(x: torch.Tensor, s: float) -> torch.Tensor:
+        return x * s
+
+    op = ops._custom_op("entry_late")(entry_late)
+    x = torch.ones(4, device=gpu, requires_grad=True)
+    assert torch.equal(op(x.detach(), 2.0), 2 * x)
+    op.register_autograd(lambda ctx, g: (ctx.saved_tensors[0] * g, None),  # a formula that keeps the output
+                         setup_context=lambda ctx, inputs, output: ctx.save_for_backward(output))
+    assert torch.equal(torch.autograd.grad(op(x, 3.0).sum(), x)[0], torch.full_like(x, 3.0))
+    torch.library.register_kernel(op, "cuda", lambda x, s: x * 0 - s)
+    assert torch.equal(op(x.detach(), 2.0), torch.full_like(x, -2.0))
+    assert torch.equal(torch.autograd.grad(op(x, 2.0).sum(), x)[0], torch.full_like(x, -2.0))
+    torch.library.opcheck(ops.swiglu_op, (torch.randn(3, 16, device=gpu).bfloat16(),))
+
+
 def _args(gpu, grad):
     g = torch.Generator(device="cuda").manual_seed(0)
     mk = lambda *s: torch.randn(*s, device=gpu, generator=g).bfloat16().requires_grad_(grad)  # noqa: E731

@@ -114,23 +114,24 @@ def _dispatcher_only() -> bool:
             or _transforms() is not None or _tracing() or _forward_ad._current_level >= 0 or _profiling())
 
 
-class _Op:
-    """A ``torch.library.custom_op`` named wsl::`name` over `fn` (called through torch.ops.wsl as
-    any other), with the direct routes above for its own callers."""
+class _Op(torch.library.CustomOpDef):
+    """A ``torch.library.custom_op`` named wsl::`name` over `fn`, with the direct routes above for its
+    own callers. It is the object that custom_op returned, as every torch function that takes one
+    expects; a CUDA kernel or a formula that a program registers on it later has the last word."""
 
-    def __init__(self, name: str, fn, mutates_args=()):
+    def _set_up(self, name: str, fn, mutates_args) -> None:
         self._fn = fn
-        self._def = torch.library.custom_op(f"wsl::{name}", fn, mutates_args=mutates_args, device_types="cuda")
         self._op = getattr(torch.ops.wsl, name).default
         params = list(inspect.signature(fn).parameters.values())
         self._tensors = tuple(i for i, q in enumerate(params) if q.annotation in ("torch.Tensor", "Optional[torch.Tensor]"))
         self._mutates = tuple(i for i, q in enumerate(params) if q.name in mutates_args)
         self._n = len(params)
         self._function = None
+        self._direct = True  # until another CUDA kernel takes the place of fn
         functools.update_wrapper(self, fn)
 
     def __call__(self, *args, **kwargs):
-        if _dispatcher_only() or kwargs or len(args) != self._n:
+        if _dispatcher_only() or not self._direct or kwargs or len(args) != self._n:
             return self._op(*args, **kwargs)
         recorded = False
         grad = _grad_on()
@@ -149,23 +150,33 @@ class _Op:
                 torch.autograd.graph.increment_version(args[i])
         return self._fn(*args)
 
-    def register_fake(self, fn):
-        return self._def.register_fake(fn)
+    def register_kernel(self, device_types, fn=None, /):
+        types = (device_types,) if isinstance(device_types, str) else device_types
+        if types is None or any(torch.device(d).type == "cuda" for d in types):
+            self._direct = False
+        return super().register_kernel(device_types, fn)
 
-    def register_autograd(self, backward, setup_context) -> None:
-        self._def.register_autograd(backward, setup_context=setup_context)
+    def register_autograd(self, backward, /, *, setup_context=None) -> None:
+        super().register_autograd(backward, setup_context=setup_context)
         impl = self._fn
 
         def forward(ctx, *args):
-            setup_context(ctx, args, None)
-            return impl(*args)
+            out = impl(*args)
+            if setup_context is not None:
+                setup_context(ctx, args, out)
+            return out
 
-        self._function = type(f"Wsl_{self._fn.__name__}", (torch.autograd.Function,),
+        self._function = type(f"Wsl_{impl.__name__}", (torch.autograd.Function,),
                               {"forward": staticmethod(forward), "backward": staticmethod(backward)})
 
 
 def _custom_op(name: str, mutates_args=()):
-    return lambda fn: _Op(name, fn, mutates_args)
+    def make(fn):
+        op = torch.library.custom_op(f"wsl::{name}", fn, mutates_args=mutates_args, device_types="cuda")
+        op.__class__ = _Op
+        op._set_up(name, fn, mutates_args)
+        return op
+    return make
 
 
 _NO_GUARD = contextlib.nullcontext()
