@@ -1,6 +1,8 @@
 """Calls of the ops go straight to their implementation only where nothing but the kernel has a
 part in them (ops._Op): every torch mechanism that must see a dispatched op still does, recorded
 calls have the gradients of the dispatched op, and mutated operands' versions count up."""
+from __future__ import annotations  # as in ops.py, whose op entry reads the parameters' declared types
+
 import pytest
 import torch
 from torch._subclasses.fake_tensor import FakeTensorMode
@@ -103,6 +105,48 @@ def test_registered_kernels_and_formulas_have_the_last_word(gpu):
     assert torch.equal(op(x.detach(), 2.0), torch.full_like(x, -2.0))
     assert torch.equal(torch.autograd.grad(op(x, 2.0).sum(), x)[0], torch.full_like(x, -2.0))
     torch.library.opcheck(ops.swiglu_op, (torch.randn(3, 16, device=gpu).bfloat16(),))
+
+
+@pytest.mark.parametrize("change", [{1: "2.0"}, {2: 1.5}, {2: None}, {4: [1.5]}, {4: 3}, {4: "1"}, {0: None}, {3: "yes"},
+                                    {1: torch.tensor(2.0)}, {2: True}, {3: 1}, {4: (1, 2)}, {4: [True]}, {1: True}])
+def test_arguments_off_the_schema_are_the_dispatchers(probe, monkeypatch, change):
+    """Only arguments of the declared types go straight to the implementation: the others are converted
+    or refused as in any call of a custom op."""
+    args = [torch.zeros(2), 2.0, 1, False, [1]]
+    for i, v in change.items():
+        args[i] = v
+    monkeypatch.setattr(probe, "_fn", lambda *a: pytest.fail("called directly"))
+    seen = []
+    monkeypatch.setattr(probe, "_op", lambda *a, **k: seen.append(a))
+    monkeypatch.setattr(ops, "_PLAIN_TYPES", (OnGpu, *ops._PLAIN_TYPES))
+    if args[0] is not None:
+        args[0] = OnGpu()
+    probe(*args)
+    assert len(seen) == 1
+    args = [OnGpu(), 2, 1, False, []]
+    monkeypatch.setattr(probe, "_fn", lambda *a: seen.append("direct"))
+    probe(*args)
+    assert seen[1:] == ["direct"]
+
+
+class OnGpu:
+    """Stands for a tensor on the GPU in the route's checks."""
+    is_cuda, requires_grad = True, False
+
+
+@pytest.mark.gpu
+def test_arguments_of_other_types_are_refused(gpu):
+    x, w, _, a, b = _args(gpu, False)
+    for op in (ops.lora_linear_op, torch.ops.wsl.lora_linear):
+        for args in ((x, w, None, a[:8], b, "2.0"), (None, w, None, a[:8], b, 2.0), (x, w, None, a[:8], 3.0, 2.0)):
+            with pytest.raises((RuntimeError, TypeError, AttributeError)):
+                op(*args)
+    for op in (ops.lora_linear_bcast_op, torch.ops.wsl.lora_linear_bcast):
+        with pytest.raises((RuntimeError, TypeError)):
+            op(x, w, None, a[:8], b, 2.0, 1.0, 1)
+    for op in (ops.lora_linear_grouped_op, torch.ops.wsl.lora_linear_grouped):
+        with pytest.raises((RuntimeError, TypeError)):
+            op(x, w, None, a, b, 2.0, [128.0, 128.0, 128.0])
 
 
 def _args(gpu, grad):

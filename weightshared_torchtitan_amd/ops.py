@@ -98,6 +98,8 @@ def _check_device(*ts: Optional[torch.Tensor]) -> torch.device:
 # as a torch.autograd.Function.
 # ------------------------------------------------------------------------------------------
 _PLAIN_TYPES = (torch.Tensor, torch.nn.Parameter)
+_TENSOR_KINDS = ("torch.Tensor", "Optional[torch.Tensor]")
+_SCALAR_KINDS = {"float": (float, int), "int": (int,), "bool": (bool,)}
 
 
 _is_compiling, _grad_on = torch.compiler.is_compiling, torch.is_grad_enabled
@@ -123,7 +125,12 @@ class _Op(torch.library.CustomOpDef):
         self._fn = fn
         self._op = getattr(torch.ops.wsl, name).default
         params = list(inspect.signature(fn).parameters.values())
-        self._tensors = tuple(i for i, q in enumerate(params) if q.annotation in ("torch.Tensor", "Optional[torch.Tensor]"))
+        kinds = [q.annotation for q in params]  # the text of the annotation
+        self._tensors = tuple((i, t != "torch.Tensor") for i, t in enumerate(kinds) if t in _TENSOR_KINDS)
+        self._scalars = tuple((i, _SCALAR_KINDS[t]) for i, t in enumerate(kinds) if t in _SCALAR_KINDS)
+        self._lists = tuple(i for i, t in enumerate(kinds) if t == "list[int]")
+        if len(self._tensors) + len(self._scalars) + len(self._lists) != len(kinds):
+            raise TypeError(f"wsl::{name}: a parameter of another kind in {kinds}")
         self._mutates = tuple(i for i, q in enumerate(params) if q.name in mutates_args)
         self._n = len(params)
         self._function = None
@@ -133,11 +140,17 @@ class _Op(torch.library.CustomOpDef):
     def __call__(self, *args, **kwargs):
         if _dispatcher_only() or not self._direct or kwargs or len(args) != self._n:
             return self._op(*args, **kwargs)
+        for i, types in self._scalars:  # anything else is the dispatcher's to convert or to refuse
+            if type(args[i]) not in types:
+                return self._op(*args)
+        for i in self._lists:
+            if type(args[i]) is not list or any(type(n) is not int for n in args[i]):
+                return self._op(*args)
         recorded = False
         grad = _grad_on()
-        for i in self._tensors:
+        for i, optional in self._tensors:
             t = args[i]
-            if t is None:
+            if t is None and optional:
                 continue
             if type(t) not in _PLAIN_TYPES or not t.is_cuda:
                 return self._op(*args)
