@@ -187,3 +187,20 @@ def test_chain_refuses_unsupported_stages(gpu):
     assert not ops.chain_supported(_chain_stages(t, outs), 32)
     with pytest.raises(ValueError):
         ops.lora_linear_chain(_chain_stages(t, outs), 32)
+
+
+def test_chain_status_of_a_device_without_index(gpu, wsl_opts):
+    """torch.device("cuda") is the current GPU: its workspace's failure word is read, and a stream without
+    chain launches has none."""
+    from weightshared_torchtitan_amd import ops
+    _say("[chain] status of torch.device('cuda')")
+    t = _layer(gpu, 8, seed=38)
+    stages = _chain_stages(t, _empty_outs(t, 8, gpu))
+    wsl_opts(decode_spin_limit=-1)
+    ops.lora_linear_chain(stages, 8)
+    torch.cuda.synchronize()
+    wsl_opts(decode_spin_limit=0)
+    with torch.cuda.stream(torch.cuda.Stream()):
+        assert not ops.chain_status(torch.device("cuda"))
+    assert ops.chain_status(torch.device("cuda"))
+    assert not ops.chain_status(torch.device("cuda")) and not ops.chain_status()

@@ -1539,7 +1539,8 @@ def lora_linear_chain(stages, M: int) -> None:
 def chain_status(dev: Optional[torch.device] = None) -> bool:
     """True when a chain launch on the current stream's workspace gave up a stage wait since
     the last call (the sticky failure word, then cleared); synchronizes the stream."""
-    dev = dev or torch.device("cuda", torch.cuda.current_device())
+    if dev is None or (dev.type == "cuda" and dev.index is None):
+        dev = torch.device("cuda", torch.cuda.current_device())
     stream = _stream(dev)
     ws = _workspaces.get((dev.index, stream, "chain"))
     if ws is None:
