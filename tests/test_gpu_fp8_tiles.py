@@ -1,7 +1,7 @@
-"""fp8 base weights decoded onto the bf16 matrix cores, on every tile the planner takes (128 x 128
-on the deep ring, split in K or not, and two to a CU; 128 x 256, 256 x 192, 256 x 256), with ragged
-M and N, T in the K loop and from the pre-pass, grouped and shared-base rows; and every code decodes
-exactly."""
+"""fp8 base weights decoded onto the bf16 matrix cores, on every tile the planner takes (two-buffer
+rings of 128 x 128, 128 x 256, 256 x 192 and 256 x 256 tiles, and the split-K form, whose deep ring
+holds the codes), with ragged M and N, T in the K loop and from the pre-pass, grouped and shared-base
+rows, splits from one K tile on; and every code decodes exactly, by either decoder."""
 import sys
 
 import pytest
@@ -31,13 +31,13 @@ def inputs(gpu, M, N, K, r, seed, groups=1):
 
 CASES = [
     # M, N, K, r, the planner's tile
-    (65, 512, 64, 0, (128, 128)),       # one K tile, deep ring
+    (65, 512, 64, 0, (128, 128)),       # one K tile
     (300, 1500, 128, 40, (128, 128)),   # two K tiles
     (70, 1000, 1088, 0, (128, 128)),    # 17 K tiles: no even split
-    (130, 1000, 256, 16, (128, 128)),   # as many K tiles as ring buffers, an N tail
+    (130, 1000, 256, 16, (128, 128)),   # an N tail
     (333, 1536, 320, 64, (128, 128)),   # two rank blocks
     (333, 6144, 448, 128, (128, 128)),  # T from the pre-pass
-    (2700, 2900, 128, 8, (128, 128)),   # more tiles than CUs: two-buffer ring
+    (2700, 2900, 128, 8, (128, 128)),   # more tiles than CUs
     (4096, 2048, 192, 32, (128, 256)),
     (3900, 2040, 448, 128, (128, 256)),
     (2700, 3072, 128, 16, (256, 192)),   # 768 chunks of codes a K tile for 512 threads
@@ -105,6 +105,26 @@ def test_fp8_splits_of_k(gpu, wsl_opts, M, N, K, r, splits):
     assert rel(ops.lora_linear_op(x, q, sc, a, b, 1.0), ref) <= TOL
 
 
+@pytest.mark.parametrize("r", [0, 32, 64, 128])
+@pytest.mark.parametrize("tiles", [1, 2, 3, 4, 5])
+def test_fp8_splits_of_few_k_tiles(gpu, wsl_opts, tiles, r):
+    """Two splits of as many K tiles as the deep ring's four buffers, of fewer and of one more: the ring's
+    start and end overlap."""
+    from weightshared_torchtitan_amd import ops
+    M, N, K = 130, 520, 128 * tiles
+    wsl_opts(prefill_split=2, fp8_prefill=1)
+    _say(f"[fp8 split-K] {tiles} K tiles a split, r={r}")
+    pl = ops.plan(M, K, r, [N], fp8=True)
+    assert pl["path"] == "prefill_splitk" and pl["k_splits"] == 2
+    x, q, sc, a, b = inputs(gpu, M, N, K, r, tiles + r)
+    y = ops.lora_linear_op(x, q, sc, a, b, 1.0)
+    ref = x.double() @ (q.double() * sc.double()[:, None]).t()
+    if r:
+        ref += (x.double() @ a.double().t()) @ b.double().t()
+    assert rel(y, ref) <= TOL
+    assert torch.equal(y, ops.lora_linear_op(x, q, sc, a, b, 1.0))
+
+
 @pytest.mark.parametrize("M,N,K,r", [(65, 512, 1024, 16), (100, 1000, 4096, 8), (333, 4096, 4096, 64),
                                      (200, 1024, 4096, 40)])
 def test_fp8_splits_keep_parts_of_t_that_cancel(gpu, wsl_opts, M, N, K, r):
@@ -160,18 +180,21 @@ def test_fp8_grouped_and_shared_base_rows(gpu, wsl_opts):
         assert rel(y[:, j * 256:(j + 1) * 256], ref) <= TOL
 
 
-@pytest.mark.parametrize("M", [80, 4096])
-def test_every_code_decodes_exactly(gpu, wsl_opts, M):
-    """Row n of W holds code n in column n % 128 alone: y picks it out."""
+@pytest.mark.parametrize("M,K,path", [(80, 128, "prefill"), (130, 128, "prefill"), (4096, 128, "prefill"),
+                                      (128, 1024, "prefill_splitk"), (130, 4096, "prefill_splitk")])
+def test_every_code_decodes_exactly(gpu, wsl_opts, M, K, path):
+    """Row n of W holds code n in column n % 128 of the last 128 alone, and x's row m a one in column
+    m % 128 of these: y picks the codes out (the first M of each half)."""
     from weightshared_torchtitan_amd import ops
     wsl_opts(fp8_prefill=1)
+    assert ops.plan(M, K, 0, [256], fp8=True)["path"] == path
     codes = torch.arange(256, dtype=torch.uint8, device=gpu)
-    W = torch.zeros(256, 128, dtype=torch.uint8, device=gpu)
-    W[torch.arange(256), torch.arange(256) % 128] = codes
+    W = torch.zeros(256, K, dtype=torch.uint8, device=gpu)
+    W[torch.arange(256), K - 128 + torch.arange(256) % 128] = codes
     W = W.view(torch.float8_e4m3fn)
-    x = torch.zeros(M, 128, device=gpu, dtype=torch.bfloat16)
+    x = torch.zeros(M, K, device=gpu, dtype=torch.bfloat16)
     m = torch.arange(M, device=gpu)
-    x[m, m % 128] = 1.0
+    x[m, K - 128 + m % 128] = 1.0
     y = ops.lora_linear_op(x, W, torch.ones(256, device=gpu), None, None, 0.0)
     want = codes.view(torch.float8_e4m3fn).float()
     for half in (0, 1):
