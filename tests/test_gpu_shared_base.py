@@ -57,22 +57,37 @@ def test_shared_base_once(gpu, M, N, K, r, base_n, g, G):
     assert torch.equal(y, ops.lora_linear_bcast_op(x, w, None, a, b, 2.0, g, G))
 
 
-def test_shared_base_rows_and_scratch(gpu):
-    """Output rows 8 bytes apart from 16-byte steps; the grouped query's smaller workspace."""
+def _call(x, w, a, b, y, M, N, K, r, base_n, g, G, ws, nbytes):
+    rc = _native.lib().wsl_lora_linear_bcast_fwd(
+        x.data_ptr(), K, w.data_ptr(), K, 0, None, a.data_ptr(), K, b.data_ptr(), r, ctypes.c_float(2.0),
+        y.data_ptr(), y.stride(0), M, N, K, r, base_n, g, G, ws.data_ptr(), nbytes, torch.cuda.current_stream().cuda_stream)
+    assert rc == _native.WSL_OK, _native.last_error()
+
+
+def test_shared_base_rows(gpu):
+    """Output rows 8 bytes apart from 16-byte steps, nothing written past them."""
     M, N, K, r, base_n, g, G = 4097, 1096, 1024, 16, 1096, 1, 3
-    print("[shared base] C entry", flush=True)
+    print("[shared base] C entry, rows off 16 bytes", flush=True)
     x, w, a, b, want, tol = _case(gpu, M, N, K, r, base_n, g, G, seed=3)
-    lib = _native.lib()
-    full = _native.bcast_workspace_bytes(M, N, K, r, G, 0)
-    for pad, nbytes in ((4, full), (0, 65536 + 2 * 256)):
-        y = torch.full((M, G * N + pad), 7.0, dtype=torch.bfloat16, device=gpu)
+    nbytes = _native.bcast_workspace_bytes(M, N, K, r, G, 0)
+    y = torch.full((M, G * N + 4), 7.0, dtype=torch.bfloat16, device=gpu)
+    _call(x, w, a, b, y, M, N, K, r, base_n, g, G, torch.zeros(nbytes, dtype=torch.uint8, device=gpu), nbytes)
+    _check(y[:, :G * N], want, tol)
+    assert bool((y[:, G * N:] == 7.0).all())
+
+
+@pytest.mark.parametrize("M,N,K,r,base_n,g,G", [(4200, 2176, 1024, 16, 1088, 2, 2), (8192, 4096, 1024, 32, 1024, 1, 1)])
+def test_shared_base_without_room_for_t(gpu, M, N, K, r, base_n, g, G):
+    """In the grouped query's workspace T of all groups does not fit (at G r <= 32 no other form wants it
+    there): the launch over the output columns runs, whose T stays in its tiles and leaves the scratch alone."""
+    print(f"[shared base] M={M} N={N} r={r} groups={G}: the grouped query's workspace", flush=True)
+    x, w, a, b, want, tol = _case(gpu, M, N, K, r, base_n, g, G, seed=M)
+    assert (G * N // base_n - 1) * M * base_n * K >= 1 << 33
+    full, small = _native.bcast_workspace_bytes(M, N, K, r, G, 0), _native.grouped_workspace_bytes(M, K, r, [N] * G, 0)
+    assert small < full
+    for nbytes, once in ((full, True), (small, False)):
+        y = torch.zeros(M, G * N, dtype=torch.bfloat16, device=gpu)
         ws = torch.zeros(full, dtype=torch.uint8, device=gpu)
-        rc = lib.wsl_lora_linear_bcast_fwd(
-            x.data_ptr(), K, w.data_ptr(), K, 0, None, a.data_ptr(), K, b.data_ptr(), r, ctypes.c_float(2.0),
-            y.data_ptr(), G * N + pad, M, N, K, r, base_n, g, G, ws.data_ptr(), nbytes,
-            torch.cuda.current_stream().cuda_stream)
-        if nbytes < full and rc == _native.WSL_E_WORKSPACE:
-            continue  # the form over the columns needs more than this as well
-        assert rc == _native.WSL_OK, _native.last_error()
-        _check(y[:, :G * N], want, tol)
-        assert pad == 0 or bool((y[:, G * N:] == 7.0).all())
+        _call(x, w, a, b, y, M, N, K, r, base_n, g, G, ws, nbytes)
+        _check(y, want, tol)
+        assert bool(ws[65536:].any()) is once
