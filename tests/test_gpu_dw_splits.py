@@ -17,6 +17,7 @@ pytestmark = pytest.mark.gpu
     (12001, 1088, 960, 0),   # 12 splits of 16 token tiles, the last short; 64 and 192 columns past whole tiles
     (3001, 1536, 1536, 8),   # 6 splits, whole tiles, rows in wider buffers
     (1601, 2112, 2112, 0),   # 3 splits, 64 columns past whole tiles both ways
+    (1001, 5120, 3328, 0),   # 260 large tiles, past one wave: product_splits' choice, 4 splits of 128 x 128 tiles
     (8192, 1024, 3072, 0),   # 5 splits of 26 token tiles, the last 24
 ])
 def test_dw_over_large_tile_splits(gpu, M, N, K, pad):

@@ -2107,8 +2107,9 @@ hipError_t launch_product(const LoraArgs& p, float* part, int splits) {
 // therefore pay for more splits, whose fp32 partials are written and read once (about 7 TB/s):
 // the cheaper of the two by these figures. dW with its reduce, 128 x 128 against 256 x 256:
 // 16384 tokens x 2048 x 2048 215 (unsplit) against 130 us (4 splits), 8192 x 1024 x 3072 77 (4)
-// against 68 (5), 4096 x 2048 x 2048 60 (unsplit) against 55 (4). Where the large tiles fill
-// the CUs alone (192 or more) the product is not split.
+// against 68 (5), 4096 x 2048 x 2048 60 (unsplit) against 55 (4). With 192 or more large tiles
+// product_splits' choice stands: the whole tokens on the tile launch_product_tn picks, or its
+// splits over 128 x 128 tiles.
 TnSplit product_tn_splits(int64_t M, int64_t N, int64_t nk) {
   const TnSplit small{product_splits(M, N, nk, false), false};
   const int64_t tb = ((M + 255) / 256) * ((N + 255) / 256), ts = ((M + 127) / 128) * ((N + 127) / 128);
