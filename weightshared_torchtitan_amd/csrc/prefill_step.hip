@@ -385,7 +385,12 @@ hipError_t launch_attention(const AttnArgs& a) {
 }
 
 // Heads per workgroup: as many of a kv head's group as divide it, up to the waves (they share
-// the K/V tiles). Two waves where four would leave CUs without a workgroup.
+// the K/V tiles): 8 x 512, 16 heads on 4 of 128: 25.6 / 25.7 / 26.5 us with 4 / 2 / 1 heads; 64
+// wide, 32 heads on 4: 23.2 / 23.2 / 24.1. Two waves where four would leave CUs without a
+// workgroup, below 1024 row blocks (graphs of 20, us, two waves against four, 16 heads on 8):
+// 1 x 64 7.9 / 9.4, 1 x 128 9.4 / 10.6, 1 x 256 12.6 / 13.3, even at 256 and 512 blocks (19.1 /
+// 18.8, 19.5 / 19.0), 768 22.0 / 19.4, 1024 22.5 / 20.1, 8 x 512 30.5 / 25.6: past 512 blocks the
+// line is late.
 template <int HD>
 hipError_t launch_attention_hd(const AttnArgs& a) {
   const int rep = a.nh / a.nkv;

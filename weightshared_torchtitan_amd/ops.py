@@ -559,7 +559,8 @@ def lora_linear_grouped_op(x: torch.Tensor, w: torch.Tensor, w_scale: Optional[t
     w [N, K] and b [N, r] stack the groups' rows (N = sum(group_n)); a [G*r, K] stacks
     their A factors (group g uses rows g*r..g*r+r-1). Output column block g is
     ``x . w_g^T (* w_scale_g) + scale * (x . a_g^T) . b_g^T``, the result of
-    ``lora_linear_op`` on that group alone.
+    ``lora_linear_op`` on that group alone (K may be summed in another order where the launch
+    splits it by its width: few row tiles, bf16 or fp8 w).
     """
     dev = _check_device(x, w, w_scale, a, b)
     K = x.shape[-1]
