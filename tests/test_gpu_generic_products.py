@@ -147,6 +147,18 @@ def test_infinities_stay_infinities_at_ranks_off_8(gpu, M, N, K, r):
         assert rel(y[ok], ref[ok]) <= TOL
 
 
+@pytest.mark.parametrize("N,K", [(100, 104), (128, 64), (64, 36)])
+@pytest.mark.parametrize("which", [2, 3])
+def test_input_gradient_refuses_factors_of_other_types(gpu, N, K, which):
+    """On every route: the generic products, the tiled kernel and the transposed copy."""
+    from weightshared_torchtitan_amd import ops
+    x, w, a, b, gy = inputs(gpu, 70, N, K, 8, 4)
+    args = [gy, w, None, a, b, 2.0]
+    args[1 + which] = args[1 + which].float()
+    with pytest.raises(TypeError):
+        ops.lora_linear_bwd_input_op(*args)
+
+
 def test_nan_stays_in_its_rows_and_columns(gpu):
     """A NaN or infinity of one row meets only that row's outputs, in products whose tiles are padded."""
     from weightshared_torchtitan_amd import ops

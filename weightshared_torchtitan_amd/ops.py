@@ -385,6 +385,8 @@ def lora_linear_bwd_input_op(gy: torch.Tensor, w: torch.Tensor, w_scale: Optiona
         r = a.shape[0]
         if a.shape[1] != K or b.shape != (N, r):
             raise ValueError(f"LoRA shapes a {tuple(a.shape)}, b {tuple(b.shape)} do not match K={K}, N={N}")
+        if a.dtype != torch.bfloat16 or b.dtype != torch.bfloat16:
+            raise TypeError("a and b must be bfloat16")
     dx = torch.empty((M, K), dtype=torch.bfloat16, device=dev)
     if M == 0:
         return dx
