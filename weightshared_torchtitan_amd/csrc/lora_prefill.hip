@@ -1137,74 +1137,81 @@ prefill_kernel(const uint16_t* __restrict__ x, int64_t ldx,
     char* sb = lora_b;                   // B chunk [BN n][64 ranks]
     // A split's part of T beside an fp8 W goes through B as three bf16 terms, whose 8 + 8 + 8 bits
     // are the fp32 value: parts rounded to bf16 would leave errors of their own size where they
-    // cancel, and the unsplit launch, which such a call took before, rounds only their sum.
+    // cancel, and the unsplit launch, which such a call took before, rounds only their sum. The
+    // second and third term take the two ring buffers that hold neither T's first nor B.
     constexpr int TTERMS = (RED && W8 && RB > 0) ? 3 : 1;
-#pragma unroll 1
-    for (int term = 0; term < TTERMS; ++term) {
-      if constexpr (RB > 0) {
-        if (t_wave && t_here) {
-          // park bf16(s * T): rows wm*TM + tj*32 + l32, ranks trb*32 + 8g + 4*lh + e. Ranks
-          // >= r (A rows past r were filled with row r-1) are zeroed here: they meet finite
-          // stand-in columns of B in the up-projection.
+    static_assert(TTERMS == 1 || C::NS == 4, "a ring buffer for each term of T and one for B");
+    auto t_area = [&](int term) { return term == 0 ? st : lds + ((nk + term) % C::NS) * STAGE; };
+    if constexpr (RB > 0) {
+      if (t_wave && t_here) {
+        // park bf16(s * T): rows wm*TM + tj*32 + l32, ranks trb*32 + 8g + 4*lh + e. Ranks
+        // >= r (A rows past r were filled with row r-1) are zeroed here: they meet finite
+        // stand-in columns of B in the up-projection.
 #pragma unroll
-          for (int q = 0; q < TPW; ++q) {
-            const int mrow = wm * C::TM + tj[q] * 32 + l32;
+        for (int q = 0; q < TPW; ++q) {
+          const int mrow = wm * C::TM + tj[q] * 32 + l32;
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
-              const int rk = trb[q] * 32 + g * 8 + lh * 4;
-              float t4[4];
+          for (int g = 0; g < 4; ++g) {
+            const int rk = trb[q] * 32 + g * 8 + lh * 4;
+            float t4[4];
 #pragma unroll
-              for (int e = 0; e < 4; ++e)
-                t4[e] = rk + e < r ? (term == 0 ? s : 1.f) * acct[q][g * 4 + e] : 0.f;
+            for (int e = 0; e < 4; ++e) t4[e] = rk + e < r ? s * acct[q][g * 4 + e] : 0.f;
+#pragma unroll
+            for (int term = 0; term < TTERMS; ++term) {
               uint2 v;
               v.x = pack_bf16x2(t4[0], t4[1]);
               v.y = pack_bf16x2(t4[2], t4[3]);
+              *reinterpret_cast<uint2*>(t_area(term) + t_off(mrow, trb[q] * 4 + g) + lh * 8) = v;
               if constexpr (TTERMS > 1) {  // what this term leaves over; nothing past an infinity or NaN
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                   const float h = bf16_bits_to_f32(((e < 2 ? v.x : v.y) >> ((e & 1) * 16)) & 0xffffu);
-                  acct[q][g * 4 + e] = fabsf(h) < INFINITY ? t4[e] - h : 0.f;
+                  t4[e] = fabsf(h) < INFINITY ? t4[e] - h : 0.f;
                 }
               }
-              *reinterpret_cast<uint2*>(st + t_off(mrow, trb[q] * 4 + g) + lh * 8) = v;
             }
           }
         }
       }
-      // RED with T from the pre-pass: the whole of T, so one split applies it
-      const int nrc = RED && EXT_T && blockIdx.y != 0 ? 0 : (r + 63) / 64;
-      for (int rc = 0; rc < nrc; ++rc) {
-        const int rk0 = rc * 64;
-        if (rc > 0) issue_b(sb, rk0);
-        if constexpr (EXT_T) {
-          constexpr int TCH = C::BM * 8 / NT;
+    }
+    // RED with T from the pre-pass: the whole of T, so one split applies it
+    const int nrc = RED && EXT_T && blockIdx.y != 0 ? 0 : (r + 63) / 64;
+    for (int rc = 0; rc < nrc; ++rc) {
+      const int rk0 = rc * 64;
+      if (rc > 0) issue_b(sb, rk0);
+      if constexpr (EXT_T) {
+        constexpr int TCH = C::BM * 8 / NT;
 #pragma unroll
-          for (int i = 0; i < TCH; ++i) {
-            const int id = i * NT + tid;
-            const int row = id >> 3, kr = rk0 + (id & 7) * 8;
-            const u32x4_t v = (kr < r) ? ld_global_16(tg + (int64_t)min(m0 + row, M - 1) * ldt + kr) : zero_u32x4();
-            lds_write16(st, lds_off(row, id & 7), v);
-          }
+        for (int i = 0; i < TCH; ++i) {
+          const int id = i * NT + tid;
+          const int row = id >> 3, kr = rk0 + (id & 7) * 8;
+          const u32x4_t v = (kr < r) ? ld_global_16(tg + (int64_t)min(m0 + row, M - 1) * ldt + kr) : zero_u32x4();
+          lds_write16(st, lds_off(row, id & 7), v);
         }
-        wait_vm0();
-        __syncthreads();
-        const int rem = r - rk0;
-        const int nkk = rem >= 64 ? 4 : (rem + 15) / 16;
-        for (int kk = 0; kk < nkk; ++kk) {
-          const int c = kk * 2 + lh;
-          bf16x8_t tf[C::MJ], bf[C::NI];
+      }
+      wait_vm0();
+      __syncthreads();
+      const int rem = r - rk0;
+      const int nkk = rem >= 64 ? 4 : (rem + 15) / 16;
+      for (int kk = 0; kk < nkk; ++kk) {
+        const int c = kk * 2 + lh;
+        bf16x8_t tf[TTERMS][C::MJ], bf[C::NI];
 #pragma unroll
-          for (int j = 0; j < C::MJ; ++j) tf[j] = as_bf16x8(lds_read16(st, t_off(wm * C::TM + j * 32 + l32, c)));
+        for (int term = 0; term < TTERMS; ++term)
 #pragma unroll
-          for (int i = 0; i < C::NI; ++i) bf[i] = as_bf16x8(lds_read16(sb, lds_off(wn * C::TN + i * 32 + l32, c)));
+          for (int j = 0; j < C::MJ; ++j)
+            tf[term][j] = as_bf16x8(lds_read16(t_area(term), t_off(wm * C::TM + j * 32 + l32, c)));
+#pragma unroll
+        for (int i = 0; i < C::NI; ++i) bf[i] = as_bf16x8(lds_read16(sb, lds_off(wn * C::TN + i * 32 + l32, c)));
+#pragma unroll
+        for (int term = 0; term < TTERMS; ++term)
 #pragma unroll
           for (int i = 0; i < C::NI; ++i)
 #pragma unroll
             for (int j = 0; j < C::MJ; ++j)
-              acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bf[i], tf[j], acc[i][j], 0, 0, 0);
-        }
-        __syncthreads();
+              acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bf[i], tf[term][j], acc[i][j], 0, 0, 0);
       }
+      __syncthreads();
     }
   }
 
@@ -1855,10 +1862,10 @@ int red_splits(int64_t M, int64_t N, int64_t K, int w_dtype, bool has_w, bool ga
 }
 
 // An fp8 W (8B shapes, graphs of 20 launches, us, the unsplit launch before): 80 x 4096 x 12288
-// 139.7 -> 39.4 at r = 16, 147.1 -> 49.1 at r = 128 (pre-pass included); 333 x 4096 x 4096 51.9 ->
-// 37.4 and 62.2 -> 47.1; 600 x 1024 x 4096 51.7 -> 26.0; 80 x 12288 x 4096 50.2 -> 36.1. T's parts
-// as three bf16 terms are 0.7-1.2 us of these at ranks 8-16, 1.5-2.2 at rank 64 (against one term
-// each, 38.5 -> 39.4 and 41.8 -> 44.0 at 80 x 4096 x 12288; the distance from 64-bit results
+// 139.7 -> 39.3 at r = 16, 147.1 -> 49.1 at r = 128 (pre-pass included); 333 x 4096 x 4096 51.9 ->
+// 37.4 and 62.2 -> 47.1; 600 x 1024 x 4096 51.7 -> 25.6; 80 x 12288 x 4096 50.2 -> 36.5. T's parts
+// as three bf16 terms are 0.6-0.9 us of these at ranks 8-16 and 0.7-1.5 at rank 64 (against one
+// term, 38.6 -> 39.3 and 41.9 -> 43.3 at 80 x 4096 x 12288; the distance from 64-bit results
 // 1.685e-3 -> 1.664e-3 at rank 64, random inputs). The splits
 // run on the deep ring, W's codes in the ring and each K tile decoded once (W8R). Unsplit
 // launches stay on the two-buffer ring: their loop is bound by the LDS (the decode's reads and
