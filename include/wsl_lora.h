@@ -44,10 +44,16 @@ extern "C" {
  *   WSL_DTYPE_FP8_E4M3_ACT8  the same weight, with the prefill product on one e4m3 term per
  *                            activation: half the matrix-core work, plus e4m3 rounding of x
  *                            (about 3.7e-2 against an fp32-W reference at config-5 shapes,
- *                            against 2.4-2.6e-2 for WSL_DTYPE_FP8_E4M3). Decode shapes as above. */
+ *                            against 2.4-2.6e-2 for WSL_DTYPE_FP8_E4M3). Decode shapes as above.
+ *   WSL_DTYPE_T_WHOLE        or'ed to one of these in a forward call: where a launch splits K, the
+ *                            splits' parts of T = scale * x . A^T go through B in fp32 (three bf16
+ *                            terms), so that parts which cancel leave no error of their own size;
+ *                            about 1 us. A bf16 W's parts are each rounded to bf16 without it, an
+ *                            fp8 W's never. */
 #define WSL_DTYPE_BF16 0
 #define WSL_DTYPE_FP8_E4M3 1
 #define WSL_DTYPE_FP8_E4M3_ACT8 2
+#define WSL_DTYPE_T_WHOLE 256
 
 /* Largest LoRA rank the kernels accept. */
 #define WSL_MAX_RANK 256
@@ -86,7 +92,8 @@ int wsl_lora_linear_workspace_bytes(int64_t M, int64_t N, int64_t K, int64_t r,
  *            r = 0 (a, b ignored) gives the plain linear.
  *   scale    LoRA scale s = alpha / rank (2.0 under the reference's alpha = 2*rank).
  *   y        [M,N] bf16 output, row stride ldy. Must not alias any input.
- *   Accumulation is fp32. x . A^T is rounded once to bf16 after scaling by s.
+ *   Accumulation is fp32. x . A^T is rounded once to bf16 after scaling by s (where a launch splits
+ *   K, as WSL_DTYPE_T_WHOLE says).
  *   M may be 0 (no work). K >= 1, N >= 1, 0 <= r <= WSL_MAX_RANK.
  */
 int wsl_lora_linear_fwd(const void* x, int64_t ldx,

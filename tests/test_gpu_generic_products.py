@@ -147,6 +147,39 @@ def test_infinities_stay_infinities_at_ranks_off_8(gpu, M, N, K, r):
         assert rel(y[ok], ref[ok]) <= TOL
 
 
+@pytest.mark.parametrize("form", ["linear", "grouped", "shared base"])
+@pytest.mark.parametrize("M,N,K,r", [(65, 512, 1024, 4), (200, 1024, 4096, 12), (333, 2048, 4096, 63)])
+def test_ranks_off_8_keep_parts_of_t_that_cancel(gpu, M, N, K, r, form):
+    """T = x . A^T whose halves of K, in different splits of the launch, nearly cancel. The operands are
+    small multiples of powers of two, so every sum is exact in fp32 in any order, and the error is T's
+    rounding (at most one, u = 2^-8 of |T|) and y's: u |y| + u (1 + u) sum |T| |B|."""
+    from weightshared_torchtitan_amd import ops
+    _say(f"[rank off 8, cancelling T] M={M} N={N} K={K} r={r} {form}")
+    G = 1 if form == "linear" else 2
+    pl = ops.plan(M, K, (r + 7) // 8 * 8, [N] * G)
+    assert pl["path"] == "prefill_splitk" and pl["k_splits"] % 2 == 0 and not pl["rank_prepass"]
+    g = torch.Generator(device="cuda").manual_seed(r)
+    ints = lambda n, *s: torch.randint(-n, n + 1, s, device=gpu, generator=g)  # noqa: E731
+    v, e = ints(16, M, K // 2), ints(1, M, K // 2) * (ints(8, M, K // 2) == 0)
+    x = (torch.cat([v, e - v], 1) / 8).bfloat16()
+    a = (ints(16, G * r, K // 2) / 64).repeat(1, 2).bfloat16()
+    b = (ints(16, G * N, r) / 64).bfloat16()
+    w = torch.zeros(N if form == "shared base" else G * N, K, device=gpu).bfloat16()
+    if form == "linear":
+        y = ops.lora_linear_op(x, w, None, a, b, 2.0)
+    elif form == "grouped":
+        y = ops.lora_linear_grouped_op(x, w, None, a, b, 2.0, [N, N])
+    else:
+        y = ops.lora_linear_bcast_op(x, w, None, a, b, 2.0, 1, 2)
+    u = 2.0 ** -8
+    for j in range(G):
+        t, bj = 2.0 * x.double() @ a[j * r:(j + 1) * r].double().t(), b[j * N:(j + 1) * N].double()
+        want = t @ bj.t()
+        tol = u * want.abs() + u * (1 + u) * t.abs() @ bj.abs().t()
+        err = (y[:, j * N:(j + 1) * N].double() - want).abs()
+        assert bool((err <= tol).all()), float((err / tol.clamp_min(1e-30)).max())
+
+
 @pytest.mark.parametrize("N,K", [(100, 104), (128, 64), (64, 36)])
 @pytest.mark.parametrize("which", [2, 3])
 def test_input_gradient_refuses_factors_of_other_types(gpu, N, K, which):

@@ -1135,12 +1135,14 @@ prefill_kernel(const uint16_t* __restrict__ x, int64_t ldx,
   if constexpr (LORA) {
     char* st = PER ? lds + C::NS * STAGE : lora_t;  // T chunk [BM m][64 ranks] (the T region with PER)
     char* sb = lora_b;                   // B chunk [BN n][64 ranks]
-    // A split's part of T beside an fp8 W goes through B as three bf16 terms, whose 8 + 8 + 8 bits
-    // are the fp32 value: parts rounded to bf16 would leave errors of their own size where they
-    // cancel, and the unsplit launch, which such a call took before, rounds only their sum. The
-    // second and third term take the two ring buffers that hold neither T's first nor B.
-    constexpr int TTERMS = (RED && W8 && RB > 0) ? 3 : 1;
-    static_assert(TTERMS == 1 || C::NS == 4, "a ring buffer for each term of T and one for B");
+    // A split's part of T can go through B as three bf16 terms, whose 8 + 8 + 8 bits are the fp32
+    // value: parts rounded to bf16 leave errors of their own size where they cancel. Always beside
+    // an fp8 W and where the call asks for it (skt_spin, free here, holds the number of terms):
+    // calls whose T was summed whole in fp32 before they were split. The second and third term
+    // take the two ring buffers that hold neither T's first nor B.
+    constexpr int TMAX = (RED && RB > 0) ? 3 : 1;
+    static_assert(TMAX == 1 || C::NS == 4, "a ring buffer for each term of T and one for B");
+    const int tterms = TMAX == 1 ? 1 : W8 ? TMAX : skt_spin;
     auto t_area = [&](int term) { return term == 0 ? st : lds + ((nk + term) % C::NS) * STAGE; };
     if constexpr (RB > 0) {
       if (t_wave && t_here) {
@@ -1148,25 +1150,27 @@ prefill_kernel(const uint16_t* __restrict__ x, int64_t ldx,
         // >= r (A rows past r were filled with row r-1) are zeroed here: they meet finite
         // stand-in columns of B in the up-projection.
 #pragma unroll
-        for (int q = 0; q < TPW; ++q) {
-          const int mrow = wm * C::TM + tj[q] * 32 + l32;
+        for (int term = 0; term < TMAX; ++term) {
+          if (term > 0 && term >= tterms) break;
 #pragma unroll
-          for (int g = 0; g < 4; ++g) {
-            const int rk = trb[q] * 32 + g * 8 + lh * 4;
-            float t4[4];
+          for (int q = 0; q < TPW; ++q) {
+            const int mrow = wm * C::TM + tj[q] * 32 + l32;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) t4[e] = rk + e < r ? s * acct[q][g * 4 + e] : 0.f;
+            for (int g = 0; g < 4; ++g) {
+              const int rk = trb[q] * 32 + g * 8 + lh * 4;
+              float t4[4];
 #pragma unroll
-            for (int term = 0; term < TTERMS; ++term) {
+              for (int e = 0; e < 4; ++e)
+                t4[e] = term > 0 ? acct[q][g * 4 + e] : rk + e < r ? s * acct[q][g * 4 + e] : 0.f;
               uint2 v;
               v.x = pack_bf16x2(t4[0], t4[1]);
               v.y = pack_bf16x2(t4[2], t4[3]);
               *reinterpret_cast<uint2*>(t_area(term) + t_off(mrow, trb[q] * 4 + g) + lh * 8) = v;
-              if constexpr (TTERMS > 1) {  // what this term leaves over; nothing past an infinity or NaN
+              if (term + 1 < TMAX) {  // what this term leaves over; nothing past an infinity or NaN
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                   const float h = bf16_bits_to_f32(((e < 2 ? v.x : v.y) >> ((e & 1) * 16)) & 0xffffu);
-                  t4[e] = fabsf(h) < INFINITY ? t4[e] - h : 0.f;
+                  acct[q][g * 4 + e] = fabsf(h) < INFINITY ? t4[e] - h : 0.f;
                 }
               }
             }
@@ -1195,21 +1199,21 @@ prefill_kernel(const uint16_t* __restrict__ x, int64_t ldx,
       const int nkk = rem >= 64 ? 4 : (rem + 15) / 16;
       for (int kk = 0; kk < nkk; ++kk) {
         const int c = kk * 2 + lh;
-        bf16x8_t tf[TTERMS][C::MJ], bf[C::NI];
-#pragma unroll
-        for (int term = 0; term < TTERMS; ++term)
-#pragma unroll
-          for (int j = 0; j < C::MJ; ++j)
-            tf[term][j] = as_bf16x8(lds_read16(t_area(term), t_off(wm * C::TM + j * 32 + l32, c)));
+        bf16x8_t bf[C::NI];
 #pragma unroll
         for (int i = 0; i < C::NI; ++i) bf[i] = as_bf16x8(lds_read16(sb, lds_off(wn * C::TN + i * 32 + l32, c)));
 #pragma unroll
-        for (int term = 0; term < TTERMS; ++term)
+        for (int term = 0; term < TMAX; ++term) {
+          if (term > 0 && term >= tterms) break;
+          bf16x8_t tf[C::MJ];
+#pragma unroll
+          for (int j = 0; j < C::MJ; ++j) tf[j] = as_bf16x8(lds_read16(t_area(term), t_off(wm * C::TM + j * 32 + l32, c)));
 #pragma unroll
           for (int i = 0; i < C::NI; ++i)
 #pragma unroll
             for (int j = 0; j < C::MJ; ++j)
-              acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bf[i], tf[term][j], acc[i][j], 0, 0, 0);
+              acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bf[i], tf[j], acc[i][j], 0, 0, 0);
+        }
       }
       __syncthreads();
     }
@@ -1903,9 +1907,11 @@ hipError_t launch_red(const LoraArgs& p, int splits) {
     if (p.r <= 32) return launch_cfg<CfgDeep, kFP8, true, 1, false, false, false, false, true>(q, nullptr, 0, splits, part, p.red_cnt);
     return launch_cfg<CfgDeep, kFP8, true, 2, false, false, false, false, true>(q, nullptr, 0, splits, part, p.red_cnt);
   }
+  const int terms = p.t_whole ? 3 : 1;
   if (p.r == 0) return launch_cfg<CfgDeep, kBF16, true, 0, false, false, false, false, true>(q, nullptr, 0, splits, part, p.red_cnt);
-  if (p.r <= 32) return launch_cfg<CfgDeep, kBF16, true, 1, false, false, false, false, true>(q, nullptr, 0, splits, part, p.red_cnt);
-  return launch_cfg<CfgDeep, kBF16, true, 2, false, false, false, false, true>(q, nullptr, 0, splits, part, p.red_cnt);
+  if (p.r <= 32)
+    return launch_cfg<CfgDeep, kBF16, true, 1, false, false, false, false, true>(q, nullptr, 0, splits, part, p.red_cnt, 1, terms);
+  return launch_cfg<CfgDeep, kBF16, true, 2, false, false, false, false, true>(q, nullptr, 0, splits, part, p.red_cnt, 1, terms);
 }
 
 // y[m][n] = bf16(sum_s part[s][m][n] + sum_j T[m][goff(n) + j] B[n][j]): the partials in split

@@ -157,14 +157,17 @@ size_t workspace_upper_bound(int64_t M, int64_t N, int64_t K, int64_t r, int w_d
 
 // The storage type the kernels see and the fp8 activation terms of a public w_dtype code:
 // WSL_DTYPE_FP8_E4M3_ACT8 is an fp8 W whose prefill product takes one activation term.
+// WSL_DTYPE_T_WHOLE (read by t_whole) is no part of it.
 int32_t kernel_dtype(int32_t w_dtype, int* terms) {
   *terms = 2;
+  w_dtype &= ~WSL_DTYPE_T_WHOLE;
   if (w_dtype == WSL_DTYPE_FP8_E4M3_ACT8) {
     *terms = 1;
     return WSL_DTYPE_FP8_E4M3;
   }
   return w_dtype;
 }
+bool t_whole(int32_t w_dtype) { return (w_dtype & WSL_DTYPE_T_WHOLE) != 0; }
 
 int validate_sizes(int64_t M, int64_t N, int64_t K, int64_t r, int32_t w_dtype) {
   if (M < 0) return fail(WSL_E_SHAPE, "M must be >= 0 (got %lld)", (long long)M);
@@ -458,6 +461,7 @@ int wsl_lora_linear_fwd(const void* x, int64_t ldx, const void* w, int64_t ldw, 
   if (rc != WSL_OK) return rc;
   wsl::LoraArgs p = make_args(x, ldx, w, ldw, w_dtype, w_scale, a, lda, b, ldb, scale, y, ldy, M, N, K, r, stream);
   p.fp8_terms = terms;
+  p.t_whole = t_whole(w_dtype_in);
   return run_call(p, workspace, workspace_bytes);
 }
 
@@ -473,6 +477,7 @@ int wsl_lora_linear_fwd_noalloc(const void* x, int64_t ldx, const void* w, int64
   wsl::LoraArgs p = make_args(x, ldx, w, ldw, w_dtype, w_scale, a, lda, b, ldb, scale, y, ldy, M, N, K, r,
                               stream);
   p.fp8_terms = terms;
+  p.t_whole = t_whole(w_dtype_in);
   if (choose_path(p) == Path::kNone) return WSL_OK;
   // the exact need of the path this call takes (sizes and alignment are known here)
   size_t need;
@@ -532,6 +537,7 @@ int wsl_lora_linear_grouped_fwd(const void* x, int64_t ldx, const void* w, int64
   if (rc != WSL_OK) return rc;
   wsl::LoraArgs p = make_args(x, ldx, w, ldw, w_dtype, w_scale, a, lda, b, ldb, scale, y, ldy, M, N, K, r, stream);
   p.fp8_terms = terms;
+  p.t_whole = t_whole(w_dtype_in);
   return run_grouped(p, n_groups, group_n, false, workspace, workspace_bytes);
 }
 
@@ -569,6 +575,7 @@ int wsl_lora_linear_bcast_fwd(const void* x, int64_t ldx, const void* w, int64_t
   if (rc != WSL_OK) return rc;
   wsl::LoraArgs p = make_args(x, ldx, w, ldw, w_dtype, w_scale, a, lda, b, ldb, scale, y, ldy, M, Nt, K, r, stream);
   p.fp8_terms = terms;
+  p.t_whole = t_whole(w_dtype_in);
   // column c of a group reads base row (c / (hpg D')) D' + c % D': the reference's
   // broadcast_add index map (D' = base_n / g templates' width, hpg = N / base_n heads each)
   const int64_t dw = base_n / g, hpg = N / base_n;

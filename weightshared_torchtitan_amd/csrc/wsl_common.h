@@ -138,6 +138,8 @@ struct LoraArgs {
   // fp8 W on prefill shapes: activation terms of the fp8 matrix-core path (2: bf16-quality
   // activations, 1: one e4m3 term); 0 decodes W to bf16 on the bf16 matrix cores instead.
   int fp8_terms = 2;
+  // WSL_DTYPE_T_WHOLE: parts of T of a launch that splits K go through B unrounded.
+  bool t_whole = false;
   // Shared-base forms: W (and w_scale) rows by output column, and W's row count.
   RowMap wmap;
   int64_t wrows = 0;

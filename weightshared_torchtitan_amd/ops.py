@@ -254,7 +254,8 @@ def _rows16(t: torch.Tensor) -> bool:
 def _pads_rank(r: int, x: torch.Tensor, K: int) -> bool:
     """Whether LoRA factors of rank r on x [M, K] go padded to a multiple of 8: where the tiled
     kernels then take the call (its reduction on their grid, its rows aligned), and below 8, where
-    the generic products would load the factors' short rows one element at a time."""
+    the generic products would load the factors' short rows one element at a time. Such a call keeps
+    T whole (WSL_DTYPE_T_WHOLE): the products it would otherwise take do not split K."""
     return r % 8 != 0 and (r < 8 or (K % 64 == 0 and _rows16(x)))
 
 
@@ -327,6 +328,7 @@ def lora_linear_op(x: torch.Tensor, w: Optional[torch.Tensor], w_scale: Optional
     if M > 0:
         if _pads_rank(r, x2, K):
             a, b, r = _pad_rank(a, b, 1)
+            w_dtype |= _native.WSL_DTYPE_T_WHOLE
         ws_bytes = _native.workspace_bytes(M, N, K, r, w_dtype)
         stream = _stream(dev)
         ws = workspace(dev, stream, ws_bytes)
@@ -604,6 +606,7 @@ def lora_linear_grouped_op(x: torch.Tensor, w: torch.Tensor, w_scale: Optional[t
     if M > 0:
         if _pads_rank(r, x2, K):
             a, b, r = _pad_rank(a, b, G)
+            w_dtype |= _native.WSL_DTYPE_T_WHOLE
         gn = _native.group_array(group_n)
         ws_bytes = _native.grouped_workspace_bytes(M, K, r, group_n, w_dtype)
         stream = _stream(dev)
@@ -680,6 +683,7 @@ def lora_linear_bcast_op(x: torch.Tensor, w: torch.Tensor, w_scale: Optional[tor
     if M > 0:
         if _pads_rank(r, x2, K):
             a, b, r = _pad_rank(a, b, G)
+            w_dtype |= _native.WSL_DTYPE_T_WHOLE
         stream = _stream(dev)
         ws = workspace(dev, stream, _native.bcast_workspace_bytes(M, N, K, r, G, w_dtype))
         with _on(dev):
