@@ -40,6 +40,20 @@ def test_mechanisms_that_need_the_dispatcher_are_seen():
     torch.func.grad(lambda t: (seen.append(ops._dispatcher_only()), t.sum())[1])(torch.zeros(2))
     torch.jit.trace(lambda t: (seen.append(ops._dispatcher_only()), t + 1)[1], torch.zeros(2), check_trace=False)
     assert seen == [True] * 3
+
+    class Seer(torch.autograd.Function):
+        @staticmethod
+        def forward(ctx, t):
+            return t * 2
+
+        @staticmethod
+        def backward(ctx, g):
+            seen.append(ops._dispatcher_only())
+            return g * 2
+
+    x = torch.zeros(2, requires_grad=True)
+    torch.autograd.grad(Seer.apply(x), x, torch.eye(2), is_grads_batched=True)
+    assert seen == [True] * 4
     assert not ops._dispatcher_only()
 
 
@@ -201,6 +215,21 @@ def test_transforms_see_the_op(gpu):
             except (RuntimeError, NotImplementedError):
                 out.append("raised")
         assert out[0] == out[1]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,tail", [("lora_linear", (2.0,)), ("lora_linear_bcast", (2.0, 1, 1))])
+def test_batches_of_gradients(gpu, name, tail):
+    """torch.autograd.grad over a batch of output gradients, one backward each (the grouped op's backward
+    writes slices in place, which the batching does not take)."""
+    x, w, _, a, b = _args(gpu, True)
+    a = a[:8].detach().requires_grad_()
+    y = getattr(ops, name + "_op")(x, w, None, a, b, *tail)
+    gy = torch.randn(3, 2, 50, 384, device=gpu).bfloat16()
+    got = torch.autograd.grad(y, [x, w, a, b], gy, is_grads_batched=True, retain_graph=True)
+    for i in range(3):
+        for g, want in zip(got, torch.autograd.grad(y, [x, w, a, b], gy[i], retain_graph=True)):
+            assert torch.equal(g[i], want)
 
 
 @pytest.mark.gpu

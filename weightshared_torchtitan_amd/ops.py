@@ -107,13 +107,16 @@ _dispatch_modes, _function_modes = torch._C._len_torch_dispatch_stack, torch._C.
 _transforms, _tracing = torch._C._functorch.peek_interpreter_stack, torch._C._is_tracing
 _autocast, _profiling = torch._C._is_any_autocast_enabled, torch._C._autograd._profiler_enabled
 _forward_ad = torch.autograd.forward_ad
+_tls_key, _vmap_mode = torch._C._dispatch_tls_is_dispatch_key_included, torch._C._parse_dispatch_key("VmapMode")
 
 
 def _dispatcher_only() -> bool:
     """Whether something in force must see calls as dispatched ops: tracing and compilation, torch
-    modes, functorch transforms, autocast, forward-mode AD, a profiler."""
+    modes, functorch transforms, batches of gradients (is_grads_batched: a vmap of its own), autocast,
+    forward-mode AD, a profiler."""
     return (_is_compiling() or _dispatch_modes() != 0 or _function_modes() != 0 or _autocast()
-            or _transforms() is not None or _tracing() or _forward_ad._current_level >= 0 or _profiling())
+            or _transforms() is not None or _tls_key(_vmap_mode) or _tracing() or _forward_ad._current_level >= 0
+            or _profiling())
 
 
 class _Op(torch.library.CustomOpDef):
