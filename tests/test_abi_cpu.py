@@ -78,6 +78,19 @@ def test_workspace_query_rejects_bad_sizes(M, Nn, K, r, dt, code):
 
 
 @needs_lib
+@pytest.mark.parametrize("dt", [N.WSL_DTYPE_BF16, N.WSL_DTYPE_FP8_E4M3, N.WSL_DTYPE_FP8_E4M3_ACT8])
+def test_whole_t_flag_is_no_type_of_its_own(dt):
+    assert _header_defines()["WSL_DTYPE_T_WHOLE"] == N.WSL_DTYPE_T_WHOLE
+    flag = dt | N.WSL_DTYPE_T_WHOLE
+    for M in (4, 200, 4096):
+        assert N.workspace_bytes(M, 1024, 4096, 16, flag) == N.workspace_bytes(M, 1024, 4096, 16, dt)
+        assert N.plan(M, 4096, 16, [512, 512], flag) == N.plan(M, 4096, 16, [512, 512], dt)
+        assert N.bcast_workspace_bytes(M, 1024, 4096, 16, 2, flag) == N.bcast_workspace_bytes(M, 1024, 4096, 16, 2, dt)
+    sz = ctypes.c_size_t()
+    assert N.lib().wsl_lora_linear_workspace_bytes(4, 64, 64, 8, 7 | flag, ctypes.byref(sz)) == N.WSL_E_DTYPE
+
+
+@needs_lib
 def test_workspace_query_null_out_pointer():
     assert N.lib().wsl_lora_linear_workspace_bytes(4, 64, 64, 8, 0, None) == N.WSL_E_INVALID_ARG
 
