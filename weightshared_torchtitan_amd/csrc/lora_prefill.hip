@@ -205,11 +205,12 @@ __device__ __forceinline__ void for_ct(F&& f) {
 //
 // RED: split-K fused LoRA linear with the reduction in the launch. Workgroup row
 // blockIdx.y takes the K range [blockIdx.y * K, (blockIdx.y + 1) * K) of x, W and A (K is
-// one split's length); every split writes its fp32 base and T partials to red_part in its
-// accumulators' own lane order, and the split that arrives last at the tile's counter
-// (red_cnt[blockIdx.x], left at zero again) sums all of them in split order and finishes
-// the tile (T, the up-projection, the store) as an unsplit launch would. The sum does not
-// depend on which split arrives last, so the result is repeatable bit for bit.
+// one split's length); every split applies its part of T through B (rounded to bf16, or with
+// an fp8 W or TWHOLE as it is; T from the pre-pass is split 0's to apply) and writes its fp32
+// output partial to red_part in its accumulators' own lane order, and the split that arrives
+// last at the tile's counter (red_cnt[blockIdx.x], left at zero again) sums all of them in
+// split order and stores the tile. The sum does not depend on which split arrives last, so the
+// result is repeatable bit for bit.
 //
 // TN: plain GEMM over operands stored with the reduction as rows ("token-major"): x'[m][k] is
 // x[k * ldx + m] and W'[n][k] is w[k * ldw + n], as the weight gradients' dY and x are (a
@@ -249,7 +250,7 @@ __device__ __forceinline__ void for_ct(F&& f) {
 // columns that read these base rows (the inverse of wmap: base row n of a template D wide is column
 // j P + (n / D) S + h D + n % D). r % 16 == 0, D % 8 == 0.
 template <class C, int WDT, bool HAS_W, int RB, bool EXT_T, bool GATHER, bool SPLIT = false, bool TN = false,
-          bool RED = false, bool PER = false, bool WT = false, bool SKT = false, bool SHARE = false>
+          bool RED = false, bool PER = false, bool WT = false, bool SKT = false, bool SHARE = false, bool TWHOLE = false>
 __global__ void __launch_bounds__(C::NT, 1)
 prefill_kernel(const uint16_t* __restrict__ x, int64_t ldx,
                const int64_t* __restrict__ gidx, int64_t grows,
@@ -1137,12 +1138,11 @@ prefill_kernel(const uint16_t* __restrict__ x, int64_t ldx,
     char* sb = lora_b;                   // B chunk [BN n][64 ranks]
     // A split's part of T can go through B as three bf16 terms, whose 8 + 8 + 8 bits are the fp32
     // value: parts rounded to bf16 leave errors of their own size where they cancel. Always beside
-    // an fp8 W and where the call asks for it (skt_spin, free here, holds the number of terms):
-    // calls whose T was summed whole in fp32 before they were split. The second and third term
-    // take the two ring buffers that hold neither T's first nor B.
-    constexpr int TMAX = (RED && RB > 0) ? 3 : 1;
-    static_assert(TMAX == 1 || C::NS == 4, "a ring buffer for each term of T and one for B");
-    const int tterms = TMAX == 1 ? 1 : W8 ? TMAX : skt_spin;
+    // an fp8 W, and with TWHOLE where the call asks for it: calls whose T was summed whole in fp32
+    // before they were split. The second and third term take the two ring buffers that hold neither
+    // T's first nor B. (TWHOLE is of the instance: asked at run time, it cost the other calls 0.5 %.)
+    constexpr int TTERMS = (RED && RB > 0 && (W8 || TWHOLE)) ? 3 : 1;
+    static_assert(TTERMS == 1 || C::NS == 4, "a ring buffer for each term of T and one for B");
     auto t_area = [&](int term) { return term == 0 ? st : lds + ((nk + term) % C::NS) * STAGE; };
     if constexpr (RB > 0) {
       if (t_wave && t_here) {
@@ -1150,27 +1150,25 @@ prefill_kernel(const uint16_t* __restrict__ x, int64_t ldx,
         // >= r (A rows past r were filled with row r-1) are zeroed here: they meet finite
         // stand-in columns of B in the up-projection.
 #pragma unroll
-        for (int term = 0; term < TMAX; ++term) {
-          if (term > 0 && term >= tterms) break;
+        for (int q = 0; q < TPW; ++q) {
+          const int mrow = wm * C::TM + tj[q] * 32 + l32;
 #pragma unroll
-          for (int q = 0; q < TPW; ++q) {
-            const int mrow = wm * C::TM + tj[q] * 32 + l32;
+          for (int g = 0; g < 4; ++g) {
+            const int rk = trb[q] * 32 + g * 8 + lh * 4;
+            float t4[4];
 #pragma unroll
-            for (int g = 0; g < 4; ++g) {
-              const int rk = trb[q] * 32 + g * 8 + lh * 4;
-              float t4[4];
+            for (int e = 0; e < 4; ++e) t4[e] = rk + e < r ? s * acct[q][g * 4 + e] : 0.f;
 #pragma unroll
-              for (int e = 0; e < 4; ++e)
-                t4[e] = term > 0 ? acct[q][g * 4 + e] : rk + e < r ? s * acct[q][g * 4 + e] : 0.f;
+            for (int term = 0; term < TTERMS; ++term) {
               uint2 v;
               v.x = pack_bf16x2(t4[0], t4[1]);
               v.y = pack_bf16x2(t4[2], t4[3]);
               *reinterpret_cast<uint2*>(t_area(term) + t_off(mrow, trb[q] * 4 + g) + lh * 8) = v;
-              if (term + 1 < TMAX) {  // what this term leaves over; nothing past an infinity or NaN
+              if constexpr (TTERMS > 1) {  // what this term leaves over; nothing past an infinity or NaN
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                   const float h = bf16_bits_to_f32(((e < 2 ? v.x : v.y) >> ((e & 1) * 16)) & 0xffffu);
-                  acct[q][g * 4 + e] = fabsf(h) < INFINITY ? t4[e] - h : 0.f;
+                  t4[e] = fabsf(h) < INFINITY ? t4[e] - h : 0.f;
                 }
               }
             }
@@ -1199,21 +1197,21 @@ prefill_kernel(const uint16_t* __restrict__ x, int64_t ldx,
       const int nkk = rem >= 64 ? 4 : (rem + 15) / 16;
       for (int kk = 0; kk < nkk; ++kk) {
         const int c = kk * 2 + lh;
-        bf16x8_t bf[C::NI];
+        bf16x8_t tf[TTERMS][C::MJ], bf[C::NI];
+#pragma unroll
+        for (int term = 0; term < TTERMS; ++term)
+#pragma unroll
+          for (int j = 0; j < C::MJ; ++j)
+            tf[term][j] = as_bf16x8(lds_read16(t_area(term), t_off(wm * C::TM + j * 32 + l32, c)));
 #pragma unroll
         for (int i = 0; i < C::NI; ++i) bf[i] = as_bf16x8(lds_read16(sb, lds_off(wn * C::TN + i * 32 + l32, c)));
 #pragma unroll
-        for (int term = 0; term < TMAX; ++term) {
-          if (term > 0 && term >= tterms) break;
-          bf16x8_t tf[C::MJ];
-#pragma unroll
-          for (int j = 0; j < C::MJ; ++j) tf[j] = as_bf16x8(lds_read16(t_area(term), t_off(wm * C::TM + j * 32 + l32, c)));
+        for (int term = 0; term < TTERMS; ++term)
 #pragma unroll
           for (int i = 0; i < C::NI; ++i)
 #pragma unroll
             for (int j = 0; j < C::MJ; ++j)
-              acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bf[i], tf[j], acc[i][j], 0, 0, 0);
-        }
+              acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(bf[i], tf[term][j], acc[i][j], 0, 0, 0);
       }
       __syncthreads();
     }
@@ -1444,12 +1442,12 @@ bool groups_fit(const LoraArgs& p, int bn) {
 }
 
 template <class C, int WDT, bool HAS_W, int RB, bool EXT_T, bool GATHER, bool SPLIT = false, bool TN = false,
-          bool RED = false, bool PER = false, bool WT = false, bool SKT = false, bool SHARE = false>
+          bool RED = false, bool PER = false, bool WT = false, bool SKT = false, bool SHARE = false, bool TWHOLE = false>
 hipError_t launch_cfg(const LoraArgs& p, const uint16_t* tg, int64_t ldt, int splits = 1,
                       uint64_t* red_part = nullptr, unsigned* red_cnt = nullptr, int tpw = 1, int skt_spin = 0) {
   const int tiles_m = (int)((p.M + C::BM - 1) / C::BM);
   const int tiles_n = (int)((p.N + C::BN - 1) / C::BN);
-  prefill_kernel<C, WDT, HAS_W, RB, EXT_T, GATHER, SPLIT, TN, RED, PER, WT, SKT, SHARE>
+  prefill_kernel<C, WDT, HAS_W, RB, EXT_T, GATHER, SPLIT, TN, RED, PER, WT, SKT, SHARE, TWHOLE>
       <<<dim3(tiles_m * tiles_n / (PER ? tpw : 1), splits), dim3(C::NT), 0, p.stream>>>(
       reinterpret_cast<const uint16_t*>(p.x), p.ldx, p.gather, p.gather_rows, p.w, p.ldw, p.w_scale,
       reinterpret_cast<const uint16_t*>(p.a), p.lda, tg, ldt,
@@ -1907,11 +1905,14 @@ hipError_t launch_red(const LoraArgs& p, int splits) {
     if (p.r <= 32) return launch_cfg<CfgDeep, kFP8, true, 1, false, false, false, false, true>(q, nullptr, 0, splits, part, p.red_cnt);
     return launch_cfg<CfgDeep, kFP8, true, 2, false, false, false, false, true>(q, nullptr, 0, splits, part, p.red_cnt);
   }
-  const int terms = p.t_whole ? 3 : 1;
   if (p.r == 0) return launch_cfg<CfgDeep, kBF16, true, 0, false, false, false, false, true>(q, nullptr, 0, splits, part, p.red_cnt);
-  if (p.r <= 32)
-    return launch_cfg<CfgDeep, kBF16, true, 1, false, false, false, false, true>(q, nullptr, 0, splits, part, p.red_cnt, 1, terms);
-  return launch_cfg<CfgDeep, kBF16, true, 2, false, false, false, false, true>(q, nullptr, 0, splits, part, p.red_cnt, 1, terms);
+  if (p.t_whole)
+    return p.r <= 32 ? launch_cfg<CfgDeep, kBF16, true, 1, false, false, false, false, true, false, false, false, false, true>(
+                           q, nullptr, 0, splits, part, p.red_cnt)
+                     : launch_cfg<CfgDeep, kBF16, true, 2, false, false, false, false, true, false, false, false, false, true>(
+                           q, nullptr, 0, splits, part, p.red_cnt);
+  if (p.r <= 32) return launch_cfg<CfgDeep, kBF16, true, 1, false, false, false, false, true>(q, nullptr, 0, splits, part, p.red_cnt);
+  return launch_cfg<CfgDeep, kBF16, true, 2, false, false, false, false, true>(q, nullptr, 0, splits, part, p.red_cnt);
 }
 
 // y[m][n] = bf16(sum_s part[s][m][n] + sum_j T[m][goff(n) + j] B[n][j]): the partials in split
